@@ -1,11 +1,12 @@
 // bfa_lapack.hip -- batched factorisations for gfx950: potrf_l, potrf_l_mn,
 // syrk_dpotrf_ln(_mn) and getrf_rp on panel-major matrices.
 //
-// One workgroup (4 waves) per instance.  Both factorisations are left-looking
-// over 16-column panels held in LDS at full height (the role of the
-// reference's 12x4 / 8x8 register blocks, blasfeo_hp_pm/d_lapack_lib4.c:954-985
-// and :2443-2634):
-//   potrf: panel <- C(+A*B^T) - L(:,0:c0) L(c0:c0+16,0:c0)^T on the matrix
+// potrf and syrk_dpotrf up to 256 columns: 16-row strips in registers
+// (bfa_potrf_wave.hpp).  potrf above 256 columns and getrf: one workgroup
+// (4 waves) per instance, left-looking over 16-column panels held in LDS at full
+// height (the role of the reference's 12x4 / 8x8 register blocks,
+// blasfeo_hp_pm/d_lapack_lib4.c:954-985 and :2443-2634):
+//   potrf: panel <- C - L(:,0:c0) L(c0:c0+16,0:c0)^T on the matrix
 //          cores, then one wave factors the top 64 rows in registers (the
 //          diagonal 16x16 Cholesky, broadcasting L(jj,j) with v_readlane) and
 //          all waves solve the remaining rows against it;
@@ -28,6 +29,10 @@ template <> struct FactArg<float> { typedef blasfeo_amd_sfact_arg type; };
 template <typename T> struct SPArg;
 template <> struct SPArg<double> { typedef blasfeo_amd_dsyrk_dpotrf_arg type; };
 
+} // namespace bfa
+#include "bfa_potrf_wave.hpp"
+namespace bfa {
+
 // potrf_l for n > 256: left-looking over 16-column LDS panels at full height,
 // the earlier panels read back from D (chol_instance)
 template <typename T, int PS>
@@ -48,484 +53,6 @@ __global__ __launch_bounds__(NTL) void k_potrf(const typename FactArg<T>::type *
 	if (threadIdx.x == 0)
 		a.sD->use_dA = (a.di == 0 && a.dj == 0) ? m : 0;
 }
-
-// The trapezoid's LDS form: square column-major with leading dimension np + 1
-// (the one-instance-per-workgroup kernels), or packed lower 16x17 tiles (the
-// bucketed launches: 78 KB instead of 133 KB at 128 rows, two instances per
-// CU instead of one).
-template <bool PACKED, typename T>
-__device__ __forceinline__ auto lds_acc(T *M, int ld)
-{
-	if constexpr (PACKED)
-		return TileLowerT<T>{M};
-	else
-		return ColMajor<T>{M, ld};
-}
-// LDS elements of the trapezoid plus the reciprocal diagonal for np rows
-__host__ __device__ __forceinline__ size_t lds_elems(int np, bool packed)
-{
-	const size_t t = (size_t)(np / 16);
-	return (packed ? t * (t + 1) / 2 * RT_SZ : (size_t)np * (np + 1)) + np;
-}
-
-// potrf_l (MN = false) and potrf_l_mn (MN = true) with the whole m x n lower
-// trapezoid in LDS (m <= 128): stage it from C, factor in place (chol_acc),
-// stream L and dA out.  NT = 64 (one wave) for m <= 32 so that several
-// instances share a CU.
-template <typename T, int PS, int NT, bool MN, bool PACKED>
-__device__ __forceinline__ void potrf_lds_instance(const typename FactArg<T>::type &a, int np, T *M, T *invd)
-{
-	const int LDM = np + 1;
-	const int m = a.m;
-	int n = MN ? a.n : a.m;
-	if (m <= 0 || n <= 0 || m > np)
-		return;
-	if (n > m)
-		n = m;
-	const int mt = (m + 15) / 16, nt = (n + 15) / 16;
-	const auto Ml = lds_acc<PACKED>(M, LDM);
-	if constexpr (PACKED)
-		g2s_acc<T, PS, NT, true>(view<T, PS>(a.sC), a.ci, a.cj, mt * 16, nt * 16, m, n, Ml);
-	else
-		g2s<T, PS, NT, false, true>(view<T, PS>(a.sC), a.ci, a.cj, mt * 16, nt * 16, m, n, M, LDM);
-	// the one-wave form serves m <= 32: one panel row per lane, no second row set
-	chol_acc<T, NT, NT == WAVE ? 64 : 128>(Ml, m, n, invd);
-	if constexpr (PACKED)
-		s2g_acc<T, PS, NT, true>(view<T, PS>(a.sD), a.di, a.dj, m, n, Ml, 0);
-	else
-		s2g<T, PS, NT, true>(view<T, PS>(a.sD), a.di, a.dj, m, n, M, LDM, 0);
-	T *dD = a.sD->dA;
-	for (int j = threadIdx.x; j < n; j += NT)
-		dD[j] = invd[j];
-	if (threadIdx.x == 0)
-		a.sD->use_dA = (a.di == 0 && a.dj == 0) ? (MN ? 1 : m) : 0;
-}
-
-// The LDS-resident factorisations run either one instance per workgroup
-// (k_potrf_lds, k_syrk_potrf_lds: workgroup b takes instance b) or as a
-// persistent launch over one size bucket (the _q forms), each workgroup
-// taking the next instance of the bucket's list from its atomic queue head.
-// Two kernels rather than one with both modes: the loop costs registers that
-// the one-instance form (several instances per CU at 32 rows) cannot spare.
-// The queued forms are compiled for three waves per SIMD (at most 168
-// registers; the syrk form then fits in 149 VGPRs without spills, against
-// 145 VGPRs + 40 AGPRs and two waves per SIMD unconstrained), so that three
-// four-wave workgroups share a CU where the LDS holds them (up to 96 rows).  The leading barrier makes every
-// thread finish the previous instance (and its read of the slot) before the
-// slot is overwritten and the LDS staged again.  Returns -1 once the bucket
-// is drained.
-__device__ __forceinline__ int queue_next(const int *count, const int *list, int *head, int *qslot)
-{
-	__syncthreads();
-	if (threadIdx.x == 0)
-		*qslot = atomicAdd(head, 1);
-	__syncthreads();
-	const int t = *qslot;
-	return t < *count ? list[t] : -1;
-}
-
-template <typename T, int PS, int NT, bool MN>
-__global__ __launch_bounds__(NT) void k_potrf_lds(const typename FactArg<T>::type *__restrict__ args, int np)
-{
-	extern __shared__ unsigned char smem_raw[];
-	T *M = reinterpret_cast<T *>(smem_raw);
-	potrf_lds_instance<T, PS, NT, MN, false>(args[blockIdx.x], np, M, M + lds_elems(np, false) - np);
-}
-template <typename T, int PS, int NT, bool MN>
-__global__ __launch_bounds__(NT, 3) void k_potrf_lds_q(const typename FactArg<T>::type *__restrict__ args, int np,
-	const int *__restrict__ count, const int *__restrict__ list, int *head)
-{
-	extern __shared__ unsigned char smem_raw[];
-	__shared__ int qslot;
-	T *M = reinterpret_cast<T *>(smem_raw);
-	for (int i; (i = queue_next(count, list, head, &qslot)) >= 0;)
-		potrf_lds_instance<T, PS, NT, MN, true>(args[i], np, M, M + lds_elems(np, true) - np);
-}
-
-// syrk_dpotrf_ln(_mn), m <= 128: D = chol(C + A B^T) on the m x n lower
-// trapezoid (blasfeo_hp_pm/d_lapack_lib4.c:1848-2077).  C's trapezoid is staged
-// in LDS, A B^T is added tile by tile on the matrix cores with A and B read
-// from global memory (a group of up to four row tiles shares B's operand), and
-// the sum is factored in place (chol_acc).
-template <typename T, int PS, int NT, bool PACKED>
-__device__ __forceinline__ void syrk_potrf_lds_instance(const typename SPArg<T>::type &a, int np, T *M, T *invd)
-{
-	typedef typename Vec4<T>::type V4;
-	constexpr int NW = NT / WAVE;
-	const int LDM = np + 1;
-	const int m = a.m, k = a.k;
-	int n = a.n;
-	if (m <= 0 || n <= 0 || m > np || k < 0)
-		return;
-	if (n > m)
-		n = m;
-	const int lane = lane_id(), w = wave_id();
-	const int mt = (m + 15) / 16, nt = (n + 15) / 16;
-	const auto Ml = lds_acc<PACKED>(M, LDM);
-	if constexpr (PACKED)
-		g2s_acc<T, PS, NT, true>(view<T, PS>(a.sC), a.ci, a.cj, mt * 16, nt * 16, m, n, Ml);
-	else
-		g2s<T, PS, NT, false, true>(view<T, PS>(a.sC), a.ci, a.cj, mt * 16, nt * 16, m, n, M, LDM);
-	__syncthreads();
-	if (k > 0)
-	{
-		const PM<T, PS> gA = view<T, PS>(a.sA), gB = view<T, PS>(a.sB);
-		int ntask = 0;
-		for (int bj = 0; bj < nt; bj++)
-			ntask += (mt - bj + 3) / 4;
-		for (int task = w; task < ntask; task += NW)
-		{
-			int bj = 0, rem = task;
-			while (rem >= (mt - bj + 3) / 4)
-			{
-				rem -= (mt - bj + 3) / 4;
-				bj++;
-			}
-			const int g = bj + 4 * rem;
-			V4 acc[4];
-#pragma unroll
-			for (int t = 0; t < 4; t++)
-				acc[t] = V4{0, 0, 0, 0};
-			const int jr = bj * 16 + (lane & 15);     // row of B for this lane's operand
-			// this lane's rows of A (one per tile) and of B at column 0 of k; a
-			// panel-major row advances by PS elements per column
-			const BFA_GLOBAL T *rb = jr < n ? &gB.at(a.bi + jr, a.bj) : nullptr;
-			const BFA_GLOBAL T *ra[4];
-#pragma unroll
-			for (int t = 0; t < 4; t++)
-			{
-				const int ir = (g + t) * 16 + (lane & 15);
-				ra[t] = (g + t < mt && ir < m) ? &gA.at(a.ai + ir, a.aj) : nullptr;
-			}
-			// KU matrix-core steps per round, all their global loads issued
-			// before the first step: one memory latency per 4 KU columns of k
-			// rather than per 4 (KU = 2 costs no registers at four waves; 3
-			// and 4 raise the kernel from 140 to 218 and 250 VGPRs)
-			constexpr int KU = 2;
-#pragma unroll 1
-			for (int kk = 0; kk < k; kk += 4 * KU)
-			{
-				T bv[KU], av[4][KU];
-#pragma unroll
-				for (int u = 0; u < KU; u++)
-				{
-					const int kq = kk + 4 * u + (lane >> 4);
-					const bool kok = kq < k;
-					bv[u] = (kok && rb) ? rb[(size_t)kq * PS] : T(0);
-#pragma unroll
-					for (int t = 0; t < 4; t++)
-						av[t][u] = (kok && ra[t]) ? ra[t][(size_t)kq * PS] : T(0);
-				}
-#pragma unroll
-				for (int u = 0; u < KU; u++)
-					if (kk + 4 * u < k)
-#pragma unroll
-						for (int t = 0; t < 4; t++)
-							if (g + t < mt)
-								acc[t] = mfma16(av[t][u], bv[u], acc[t]);
-			}
-#pragma unroll
-			for (int t = 0; t < 4; t++)
-				if (g + t < mt)
-#pragma unroll
-					for (int r = 0; r < 4; r++)
-					{
-						const int ir = (g + t) * 16 + acc_row<T>(lane, r), jc = bj * 16 + (lane & 15);
-						if (ir < m && jc < n && ir >= jc)
-							Ml(ir, jc) += acc[t][r];
-					}
-		}
-	}
-	chol_acc<T, NT, 128>(Ml, m, n, invd);
-	if constexpr (PACKED)
-		s2g_acc<T, PS, NT, true>(view<T, PS>(a.sD), a.di, a.dj, m, n, Ml, 0);
-	else
-		s2g<T, PS, NT, true>(view<T, PS>(a.sD), a.di, a.dj, m, n, M, LDM, 0);
-	T *dD = a.sD->dA;
-	for (int j = threadIdx.x; j < n; j += NT)
-		dD[j] = invd[j];
-	if (threadIdx.x == 0)
-		a.sD->use_dA = (a.di == 0 && a.dj == 0) ? 1 : 0;
-}
-
-template <typename T, int PS, int NT>
-__global__ __launch_bounds__(NT) void k_syrk_potrf_lds(const typename SPArg<T>::type *__restrict__ args, int np)
-{
-	extern __shared__ unsigned char smem_raw[];
-	T *M = reinterpret_cast<T *>(smem_raw);
-	syrk_potrf_lds_instance<T, PS, NT, false>(args[blockIdx.x], np, M, M + lds_elems(np, false) - np);
-}
-template <typename T, int PS, int NT>
-__global__ __launch_bounds__(NT, 3) void k_syrk_potrf_lds_q(const typename SPArg<T>::type *__restrict__ args, int np,
-	const int *__restrict__ count, const int *__restrict__ list, int *head)
-{
-	extern __shared__ unsigned char smem_raw[];
-	__shared__ int qslot;
-	T *M = reinterpret_cast<T *>(smem_raw);
-	for (int i; (i = queue_next(count, list, head, &qslot)) >= 0;)
-		syrk_potrf_lds_instance<T, PS, NT, true>(args[i], np, M, M + lds_elems(np, true) - np);
-}
-
-// ---------------------------------------------------------------------------
-// potrf_l for 128 < n <= 256: left-looking over block panels of 16 BW columns
-// held in LDS as 16x16 tiles (col-major inside a tile, tile (r, jj) of the
-// panel at (BW r + jj) * 256), one workgroup of NTH threads per instance: BW =
-// 4 (128 KB, one instance per CU, 8 waves), 2 (64 KB, two per CU, 4 waves
-// each) or 1 (32 KB, four per CU): more resident instances overlap their
-// serial chains, at the cost of reading the earlier columns more often.
-//   1. the panel's lower part is staged from C (identity beyond n);
-//   2. the earlier block columns are applied on the matrix cores,
-//      P(r, jj) -= L(rows r, 0:c0) L(rows jj, 0:c0)^T, with L read from D
-//      (one wave per tile row, the A operand shared by the row's BW tiles);
-//   3. the panel is factored right-looking in LDS: wave 0 factors the
-//      diagonal tile in registers (as chol_lds), every thread then solves one
-//      row below it against L_jj with the reciprocal diagonal, and the
-//      panel's remaining tile columns get a rank-16 matrix-core update;
-//   4. L and the reciprocal diagonal are written to D.
-// Compared with the 16-column left-looking form this reads the earlier
-// columns once per 16 BW columns instead of once per 16.
-// ---------------------------------------------------------------------------
-constexpr int PT_NMAX = 256;
-
-template <typename T, int BW>
-__host__ __device__ inline size_t potrf_tiles_lds_bytes()
-{
-	return sizeof(T) * (16 * BW * 256 + 16 * 17 + 16);
-}
-
-template <typename T, int PS, int BW, int NTH>
-__global__ __launch_bounds__(NTH) void k_potrf_tiles(const typename FactArg<T>::type *__restrict__ args, int nmax)
-{
-	constexpr int PT_NT = NTH;
-	constexpr int PT_NW = NTH / WAVE;
-	typedef typename Vec4<T>::type V4;
-	extern __shared__ unsigned char smem_raw[];
-	T *P = reinterpret_cast<T *>(smem_raw);
-	T *L11 = P + 16 * BW * 256;
-	T *invs = L11 + 16 * 17;
-	const typename FactArg<T>::type &a = args[blockIdx.x];
-	const int n = a.m;
-	if (n <= 0 || n > nmax)
-		return;
-	const int lane = lane_id();
-	const int w = wave_id();
-	const int nb = (n + 15) / 16;
-	const PM<T, PS> gC = view<T, PS>(a.sC);
-	PM<T, PS> gD = view<T, PS>(a.sD);
-	const int ci = a.ci, cj = a.cj, di = a.di, dj = a.dj;
-	T *dD = a.sD->dA;
-
-	for (int J0 = 0; J0 < nb; J0 += BW)
-	{
-		const int R = nb - J0;           // tile rows of the panel
-		const int C = min(BW, R);        // tile columns of the panel
-		const int c0 = 16 * J0;          // first column of the panel
-		__syncthreads();
-		// 1. stage the panel (lower part; identity beyond n), four tiles per
-		// wave at a time: their 16 loads per lane are issued before any store
-		for (int t0 = w; t0 < R * BW; t0 += 4 * PT_NW)
-		{
-			T v[4][4];
-#pragma unroll
-			for (int u = 0; u < 4; u++)
-			{
-				const int t = t0 + u * PT_NW;
-				const int r = t / BW, jj = t % BW;
-				const int i = lane & 15;
-				const int gr = c0 + 16 * r + i;
-#pragma unroll
-				for (int k = 0; k < 4; k++)
-				{
-					const int j = 4 * k + (lane >> 4);
-					const int gc = c0 + 16 * jj + j;
-					const bool live = t < R * BW && jj < C && r >= jj;
-					v[u][k] = (live && gr < n && gc < n && gr >= gc) ? gC.at(ci + gr, cj + gc)
-					                                                  : ((gr == gc) ? T(1) : T(0));
-				}
-			}
-#pragma unroll
-			for (int u = 0; u < 4; u++)
-			{
-				const int t = t0 + u * PT_NW;
-				const int r = t / BW, jj = t % BW;
-				if (t >= R * BW || jj >= C || r < jj)
-					continue;
-				T *PT = P + t * 256;
-				const int i = lane & 15;
-#pragma unroll
-				for (int k = 0; k < 4; k++)
-					PT[(4 * k + (lane >> 4)) * 16 + i] = v[u][k];
-			}
-		}
-		__syncthreads();
-		// 2. apply the earlier block columns (L from D)
-		if (J0 > 0)
-		{
-			for (int r = w; r < R; r += PT_NW)
-			{
-				V4 acc[BW];
-#pragma unroll
-				for (int jj = 0; jj < BW; jj++)
-				{
-					acc[jj] = V4{0, 0, 0, 0};
-					if (jj < C && jj <= r)
-#pragma unroll
-						for (int q = 0; q < 4; q++)
-							acc[jj][q] = P[(r * BW + jj) * 256 + (lane & 15) * 16 + acc_row<T>(lane, q)];
-				}
-				const int ar = c0 + 16 * r + (lane & 15);
-				const bool aok = ar < n;
-
-				// 16 columns of L per step (c0 is a multiple of 16 BW): all of a
-				// step's loads are issued before its products, so a wave waits
-				// for memory once per 16 columns instead of once per 4
-				for (int kk = 0; kk < c0; kk += 16)
-				{
-					T av[4], bv[4][BW];
-#pragma unroll
-					for (int u = 0; u < 4; u++)
-					{
-						const int kq = kk + 4 * u + (lane >> 4);
-						av[u] = aok ? gD.at(di + ar, dj + kq) : T(0);
-#pragma unroll
-						for (int jj = 0; jj < BW; jj++)
-						{
-							const int br = c0 + 16 * jj + (lane & 15);
-							bv[u][jj] = (jj < C && jj <= r && br < n) ? gD.at(di + br, dj + kq) : T(0);
-						}
-					}
-#pragma unroll
-					for (int u = 0; u < 4; u++)
-#pragma unroll
-						for (int jj = 0; jj < BW; jj++)
-							if (jj < C && jj <= r)
-								acc[jj] = mfma16(-av[u], bv[u][jj], acc[jj]);
-				}
-#pragma unroll
-				for (int jj = 0; jj < BW; jj++)
-					if (jj < C && jj <= r)
-#pragma unroll
-						for (int q = 0; q < 4; q++)
-							P[(r * BW + jj) * 256 + (lane & 15) * 16 + acc_row<T>(lane, q)] = acc[jj][q];
-			}
-			__syncthreads();
-		}
-		// 3. factor the panel
-		for (int jj = 0; jj < C; jj++)
-		{
-			T *D = P + (jj * BW + jj) * 256;
-			if (w == 0)
-			{
-				T x[16];
-#pragma unroll
-				for (int j = 0; j < 16; j++)
-					x[j] = lane < 16 ? D[j * 16 + lane] : T(0);
-				// no per-lane guards: the upper triangle of the tile (lanes < j)
-				// is updated too, but only the lower triangle is read (the
-				// row solve, L11 below its diagonal) or written to D.  Lane j
-				// holds the pivot c, so scaling every lane gives it c * inv;
-				// every lane stores the uniform reciprocal (no per-column lane
-				// masks, which held SGPRs across the tile)
-#pragma unroll
-				for (int j = 0; j < 16; j++)
-				{
-					const T c = readlane(x[j], j);
-					const T inv = (c > T(0)) ? rsqrt_fast(c) : T(0);
-					x[j] *= inv;
-					invs[j] = inv;
-#pragma unroll
-					for (int jn = j + 1; jn < 16; jn++)
-					{
-						const T l = readlane(x[j], jn);
-						x[jn] -= x[j] * l;
-					}
-				}
-				if (lane < 16)
-#pragma unroll
-					for (int j = 0; j < 16; j++)
-					{
-						D[j * 16 + lane] = x[j];
-						L11[lane * 17 + j] = x[j];
-					}
-			}
-			__syncthreads();
-			// rows below the diagonal tile: x_j = (x_j - sum_{l<j} x_l L_jl) * inv_j
-			{
-				const int nrow = (R - jj - 1) * 16;
-				for (int q = threadIdx.x; q < nrow; q += PT_NT)
-				{
-					asm volatile("" ::: "memory");
-					const int r = jj + 1 + (q >> 4), i = q & 15;
-					T *row = P + (r * BW + jj) * 256 + i;
-					T x[16];
-#pragma unroll
-					for (int j = 0; j < 16; j++)
-						x[j] = row[j * 16];
-#pragma unroll
-					for (int j = 0; j < 16; j++)
-					{
-						T c = x[j];
-#pragma unroll
-						for (int l = 0; l < j; l++)
-							c -= x[l] * L11[j * 17 + l];
-						x[j] = c * invs[j];
-					}
-#pragma unroll
-					for (int j = 0; j < 16; j++)
-						row[j * 16] = x[j];
-				}
-			}
-			__syncthreads();
-			// rank-16 update of the panel's later tile columns
-			{
-				const int ntask = (C - jj - 1) * R;
-				for (int t = w; t < ntask; t += PT_NW)
-				{
-					const int j2 = jj + 1 + t / R, r = t % R;
-					if (r < j2)
-						continue;
-					V4 acc;
-#pragma unroll
-					for (int q = 0; q < 4; q++)
-						acc[q] = P[(r * BW + j2) * 256 + (lane & 15) * 16 + acc_row<T>(lane, q)];
-#pragma unroll
-					for (int kk = 0; kk < 16; kk += 4)
-					{
-						const int o = (kk + (lane >> 4)) * 16 + (lane & 15);
-						acc = mfma16(-P[(r * BW + jj) * 256 + o], P[(j2 * BW + jj) * 256 + o], acc);
-					}
-#pragma unroll
-					for (int q = 0; q < 4; q++)
-						P[(r * BW + j2) * 256 + (lane & 15) * 16 + acc_row<T>(lane, q)] = acc[q];
-				}
-			}
-			if (threadIdx.x < 16 && c0 + 16 * jj + threadIdx.x < n)
-				dD[c0 + 16 * jj + threadIdx.x] = invs[threadIdx.x];
-			__syncthreads();
-		}
-		// 4. write L (lower part, rows and columns < n)
-		for (int t = w; t < R * BW; t += PT_NW)
-		{
-			const int r = t / BW, jj = t % BW;
-			if (jj >= C || r < jj)
-				continue;
-			const T *PT = P + t * 256;
-			const int i = lane & 15;
-			const int gr = c0 + 16 * r + i;
-#pragma unroll
-			for (int k = 0; k < 4; k++)
-			{
-				const int j = 4 * k + (lane >> 4);
-				const int gc = c0 + 16 * jj + j;
-				if (gr < n && gc < n && gr >= gc)
-					gD.at(di + gr, dj + gc) = PT[j * 16 + i];
-			}
-		}
-	}
-	if (threadIdx.x == 0)
-		a.sD->use_dA = (a.di == 0 && a.dj == 0) ? n : 0;
-}
-
 
 // ---------------------------------------------------------------------------
 // LU with partial row pivoting (blasfeo_ref/x_lapack_ref.c:1156-1536 semantics);
@@ -1016,68 +543,6 @@ static int launch_potrf_mn_split(int ps, int batch, const blasfeo_amd_dfact_arg 
 	return check_launch(name);
 }
 
-// The m <= 128 LDS-resident launches hold the whole trapezoid in LDS, sized
-// for np rows.  With a bound above 32 rows a plan kernel sorts the instances
-// into buckets of 16 rows (instance i to bucket ceil(m/16) - 1) and each
-// bucket gets a persistent launch whose LDS is sized for that bucket, largest
-// first, so that an instance is charged its own footprint rather than the
-// bound's, and holds it as packed lower tiles (79 KB at 128 rows: two
-// workgroups per CU; the square form, 133 KB, allowed one).  Up to 32 rows,
-// one workgroup per instance with the square form (at most 8.7 KB).
-// counts[0..LDS_NB-1] and the queue heads counts[16..] start at 0.
-constexpr int LDS_NB = 8;
-template <typename R>
-__global__ void k_lds_plan(const R *__restrict__ args, int batch, int *counts, int *lists)
-{
-	const int i = blockIdx.x * blockDim.x + threadIdx.x;
-	plan_bucket<LDS_NB>(i, i < batch ? min(LDS_NB - 1, max(0, (args[i].m - 1) / 16)) : -1, batch, counts, lists);
-}
-
-// Eight waves rather than four for a bucket's queued launch (tuning knob
-// lds_threads[bucket] = 512): the update tasks of a panel step and of the
-// syrk are shared by twice the waves, but the registers of the eight-wave
-// form leave one workgroup per CU.  Four waves by default: with the packed
-// tiles two 128-row instances share a CU, and 65536 x dsyrk_dpotrf_ln of
-// m, k ~ U{8..128} take 8.38 ms on MI355X against 9.97 ms with eight waves
-// from 97 rows (with the square LDS form, one instance per CU from 97 rows,
-// eight waves there had won: 10.17 against 10.72 ms).
-static bool lds_wide(int np, const int *queued)
-{
-	return queued && np > 32 && tune_value(TUNE_LDS_THREADS, (np - 1) / 16) == 512;
-}
-
-// go(np, grid, shm, count, list, head) launches the kernel form for np rows
-// (the one-wave form for np <= 32)
-template <typename R, typename Go>
-static int launch_lds_buckets(const R *args, int batch, int npad, size_t elem, hipStream_t st, const char *name, Go go)
-{
-	if (npad <= 32)
-		return go(npad, batch, elem * lds_elems(npad, false), (const int *)nullptr, (const int *)nullptr, (int *)nullptr);
-	const size_t wsbytes = sizeof(int) * (64 + (size_t)LDS_NB * batch);
-	int *ws = (int *)plan_workspace(wsbytes, st);
-	if (!ws)
-		return set_error(BLASFEO_AMD_ENOMEM, "%s: cannot allocate the %zu-byte plan workspace", name, wsbytes);
-	int *counts = ws, *heads = ws + 16, *lists = ws + 64;
-	hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(64), 0, st, ws, 64);
-	hipLaunchKernelGGL((k_lds_plan<R>), dim3((batch + 255) / 256), dim3(256), 0, st, args, batch, counts, lists);
-	int rc = check_launch(name);
-	if (rc)
-		return rc;
-	const int cus = num_cus() > 0 ? num_cus() : 256;
-	for (int b = LDS_NB - 1; b >= 0; b--)
-	{
-		if (16 * b >= npad)
-			continue;   // m beyond the bound: no instance runs (as in the one-launch form)
-		const int np = min(16 * (b + 1), npad);
-		const size_t shm = elem * lds_elems(np, true);
-		// as many workgroups as the LDS holds, at most 16 one-wave or 8 four-wave ones per CU
-		const int per_cu = max(1, min(np <= 32 ? 16 : 8, (int)(163840 / shm)));
-		if ((rc = go(np, min(batch, per_cu * cus), shm, counts + b, lists + (size_t)b * batch, heads + b)))
-			return rc;
-	}
-	return 0;
-}
-
 template <typename T, int MODE>
 static int launch_potrf(int ps, int batch, const typename FactArg<T>::type *args, const blasfeo_amd_hint *hint, hipStream_t st, const char *name)
 {
@@ -1087,92 +552,52 @@ static int launch_potrf(int ps, int batch, const typename FactArg<T>::type *args
 	int mmax;
 	if ((rc = fact_mmax_arg<T>(hint, name, &mmax)))
 		return rc;
-	if (mmax <= 128)
+	if (mmax <= (MODE == 0 ? 256 : 128))
 	{
-		auto go = [&](int np, int grid, size_t shm, const int *cnt, const int *lst, int *hd) {
-#define BFA_POTRF_LDS(PS_, NT_)                                                                            \
-	do                                                                                                     \
-	{                                                                                                      \
-		if (cnt)                                                                                           \
-			hipLaunchKernelGGL((k_potrf_lds_q<T, PS_, NT_, MODE == 1>), dim3(grid), dim3(NT_), shm, st, args, np, cnt, lst, hd); \
-		else                                                                                               \
-			hipLaunchKernelGGL((k_potrf_lds<T, PS_, NT_, MODE == 1>), dim3(grid), dim3(NT_), shm, st, args, np); \
+		// sizes up to 128 are bounded to whole strips
+		if (mmax <= 128)
+			mmax = (mmax + 15) / 16 * 16;
+		// One wave per instance once the batch gives every CU more than two
+		// instances, NW waves per instance below: n = 64, 128 and 256 in batches
+		// of 256 take 16, 59 and 311 us against 14, 41 and 114 us, in batches of
+		// 8192 88, 489 and 2715 us against 106, 597 and 3431 us (MI355X; they
+		// cross between 512 and 1000 instances).  The "potrf_bw" knob forces the
+		// first (1) or the second (2, 4).
+		const int cus = num_cus() > 0 ? num_cus() : 256;
+		const int knob = tune_value(TUNE_POTRF_BW, 0);
+		const bool wave = knob == 1 || (knob == 0 && batch > 2 * cus);
+#define BFA_POTRF(PS_, NB_, NW_)                                                                                           \
+	do                                                                                                                     \
+	{                                                                                                                      \
+		if (wave)                                                                                                          \
+			hipLaunchKernelGGL((k_potrf_wave<T, PS_, NB_>), dim3(batch), dim3(WAVE), 0, st, args, mmax, MODE == 1);        \
+		else                                                                                                               \
+			hipLaunchKernelGGL((k_potrf_coop<T, PS_, NW_>), dim3(batch), dim3(WAVE * NW_), 0, st, args, mmax, MODE == 1);  \
 	} while (0)
-			if (np <= 32)
-			{
-				if (ps == 4)
-					BFA_POTRF_LDS(4, 64);
-				else if (ps == 8)
-					BFA_POTRF_LDS(8, 64);
-				else
-					BFA_POTRF_LDS(16, 64);
-			}
-			else if (lds_wide(np, cnt))
-			{
-				if (ps == 4)
-					hipLaunchKernelGGL((k_potrf_lds_q<T, 4, 2 * NTL, MODE == 1>), dim3(grid), dim3(2 * NTL), shm, st, args, np, cnt, lst, hd);
-				else if (ps == 8)
-					hipLaunchKernelGGL((k_potrf_lds_q<T, 8, 2 * NTL, MODE == 1>), dim3(grid), dim3(2 * NTL), shm, st, args, np, cnt, lst, hd);
-				else
-					hipLaunchKernelGGL((k_potrf_lds_q<T, 16, 2 * NTL, MODE == 1>), dim3(grid), dim3(2 * NTL), shm, st, args, np, cnt, lst, hd);
-			}
-			else
-			{
-				if (ps == 4)
-					BFA_POTRF_LDS(4, NTL);
-				else if (ps == 8)
-					BFA_POTRF_LDS(8, NTL);
-				else
-					BFA_POTRF_LDS(16, NTL);
-			}
-#undef BFA_POTRF_LDS
-			return check_launch(name);
-		};
-		return launch_lds_buckets(args, batch, (mmax + 15) / 16 * 16, sizeof(T), st, name, go);
+#define BFA_POTRF_N(PS_)              \
+	do                                \
+	{                                 \
+		if (mmax <= 32)               \
+			BFA_POTRF(PS_, 2, 1);     \
+		else if (mmax <= 64)          \
+			BFA_POTRF(PS_, 4, 2);     \
+		else if (mmax <= 128)         \
+			BFA_POTRF(PS_, 8, 4);     \
+		else                          \
+			BFA_POTRF(PS_, 16, 8);    \
+	} while (0)
+		if (ps == 4)
+			BFA_POTRF_N(4);
+		else if (ps == 8)
+			BFA_POTRF_N(8);
+		else if constexpr (sizeof(T) == 4)
+			BFA_POTRF_N(16);
+#undef BFA_POTRF_N
+#undef BFA_POTRF
+		return check_launch(name);
 	}
 	if (MODE == 1)
 		return launch_potrf_mn_split(ps, batch, (const blasfeo_amd_dfact_arg *)args, hint, mmax, st, name);
-	if (MODE == 0 && mmax <= PT_NMAX)
-	{
-		// block panels of 16 columns (four 4-wave instances per CU, whose
-		// chains overlap), 32 (two per CU) or 64 (one 8-wave instance per
-		// CU): the potrf + trsm solve sequence for 2048 x n = 256 takes 1.31,
-		// 1.65 and 1.90 ms on MI355X.  16 by default, the tuning knob
-		// potrf_bw overrides
-		const int knob = tune_value(TUNE_POTRF_BW, 0);
-		const int bw = knob == 4 ? 4 : (knob == 2 ? 2 : 1);
-		if (bw == 1)
-		{
-			const size_t shm3 = potrf_tiles_lds_bytes<T, 1>();
-			if (ps == 4)
-				hipLaunchKernelGGL((k_potrf_tiles<T, 4, 1, 256>), dim3(batch), dim3(256), shm3, st, args, mmax);
-			else if (ps == 8)
-				hipLaunchKernelGGL((k_potrf_tiles<T, 8, 1, 256>), dim3(batch), dim3(256), shm3, st, args, mmax);
-			else
-				hipLaunchKernelGGL((k_potrf_tiles<T, 16, 1, 256>), dim3(batch), dim3(256), shm3, st, args, mmax);
-		}
-		else if (bw == 4)
-		{
-			const size_t shm3 = potrf_tiles_lds_bytes<T, 4>();
-			if (ps == 4)
-				hipLaunchKernelGGL((k_potrf_tiles<T, 4, 4, 512>), dim3(batch), dim3(512), shm3, st, args, mmax);
-			else if (ps == 8)
-				hipLaunchKernelGGL((k_potrf_tiles<T, 8, 4, 512>), dim3(batch), dim3(512), shm3, st, args, mmax);
-			else
-				hipLaunchKernelGGL((k_potrf_tiles<T, 16, 4, 512>), dim3(batch), dim3(512), shm3, st, args, mmax);
-		}
-		else
-		{
-			const size_t shm3 = potrf_tiles_lds_bytes<T, 2>();
-			if (ps == 4)
-				hipLaunchKernelGGL((k_potrf_tiles<T, 4, 2, 256>), dim3(batch), dim3(256), shm3, st, args, mmax);
-			else if (ps == 8)
-				hipLaunchKernelGGL((k_potrf_tiles<T, 8, 2, 256>), dim3(batch), dim3(256), shm3, st, args, mmax);
-			else
-				hipLaunchKernelGGL((k_potrf_tiles<T, 16, 2, 256>), dim3(batch), dim3(256), shm3, st, args, mmax);
-		}
-		return check_launch(name);
-	}
 	const size_t shm = sizeof(T) * PW * ((mmax + 15) / 16 * 16 + 1);
 	if (ps == 4)
 		hipLaunchKernelGGL((k_potrf<T, 4>), dim3(batch), dim3(NTL), shm, st, args, mmax);
@@ -1252,40 +677,25 @@ static int launch_syrk_potrf(int ps, int batch, const blasfeo_amd_dsyrk_dpotrf_a
 		hipLaunchKernelGGL(k_mn_finish, dim3(nb), dim3(256), 0, st, fact, batch);
 		return check_launch(name);
 	}
-	auto go = [&](int np, int grid, size_t shm, const int *cnt, const int *lst, int *hd) {
-#define BFA_SP_LDS(PS_, NT_)                                                                               \
-	do                                                                                                     \
-	{                                                                                                      \
-		if (cnt)                                                                                           \
-			hipLaunchKernelGGL((k_syrk_potrf_lds_q<double, PS_, NT_>), dim3(grid), dim3(NT_), shm, st, args, np, cnt, lst, hd); \
-		else                                                                                               \
-			hipLaunchKernelGGL((k_syrk_potrf_lds<double, PS_, NT_>), dim3(grid), dim3(NT_), shm, st, args, np); \
+	mmax = (mmax + 15) / 16 * 16;
+#define BFA_SP(PS_, NW_) hipLaunchKernelGGL((k_syrk_potrf_coop<double, PS_, NW_>), dim3(batch), dim3(WAVE * NW_), 0, st, args, mmax)
+#define BFA_SP_N(PS_)           \
+	do                          \
+	{                           \
+		if (mmax <= 32)         \
+			BFA_SP(PS_, 1);     \
+		else if (mmax <= 64)    \
+			BFA_SP(PS_, 2);     \
+		else                    \
+			BFA_SP(PS_, 4);     \
 	} while (0)
-		if (np <= 32)
-		{
-			if (ps == 4)
-				BFA_SP_LDS(4, 64);
-			else
-				BFA_SP_LDS(8, 64);
-		}
-		else if (lds_wide(np, cnt))
-		{
-			if (ps == 4)
-				hipLaunchKernelGGL((k_syrk_potrf_lds_q<double, 4, 2 * NTL>), dim3(grid), dim3(2 * NTL), shm, st, args, np, cnt, lst, hd);
-			else
-				hipLaunchKernelGGL((k_syrk_potrf_lds_q<double, 8, 2 * NTL>), dim3(grid), dim3(2 * NTL), shm, st, args, np, cnt, lst, hd);
-		}
-		else
-		{
-			if (ps == 4)
-				BFA_SP_LDS(4, NTL);
-			else
-				BFA_SP_LDS(8, NTL);
-		}
-#undef BFA_SP_LDS
-		return check_launch(name);
-	};
-	return launch_lds_buckets(args, batch, (mmax + 15) / 16 * 16, sizeof(double), st, name, go);
+	if (ps == 4)
+		BFA_SP_N(4);
+	else
+		BFA_SP_N(8);
+#undef BFA_SP_N
+#undef BFA_SP
+	return check_launch(name);
 }
 
 } // namespace bfa

@@ -45,16 +45,14 @@ bool valid(const char *name, int index, int value)
 		return true;
 	if (!std::strcmp(name, "ric_per_cu") || !std::strcmp(name, "gemm_grid_y"))
 		return value >= 1 && value <= 64;
-	// potrf_bw: tile columns per block panel of potrf_l for 128 < n <= 256
+	// potrf_bw: 1 = one wave per instance of potrf_l(_mn), 2 or 4 = several
 	if (!std::strcmp(name, "potrf_bw"))
 		return value == 1 || value == 2 || value == 4;
 	// trsm_thin: 1 = always the one-wavefront left solve when it applies, 2 = never
 	// gemm_wave: 1 = the one-wavefront-per-tile gemm when the sizes allow it, 2 = never
 	if (!std::strcmp(name, "trsm_thin") || !std::strcmp(name, "gemm_wave"))
 		return value == 1 || value == 2;
-	// lds_threads: threads per workgroup of the LDS-resident potrf_l(_mn) and
-	// dsyrk_dpotrf_ln launch of 16-row bucket index (rows 16 index + 1 ..
-	// 16 index + 16); the buckets up to 32 rows always run one wave.  0: 256
+	// lds_threads: accepted and returned, no launch uses it
 	if (!std::strcmp(name, "lds_threads"))
 		return index >= 2 && (value == 256 || value == 512);
 	// ric_threads: one wave only for the classes whose stages have nu+nx <= 64

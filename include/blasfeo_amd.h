@@ -134,9 +134,9 @@ const char *blasfeo_amd_last_error(void);
  *   "ric_threads", index = class 0..7: threads per instance (64, 128 or 256;
  *                  64 only for classes 0..4);
  *   "gemm_grid_y", index 0: most workgroups per gemm/syrk/trmm instance (1..64);
- *   "potrf_bw",    index 0: tile columns per block panel of potrf_l for
- *                  128 < n <= 256 (1, 2 or 4: 16-, 32- or 64-column panels,
- *                  four, two or one instance per CU; built-in 1);
+ *   "potrf_bw",    index 0: potrf_l(_mn) up to 256 columns with one wave per
+ *                  instance (1) or with several (2, 4); built-in: one when the
+ *                  batch gives every CU more than two instances;
  *   "trsm_thin",   index 0: left-side solves (llnn, lltn, llnu, lunn) with
  *                  hint->max_n <= 4 and m <= 256 on one wavefront per instance:
  *                  1 always, 2 never; built-in: when the batch has at least
@@ -146,10 +146,8 @@ const char *blasfeo_amd_last_error(void);
  *                  (operands from global memory): 1 or 0 (built-in) when the
  *                  hint bounds m and n by 256, 2 never (the LDS-staged
  *                  64 x 64 engine);
- *   "lds_threads", index = 16-row bucket 2..7 (rows 16 index + 1 .. 16 index + 16)
- *                  of the LDS-resident potrf_l(_mn) and dsyrk_dpotrf_ln launches
- *                  (size bound 33..128): threads per workgroup, 256 or 512;
- *                  built-in 256.
+ *   "lds_threads", index 2..7: 256 or 512, kept and returned; no launch uses it
+ *                  (the kernels it shaped have no such choice any more).
  * blasfeo_amd_tune_set returns BLASFEO_AMD_OK or BLASFEO_AMD_EINVAL;
  * blasfeo_amd_tune_get returns the value (0 = built-in) or BLASFEO_AMD_EINVAL. */
 int blasfeo_amd_tune_set(const char *name, int index, int value);

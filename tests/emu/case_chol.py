@@ -10,6 +10,8 @@ exactly-sized block, checked against the oracle:
   syrk_potrf_lds <ps>  blasfeo_amd_dsyrk_dpotrf_ln_batched with m <= 128, the same launches
   <case>_wide <ps>  potrf_lds, potrf_lds_mn or syrk_potrf_lds with eight-wave workgroups
                     for the buckets above 32 rows (tuning knob lds_threads = 512)
+  <case>_one <ps>   potrf_lds or potrf_lds_mn with one wave per instance (tuning knob
+                    potrf_bw = 1; by default a small batch takes several)
 Usage: python case_chol.py <case> <ps>"""
 import ctypes
 import sys
@@ -22,6 +24,9 @@ HINT = bfa.HINT
 
 def run(which, ps):
     E = emu_lib("emu_lapack")
+    if which.endswith("_one"):
+        which = which[:-4]
+        assert E.blasfeo_amd_tune_set(b"potrf_bw", 0, 1) == 0, E.emu_last_error()
     if which.endswith("_wide"):
         # the eight-wave form of the queued bucket launches (rows 33 .. 128)
         which = which[:-5]

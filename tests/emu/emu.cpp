@@ -146,6 +146,8 @@ uint64_t exch_dpp(uint64_t old, uint64_t v, int ctrl, int row_mask, int bank_mas
 		const int s = ctrl & 15;
 		src = (l & ~15) | ((r16 - s) & 15);
 	}
+	else if (ctrl >= 0x150 && ctrl <= 0x15f)
+		src = (l & ~15) | (ctrl & 15);
 	else if (ctrl == 0x142)
 		src = row >= 1 ? 16 * row - 1 : -1;
 	else if (ctrl == 0x143)

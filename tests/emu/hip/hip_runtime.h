@@ -90,7 +90,29 @@ inline int emu_dpp_i(int old, int v, int ctrl, int rm, int bm, bool bc)
 {
 	return (int)emu::exch_dpp((uint64_t)(uint32_t)old, (uint64_t)(uint32_t)v, ctrl, rm, bm, bc);
 }
+inline double emu_dpp_i(double old, double v, int ctrl, int rm, int bm, bool bc)
+{
+	uint64_t o, x;
+	memcpy(&o, &old, 8);
+	memcpy(&x, &v, 8);
+	x = emu::exch_dpp(o, x, ctrl, rm, bm, bc);
+	memcpy(&v, &x, 8);
+	return v;
+}
 #define __builtin_amdgcn_update_dpp(old, v, ctrl, rm, bm, bc) emu_dpp_i((old), (v), (ctrl), (rm), (bm), (bc))
+// v_permlane16_swap / v_permlane32_swap: {first, second} after the odd rows of
+// 16 lanes (the upper 32 lanes) of the first operand changed places with the
+// even rows (the lower 32 lanes) of the second
+typedef unsigned emu_u2 __attribute__((ext_vector_type(2)));
+inline emu_u2 emu_permlane_swap(unsigned a, unsigned b, int width)
+{
+	const int l = emu::lane();
+	const bool up = (l & width) != 0;
+	const unsigned af = (unsigned)emu::exch(a, l ^ width), bf = (unsigned)emu::exch(b, l ^ width);
+	return emu_u2{up ? bf : a, up ? b : af};
+}
+#define __builtin_amdgcn_permlane16_swap(a, b, fi, bc) emu_permlane_swap((a), (b), 16)
+#define __builtin_amdgcn_permlane32_swap(a, b, fi, bc) emu_permlane_swap((a), (b), 32)
 #define __builtin_amdgcn_wave_barrier() emu::wave_bar()
 #define __builtin_amdgcn_fence(...) ((void)0)
 #define __builtin_amdgcn_rsq(c) (1.0 / sqrt((double)(c)))
@@ -161,6 +183,7 @@ inline void emu_launch(void (*k)(KA...), dim3 grid, dim3 block, size_t shm, A...
 #define hipLaunchKernelGGL(k, grid, block, shm, stream, ...) emu_launch(k, dim3(grid), dim3(block), (size_t)(shm), __VA_ARGS__)
 
 #define BFA_GLOBAL   // host memory: no address-space qualifier
+#define BFA_PIN(x) ((void)0)   // scheduling barrier of the device compiler
 #define __align__(n) __attribute__((aligned(n)))
 #define HIP_SYMBOL(x) (&(x))
 inline hipError_t hipGetSymbolAddress(void **p, const void *sym) { *p = const_cast<void *>(sym); return hipSuccess; }

@@ -63,6 +63,14 @@ def test_lds_size_buckets(emu_build, case, ps):
     run_case("case_chol.py", case, ps)
 
 
+@pytest.mark.parametrize("case", ["potrf_lds_one", "potrf_lds_mn_one", "potrf_l_mn_one"])
+@pytest.mark.parametrize("ps", [4, 8])
+def test_potrf_one_wave(emu_build, case, ps):
+    """potrf_l and potrf_l_mn with one wave per instance, the form of large
+    batches (the default of these small ones is several waves)."""
+    run_case("case_chol.py", case, ps)
+
+
 @pytest.mark.parametrize("ps", [4, 8])
 def test_potrf_global_kernel(emu_build, ps):
     """k_potrf (potrf_l for n > 256; 16-column panels at full height, the
