@@ -14,6 +14,7 @@
 #include "bfa_gemm_core.hpp"
 #include "bfa_gemm_wave.hpp"
 #include "bfa_chol_core.hpp"
+#include "bfa_trsm_strip.hpp"
 #include "bfa_internal.hpp"
 
 namespace bfa {
@@ -59,171 +60,6 @@ __global__ __launch_bounds__(NT3) __attribute__((amdgpu_waves_per_eu(3))) void k
 	gemm_core<T, PS, OP_TRMM_RLNN>(As, Bs, a.m, a.n, a.n, a.alpha, T(0),
 		gA, a.ai, a.aj, view<T, PS>(a.sB), a.bi, a.bj,
 		gA, 0, 0, view<T, PS>(a.sD), a.di, a.dj, slot, slots);
-}
-
-// ---------------------------------------------------------------------------
-// trsm_rltn: D = alpha * B * A^{-T}, A lower n x n (blasfeo_ref/x_blas3_ref.c:1642-1752)
-// A workgroup solves a 64-row block of B: D's row block lives in LDS while
-// the columns are produced 16 at a time: the already-solved columns are
-// applied with matrix-core steps (X -= D(:,0:j) A(j,0:j)^T), then one wave
-// solves the 16x16 diagonal triangle row by row with the reciprocal diagonal.
-// ---------------------------------------------------------------------------
-constexpr int TRSM_NMAX = 256;
-constexpr int LDX = TM + 1;
-
-// One instance of trsm_rltn, row blocks t0, t0 + tstep, ... (all threads of
-// the workgroup call it together).  DA_GIVEN: the reciprocal diagonal is
-// read from sA->dA whatever use_dA says (the trapezoid Cholesky, whose
-// diagonal block was just factored into the same descriptor with its
-// reciprocals stored there).
-template <typename T, int PS, bool DA_GIVEN>
-__device__ __forceinline__ void trsm_rltn_instance(const typename TrsmArg<T>::type &a, int nmax, int t0, int tstep,
-	T *Xs, T *inv_s, T *Ad)
-{
-	typedef typename Vec4<T>::type V4;
-	const int m = a.m, n = a.n;
-	if (m <= 0 || n <= 0 || n > nmax)
-		return;
-	const PM<T, PS> gA = view<T, PS>(a.sA);
-	const PM<T, PS> gB = view<T, PS>(a.sB);
-	PM<T, PS> gD = view<T, PS>(a.sD);
-	const T alpha = a.alpha;
-	const int lane = lane_id();
-	const int w = wave_id();
-
-	// reciprocal diagonal: cached copy when valid at launch, else 1/A_jj
-	// (an output aliasing A invalidates the cache first, as in the reference)
-	const bool cached = DA_GIVEN || (a.ai == 0 && a.aj == 0 && a.sD != a.sA && a.sA->use_dA >= n);
-	for (int j = threadIdx.x; j < n; j += NT3)
-		inv_s[j] = cached ? a.sA->dA[j] : T(1) / gA.at(a.ai + j, a.aj + j);
-
-	const int mt = (m + TM - 1) / TM;
-	const int nb = (n + 15) / 16;
-	for (int t = t0; t < mt; t += tstep)
-	{
-		const int i0 = t * TM;
-		const int mv = min(TM, m - i0);
-		__syncthreads();
-		// X <- alpha * B(row block, :)
-		g2s<T, PS, NT3, false>(gB, a.bi + i0, a.bj, TM, nb * 16, mv, n, Xs, LDX);
-		__syncthreads();
-		if (alpha != T(1))   // (x * 1 == x: nothing to do for alpha = 1)
-			for (int e = threadIdx.x; e < nb * 16 * LDX; e += NT3)
-				Xs[e] *= alpha;
-		for (int cb = 0; cb < nb; cb++)
-		{
-			const int c0 = cb * 16;
-			const int cv = min(16, n - c0);
-			// diagonal block of A (zero outside the valid triangle): loaded
-			// here, stored to LDS after the update below, so that its load
-			// latency overlaps the update (NT3 = 256 threads, one element each)
-			__syncthreads();
-			T adv;
-			{
-				const int r = threadIdx.x & 15, c = threadIdx.x >> 4;
-				adv = (r < cv && c < cv && r > c) ? gA.at(a.ai + c0 + r, a.aj + c0 + c) : T(0);
-			}
-			// X(:, c0:c0+16) -= X(:, 0:c0) * A(c0:c0+16, 0:c0)^T ; wave w owns rows 16w..16w+15.
-			// A is read from global memory four K steps (16 columns) at a time
-			// with the next four in flight; c0 is a multiple of 16, so no
-			// step runs past it.  The products are accumulated in the same
-			// order as one step at a time.
-			if (c0 > 0)
-			{
-				V4 acc = V4{0, 0, 0, 0};
-				const int jrow = a.ai + c0 + (lane & 15);
-				const bool jok = (lane & 15) < cv;
-				T bn[4];
-#pragma unroll
-				for (int u = 0; u < 4; u++)
-					bn[u] = jok ? gA.at(jrow, a.aj + 4 * u + (lane >> 4)) : T(0);
-				for (int kk = 0; kk < c0; kk += 16)
-				{
-					T bv[4], av[4];
-#pragma unroll
-					for (int u = 0; u < 4; u++)
-						bv[u] = bn[u];
-					if (kk + 16 < c0)
-#pragma unroll
-						for (int u = 0; u < 4; u++)
-							bn[u] = jok ? gA.at(jrow, a.aj + kk + 16 + 4 * u + (lane >> 4)) : T(0);
-#pragma unroll
-					for (int u = 0; u < 4; u++)
-						av[u] = Xs[(kk + 4 * u + (lane >> 4)) * LDX + 16 * w + (lane & 15)];
-#pragma unroll
-					for (int u = 0; u < 4; u++)
-						acc = mfma16(av[u], bv[u], acc);
-				}
-#pragma unroll
-				for (int r = 0; r < 4; r++)
-				{
-					const int il = 16 * w + acc_row<T>(lane, r);
-					const int jl = c0 + (lane & 15);
-					Xs[jl * LDX + il] -= acc[r];
-				}
-			}
-			Ad[(threadIdx.x & 15) * 17 + (threadIdx.x >> 4)] = adv;
-			__syncthreads();
-			// triangular solve of the 16 columns, one row per thread of wave 0
-			if (w == 0)
-			{
-				const int il = lane;
-				T x[16];
-#pragma unroll
-				for (int j = 0; j < 16; j++)
-					x[j] = Xs[(c0 + j) * LDX + il];
-#pragma unroll
-				for (int j = 0; j < 16; j++)
-				{
-					if (j < cv)
-					{
-						T c = x[j];
-#pragma unroll
-						for (int l = 0; l < j; l++)
-							c -= x[l] * Ad[j * 17 + l];
-						x[j] = c * inv_s[c0 + j];
-					}
-				}
-#pragma unroll
-				for (int j = 0; j < 16; j++)
-					Xs[(c0 + j) * LDX + il] = x[j];
-			}
-		}
-		__syncthreads();
-		s2g<T, PS, NT3, false>(gD, a.di + i0, a.dj, mv, n, Xs, LDX, 0);
-	}
-}
-
-// With a queue (count != nullptr) the launch is persistent: each workgroup
-// takes instances from the list (one atomic per instance on *head) and
-// solves all their row blocks; otherwise instance blockIdx.x, row blocks
-// blockIdx.y, blockIdx.y + gridDim.y, ...
-template <typename T, int PS, bool DA_GIVEN = false>
-__global__ __launch_bounds__(NT3) void k_trsm_rltn(const typename TrsmArg<T>::type *__restrict__ args, int nmax,
-	const int *__restrict__ count, const int *__restrict__ list, int *head)
-{
-	extern __shared__ unsigned char smem_raw[];
-	T *Xs = reinterpret_cast<T *>(smem_raw);      // [npad][LDX] column-major row block
-	__shared__ T inv_s[TRSM_NMAX];
-	__shared__ T Ad[16 * 17];                       // diagonal 16x16 block of A
-	__shared__ int qslot;
-	if (!count)
-	{
-		trsm_rltn_instance<T, PS, DA_GIVEN>(args[blockIdx.x], nmax, blockIdx.y, gridDim.y, Xs, inv_s, Ad);
-		return;
-	}
-	const int cnt = *count;
-	for (;;)
-	{
-		__syncthreads();   // every thread has read the previous slot
-		if (threadIdx.x == 0)
-			qslot = atomicAdd(head, 1);
-		__syncthreads();
-		const int t = qslot;
-		if (t >= cnt)
-			break;
-		trsm_rltn_instance<T, PS, DA_GIVEN>(args[list[t]], nmax, 0, 1, Xs, inv_s, Ad);
-	}
 }
 
 // ---------------------------------------------------------------------------
@@ -673,72 +509,44 @@ static int launch_trmm(int ps, int batch, const typename TrsmArg<T>::type *args,
 	return check_launch(name);
 }
 
-// trsm_rltn's instances sorted by n into buckets of 64 columns, so that each
-// bucket's launch sizes its LDS row block for that bucket: 64 columns take
-// 37 KB (four workgroups per CU), 128 take 71 KB (two), 256 take 137 KB
-// (one).  counts[0..TRSM_NB-1] and the queue heads counts[16..] start at 0.
-constexpr int TRSM_NB = TRSM_NMAX / 64;
-__global__ void k_trsm_zero(int *ws)
+// trsm_rltn: one launch per range of n, up to 64, 128 and 256 columns (the
+// registers that hold a strip, and with them the waves per SIMD, go with the
+// range), the largest first; a workgroup whose instance is not in its launch's
+// range leaves at once.
+template <typename T, int PS, int NB, bool GIVEN>
+static int launch_trsm_nb(int batch, const typename TrsmArg<T>::type *args, int mmax, int nlo, int nmax, hipStream_t st, const char *name)
 {
-	if (threadIdx.x < 64)
-		ws[threadIdx.x] = 0;
-}
-template <typename T>
-__global__ void k_trsm_plan(const typename TrsmArg<T>::type *__restrict__ args, int batch, int *counts, int *lists)
-{
-	const int i = blockIdx.x * blockDim.x + threadIdx.x;
-	const int n = i < batch ? args[i].n : 0;
-	plan_bucket<TRSM_NB>(i, i < batch ? (n <= 64 ? 0 : min(TRSM_NB - 1, (n - 1) / 64)) : -1, batch, counts, lists);
-}
-
-// the batched entry: plan, then one persistent launch per n bucket, largest
-// first (measured on 16384 calls of m, n ~ U{16..256} against one launch
-// sized for the hint's n)
-template <typename T, int PS>
-static int launch_trsm_ps(int batch, const typename TrsmArg<T>::type *args, int npad, hipStream_t st, const char *name)
-{
-	const size_t wsbytes = sizeof(int) * (64 + (size_t)TRSM_NB * batch);
-	int *ws = (int *)workspace(wsbytes, st);
-	if (!ws)
-		return set_error(BLASFEO_AMD_ENOMEM, "%s: cannot allocate the %zu-byte plan workspace", name, wsbytes);
-	int *counts = ws, *heads = ws + 16, *lists = ws + 64;
-	hipLaunchKernelGGL(k_trsm_zero, dim3(1), dim3(64), 0, st, ws);
-	hipLaunchKernelGGL((k_trsm_plan<T>), dim3((batch + 255) / 256), dim3(256), 0, st, args, batch, counts, lists);
-	int rc = check_launch(name);
+	constexpr int rows = 64 * trsm_strips<NB>();
+	const int slots = mmax > 0 ? min(64, (mmax + rows - 1) / rows) : 4;
+	constexpr size_t shm = trsm_lds<T, NB>();
+	dim3 grid;
+	int rc = xcd_grid(batch, slots, NT3, &grid, name);
+	if (!rc)
+		rc = lds_check(reinterpret_cast<const void *>(&k_trsm_rltn<T, PS, NB, GIVEN>), shm, name);
 	if (rc)
 		return rc;
-	const int cus = num_cus() > 0 ? num_cus() : 256;
-	constexpr size_t static_lds = sizeof(T) * (TRSM_NMAX + 16 * 17) + sizeof(int);
-	for (int b = TRSM_NB - 1; b >= 0; b--)
-	{
-		if (64 * b >= npad)
-			continue;   // n beyond the hint: no instance runs (as in the unbucketed launch)
-		const int np = min(64 * (b + 1), npad);
-		const size_t shm = (size_t)np * LDX * sizeof(T);
-		// at most four workgroups per CU (registers: four waves per SIMD)
-		const int per_cu = max(1, min(4, (int)(163840 / (shm + static_lds))));
-		const int grid = min(batch, per_cu * cus);
-		if ((rc = lds_check(reinterpret_cast<const void *>(&k_trsm_rltn<T, PS>), shm, name)))
-			return rc;
-		hipLaunchKernelGGL((k_trsm_rltn<T, PS>), dim3(grid), dim3(NT3), shm, st, args, np, counts + b,
-			lists + (size_t)b * batch, heads + b);
-		if ((rc = check_launch(name)))
-			return rc;
-	}
+	hipLaunchKernelGGL((k_trsm_rltn<T, PS, NB, GIVEN>), grid, dim3(NT3), shm, st, args, batch, slots, nlo, nmax);
+	return check_launch(name);
+}
+template <typename T, int PS, bool GIVEN = false>
+static int launch_trsm_ps(int batch, const typename TrsmArg<T>::type *args, const blasfeo_amd_hint *hint, hipStream_t st, const char *name)
+{
+	const int nmax = (hint->max_n + 15) / 16 * 16;
+	int rc = 0;
+	if (nmax > 128)
+		rc = launch_trsm_nb<T, PS, 16, GIVEN>(batch, args, hint->max_m, 128, nmax, st, name);
+	if (!rc && nmax > 64)
+		rc = launch_trsm_nb<T, PS, 8, GIVEN>(batch, args, hint->max_m, 64, nmax, st, name);
+	if (!rc)
+		rc = launch_trsm_nb<T, PS, 4, GIVEN>(batch, args, hint->max_m, 0, nmax, st, name);
+	if (rc || GIVEN)
+		return rc;
 	hipLaunchKernelGGL((k_trsm_dA<T, PS, false>), dim3(batch), dim3(64), 0, st, args);
 	return check_launch(name);
 }
 
-// the solve of the rows below the diagonal block in the trapezoid Cholesky:
-// reciprocals from sA->dA, no cache update (the caller sets use_dA)
-template <int PS>
-static int launch_trsm_given(int batch, const blasfeo_amd_dtrsm_arg *args, dim3 grid, size_t shm, int nmax, hipStream_t st, const char *name)
-{
-	hipLaunchKernelGGL((k_trsm_rltn<double, PS, true>), grid, dim3(NT3), shm, st, args, nmax, (const int *)nullptr,
-		(const int *)nullptr, (int *)nullptr);
-	return check_launch(name);
-}
-
+// given: the solve of the rows below the diagonal block in the trapezoid
+// Cholesky: reciprocals from sA->dA, no cache update (the caller sets use_dA)
 template <typename T>
 static int launch_trsm(int ps, int batch, const typename TrsmArg<T>::type *args, const blasfeo_amd_hint *hint, hipStream_t st, const char *name, bool given = false)
 {
@@ -749,23 +557,17 @@ static int launch_trsm(int ps, int batch, const typename TrsmArg<T>::type *args,
 		return set_error(BLASFEO_AMD_EINVAL, "%s: hint->max_n (upper bound of n) is required", name);
 	if (hint->max_n > TRSM_NMAX)
 		return set_error(BLASFEO_AMD_ETOOBIG, "%s: n up to %d supported, got %d", name, TRSM_NMAX, hint->max_n);
-	const int npad = (hint->max_n + 15) / 16 * 16;
-	const size_t shm = (size_t)npad * LDX * sizeof(T);
-	const int gy = hint->max_m > 0 ? min(64, (hint->max_m + TM - 1) / TM) : 1;
-	dim3 grid(batch, gy);
-	if (given)
-	{
-		if (sizeof(T) != 8 || (ps != 4 && ps != 8))
-			return set_error(BLASFEO_AMD_EINVAL, "%s: unsupported panel size %d", name, ps);
-		const blasfeo_amd_dtrsm_arg *d = reinterpret_cast<const blasfeo_amd_dtrsm_arg *>(args);
-		return ps == 4 ? launch_trsm_given<4>(batch, d, grid, shm, npad, st, name)
-		               : launch_trsm_given<8>(batch, d, grid, shm, npad, st, name);
-	}
+	if constexpr (sizeof(T) == 8)
+		if (given)
+			return ps == 4 ? launch_trsm_ps<T, 4, true>(batch, args, hint, st, name)
+			               : launch_trsm_ps<T, 8, true>(batch, args, hint, st, name);
 	if (ps == 4)
-		return launch_trsm_ps<T, 4>(batch, args, npad, st, name);
+		return launch_trsm_ps<T, 4>(batch, args, hint, st, name);
 	if (ps == 8)
-		return launch_trsm_ps<T, 8>(batch, args, npad, st, name);
-	return launch_trsm_ps<T, 16>(batch, args, npad, st, name);
+		return launch_trsm_ps<T, 8>(batch, args, hint, st, name);
+	if constexpr (sizeof(T) == 4)
+		return launch_trsm_ps<T, 16>(batch, args, hint, st, name);
+	return BLASFEO_AMD_EINVAL;
 }
 
 template <typename T, int PS, int MODE>

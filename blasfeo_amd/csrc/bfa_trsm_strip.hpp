@@ -1,0 +1,278 @@
+// bfa_trsm_strip.hpp -- trsm_rltn (D = alpha * B * A^{-T}, A lower n x n,
+// blasfeo_ref/x_blas3_ref.c:1642-1752) with the 16-row strips of B in registers
+// (bfa_strip.hpp).
+//
+// A wave holds S strips from their first block column to the last: block K is
+// alpha B_K minus the products of the finished blocks with the row block A_K, then
+// the solve with A_KK.  The four waves of a workgroup walk the block columns
+// together: the tiles of row block A_K are brought to LDS once for all of them, as
+// operand tiles, dealt to the waves and loaded one block column ahead (read by
+// every wave for itself they came from L2 at a rate that bound the kernel).
+// Per block column one barrier.
+// Measured (MI355X, 8192 FP64 solves, ps = 4; before: the row block in LDS, one of
+// four waves solving the diagonal blocks): m = n = 32 125 -> 54 us, 64 235 -> 159,
+// 128 1608 -> 795, 256 15.3 -> 4.4 ms (31 TFLOP/s; 6.2 ms with every wave reading
+// A for itself); m, n ~ U{16..256} 4.61 -> 2.15 ms.  Bound by memory up to 64
+// columns, then by the matrix cores and the substitution's vector instructions,
+// with two waves per SIMD.
+#pragma once
+#include "bfa_strip.hpp"
+#include "bfa_gemm_core.hpp"
+
+namespace bfa {
+
+constexpr int TRSM_NMAX = 256;
+
+// Strips per wave for NB block columns: NB S block accumulators stay in registers.
+template <int NB> constexpr int trsm_strips() { return NB == 8 ? 2 : 1; }
+// The whole triangle of A in LDS?
+template <int NB> constexpr bool trsm_whole() { return NB <= 4; }
+template <typename T, int NB>
+constexpr size_t trsm_lds()
+{
+	return sizeof(T) * 256 * (trsm_whole<NB>() ? NB * (NB + 1) / 2 : 2 * NB);
+}
+// Waves per SIMD that the kernel is compiled for.
+template <typename T, int NB>
+constexpr int trsm_waves()
+{
+	return sizeof(T) * NB * trsm_strips<NB>() <= 64 ? 3 : 2;
+}
+
+// Workgroup (instance, slot) solves the blocks of 64 S rows slot, slot + slots, ...
+// of its instance; instances with n outside (nlo, 16 NB] belong to another launch.
+// DA_GIVEN: the reciprocal diagonal is read from sA->dA whatever use_dA says
+// (the trapezoid Cholesky, whose diagonal block was just factored into the same
+// descriptor with its reciprocals stored there).
+template <typename T, int PS, int NB, bool DA_GIVEN>
+__global__ __launch_bounds__(NT3, (trsm_waves<T, NB>())) void k_trsm_rltn(const typename TrsmArg<T>::type *__restrict__ args,
+	int batch, int slots, int nlo, int nmax)
+{
+	typedef typename Vec4<T>::type V4;
+	constexpr int S = trsm_strips<NB>(), NW = NT3 / WAVE, NT = NB / NW;
+	extern __shared__ unsigned char smem_raw[];
+	T *tiles = reinterpret_cast<T *>(smem_raw);
+	__shared__ T inv_s[16 * NB];
+	const unsigned li = xcd_local_index(blockIdx.x, gridDim.x);
+	const int inst = (int)(li / (unsigned)slots), slot = (int)(li % (unsigned)slots);
+	if (inst >= batch)
+		return;
+	const typename TrsmArg<T>::type &a = args[inst];
+	const int m = __builtin_amdgcn_readfirstlane(a.m), n = __builtin_amdgcn_readfirstlane(a.n);
+	if (m <= 0 || n <= nlo || n > nmax || n > 16 * NB || slot * 64 * S >= m)
+		return;
+	const StripView<T, PS> A = strip_view<T, PS>(a.sA), B = strip_view<T, PS>(a.sB), D = strip_view<T, PS>(a.sD);
+	const int ai = a.ai, aj = a.aj;
+	const T alpha = a.alpha;
+	// reciprocal diagonal: cached copy when valid at launch, else 1/A_jj
+	// (an output aliasing A invalidates the cache first, as in the reference)
+	const bool cached = DA_GIVEN || (ai == 0 && aj == 0 && a.sD != a.sA && a.sA->use_dA >= n);
+	const BFA_GLOBAL T *dA = (const BFA_GLOBAL T *)a.sA->dA;
+	for (int j = threadIdx.x; j < 16 * NB; j += NT3)
+		inv_s[j] = j < n ? (cached ? dA[j] : T(1) / A.ld(0, A.at(ai + j, aj + j))) : T(0);
+	const int w = __builtin_amdgcn_readfirstlane(wave_id());
+	const int lane = lane_id(), g = lane >> 4, c = lane & 15, rid = strip_row<T>(c);
+	const int nb = (n + 15) / 16;
+	// where this lane's entries of the 4 x 4 triangles of A_KK (strip_solve) are
+	// in the diagonal tile: entry (4 s + tr, 4 s + tc)
+	const int tr = c >> 2, tc = c & 3;
+	int trio[4];
+#pragma unroll
+	for (int s = 0; s < 4; s++)
+		trio[s] = 64 * s + 16 * tc + strip_row<T>(4 * s + tr);
+	if constexpr (trsm_whole<NB>())
+	{
+		// tile (K, p) at 256 (K (K + 1) / 2 + p), dealt round-robin to the waves
+		constexpr int NTT = (NB * (NB + 1) / 2 + NW - 1) / NW;
+		const int ntile = nb * (nb + 1) / 2;
+		T ta[NTT][4];
+#pragma unroll
+		for (int t = 0; t < NTT; t++)
+			if (w + NW * t < ntile)
+			{
+				int p = w + NW * t, K = 0;
+				while (p > K)
+					p -= ++K;
+				strip_load<4>(A, A.at(ai + min(16 * K + rid, n - 1), aj + g), g, 16 * p, n, ta[t]);
+			}
+		bool first = true;
+		for (int r0 = slot * 64 * S; r0 < m; r0 += slots * 64 * S)
+		{
+			int row[S];
+			V4 nx[S][NB];   // alpha B, then -X of the finished blocks
+#pragma unroll
+			for (int t = 0; t < S; t++)
+			{
+				row[t] = r0 + 16 * (S * w + t) + rid;
+				const unsigned ob = B.at(a.bi + min(row[t], m - 1), a.bj + g);
+#pragma unroll
+				for (int K = 0; K < NB; K++)
+					if (K < nb)
+						strip_load<4>(B, ob, g, 16 * K, n, nx[t][K]);
+			}
+			if (first)
+			{
+#pragma unroll
+				for (int t = 0; t < NTT; t++)
+					if (w + NW * t < ntile)
+#pragma unroll
+						for (int s = 0; s < 4; s++)
+							tiles[256 * (w + NW * t) + 64 * s + lane] = ta[t][s];
+				__syncthreads();
+				first = false;
+			}
+			// the waves past the last row have shared in the loads above
+			if (r0 + 16 * S * w >= m)
+				continue;
+#pragma unroll
+			for (int K = 0; K < NB; K++)
+				if (K < nb)
+				{
+					const T *buf = tiles + 256 * (K * (K + 1) / 2);
+					T lk[3], d[4];
+#pragma unroll
+					for (int s = 0; s < 3; s++)
+						lk[s] = buf[256 * K + 64 * s + lane];
+#pragma unroll
+					for (int s = 0; s < 4; s++)
+						d[s] = tr == tc ? inv_s[16 * K + 4 * s + tc] : buf[256 * K + trio[s]];
+					V4 acc[S];
+#pragma unroll
+					for (int t = 0; t < S; t++)
+						acc[t] = alpha * nx[t][K];
+#pragma unroll
+					for (int p = 0; p < K; p++)
+					{
+						T l[4];
+#pragma unroll
+						for (int s = 0; s < 4; s++)
+							l[s] = buf[256 * p + 64 * s + lane];
+#pragma unroll
+						for (int s = 0; s < 4; s++)
+#pragma unroll
+							for (int t = 0; t < S; t++)
+								acc[t] = mfma16(l[s], nx[t][p][s], acc[t]);
+					}
+					T x[S][4];
+					if constexpr (S == 2)
+						strip_solve2<T>(acc[0], acc[1], lk, d, x[0], x[1]);
+					else
+						strip_solve<T>(acc[0], lk, d, x[0]);
+#pragma unroll
+					for (int t = 0; t < S; t++)
+					{
+						const unsigned od = D.at(a.di + min(row[t], m - 1), a.dj + g);
+						strip_store(D, od, g, 16 * K, n, row[t] < m, x[t]);
+#pragma unroll
+						for (int s = 0; s < 4; s++)
+							nx[t][K][s] = -x[t][s];
+					}
+				}
+		}
+		return;
+	}
+	// tiles w, w + NW, ... of row block K, loaded into registers and, a block
+	// column later, to LDS
+	T st[NT][4];
+	auto fetch = [&](int K) {
+		const unsigned ol = A.at(ai + min(16 * K + rid, n - 1), aj + g);
+#pragma unroll
+		for (int t = 0; t < NT; t++)
+			if (w + NW * t <= K)
+				strip_load<4>(A, ol, g, 16 * (w + NW * t), n, st[t]);
+	};
+	auto stage = [&](int K) {
+		T *buf = tiles + (K & 1) * (NB * 256);
+#pragma unroll
+		for (int t = 0; t < NT; t++)
+			if (w + NW * t <= K)
+#pragma unroll
+				for (int s = 0; s < 4; s++)
+					buf[256 * (w + NW * t) + 64 * s + lane] = st[t][s];
+	};
+	for (int r0 = slot * 64 * S; r0 < m; r0 += slots * 64 * S)
+	{
+		int row[S];
+		unsigned ob[S];
+		V4 nx[S][NB], cn[S];
+#pragma unroll
+		for (int t = 0; t < S; t++)
+		{
+			row[t] = r0 + 16 * (S * w + t) + rid;
+			ob[t] = B.at(a.bi + min(row[t], m - 1), a.bj + g);
+			strip_load<4>(B, ob[t], g, 0, n, cn[t]);
+		}
+		fetch(0);
+		stage(0);
+		__syncthreads();
+#pragma unroll 1
+		for (int K = 0; K < nb; K++)
+		{
+			const T *buf = tiles + (K & 1) * (NB * 256);
+			V4 acc[S];
+#pragma unroll
+			for (int t = 0; t < S; t++)
+				acc[t] = alpha * cn[t];
+			if (K + 1 < nb)
+			{
+				fetch(K + 1);
+#pragma unroll
+				for (int t = 0; t < S; t++)
+					strip_load<4>(B, ob[t], g, 16 * (K + 1), n, cn[t]);
+			}
+			T lk[3], d[4];
+#pragma unroll
+			for (int s = 0; s < 3; s++)
+				lk[s] = buf[256 * K + 64 * s + lane];
+#pragma unroll
+			for (int s = 0; s < 4; s++)
+				d[s] = tr == tc ? inv_s[16 * K + 4 * s + tc] : buf[256 * K + trio[s]];
+#pragma unroll
+			for (int p = 0; p < NB - 1; p++)
+				if (p < K)
+				{
+					T l[4];
+#pragma unroll
+					for (int s = 0; s < 4; s++)
+						l[s] = buf[256 * p + 64 * s + lane];
+#pragma unroll
+					for (int s = 0; s < 4; s++)
+#pragma unroll
+						for (int t = 0; t < S; t++)
+							acc[t] = mfma16(l[s], nx[t][p][s], acc[t]);
+				}
+			T x[S][4];
+			if constexpr (S == 2)
+				strip_solve2<T>(acc[0], acc[1], lk, d, x[0], x[1]);
+			else
+				strip_solve<T>(acc[0], lk, d, x[0]);
+#pragma unroll
+			for (int t = 0; t < S; t++)
+			{
+				V4 y;
+#pragma unroll
+				for (int s = 0; s < 4; s++)
+					y[s] = -x[t][s];
+				strip_set(nx[t], K, y);
+			}
+			if (K + 1 < nb)
+				stage(K + 1);
+			__syncthreads();
+		}
+		// (pinned: the column masks of all blocks would be formed at the start
+		// and kept in registers)
+		int ge = g;
+		BFA_PIN(ge);
+#pragma unroll
+		for (int t = 0; t < S; t++)
+		{
+			const unsigned od = D.at(a.di + min(row[t], m - 1), a.dj + g);
+#pragma unroll
+			for (int K = 0; K < NB; K++)
+				if (K < nb)
+					strip_store(D, od, ge, 16 * K, n, row[t] < m, -nx[t][K]);
+		}
+	}
+}
+
+} // namespace bfa

@@ -1,7 +1,8 @@
 """Emulator cases (TEST INFRASTRUCTURE ONLY) for the left-side solves on the
 record sets of the GPU tests (tests/trsm_cases.py), checked against the
 oracle element for element (NaN and Inf included).
-Usage: python case_trsm.py nonfinite <op> <thin: 0|1>"""
+Usage: python case_trsm.py nonfinite <op> <thin: 0|1>
+       python case_trsm.py rltn <ps> <finite: 0|1>   (trsm_rltn, trsm_cases.rltn)"""
 import ctypes
 import sys
 
@@ -14,12 +15,17 @@ import trsm_cases
 def run(op, thin):
     ps = 4
     E = emu_lib("emu_lapack")
-    re, ro = to_mats(ps, trsm_cases.nonfinite(ps, op, 970 + 3 * len(op) + thin))
-    blk = records(bfa.DTRSM_ARG, re)
-    print("emu %s nonfinite thin=%d batch=%d" % (op, thin, len(re)), flush=True)
     assert E.blasfeo_amd_tune_set(b"trsm_thin", 0, 1 if thin else 2) == 0
+    print("thin=%d" % thin)
+    check(E, op, ps, trsm_cases.nonfinite(ps, op, 970 + 3 * len(op) + thin), (256, 4, 0))
+
+
+def check(E, op, ps, cases, hint):
+    re, ro = to_mats(ps, cases)
+    blk = records(bfa.DTRSM_ARG, re)
+    print("emu %s ps=%d batch=%d" % (op, ps, len(re)), flush=True)
     rc = getattr(E, "blasfeo_amd_d%s_batched" % op)(ps, len(re), ctypes.c_void_p(blk.addr),
-                                                    ctypes.byref(bfa.HINT(256, 4, 0)), None)
+                                                    ctypes.byref(bfa.HINT(*hint)), None)
     assert rc == 0, E.emu_last_error()
     f = oracle.fn("d", op)
     for r in ro:
@@ -37,5 +43,9 @@ def run(op, thin):
 
 
 if __name__ == "__main__":
-    assert sys.argv[1] == "nonfinite"
-    run(sys.argv[2], int(sys.argv[3]))
+    if sys.argv[1] == "rltn":
+        psz, fin = int(sys.argv[2]), int(sys.argv[3])
+        check(emu_lib("emu_lapack"), "trsm_rltn", psz, trsm_cases.rltn(psz, 990 + psz, bool(fin)), (130, 256, 0))
+    else:
+        assert sys.argv[1] == "nonfinite"
+        run(sys.argv[2], int(sys.argv[3]))

@@ -71,6 +71,14 @@ def test_potrf_one_wave(emu_build, case, ps):
     run_case("case_chol.py", case, ps)
 
 
+@pytest.mark.parametrize("finite", [1, 0])
+@pytest.mark.parametrize("ps", [4, 8])
+def test_trsm_rltn(emu_build, ps, finite):
+    """trsm_rltn at the edges of strips, workgroups, blocks and launches; with a
+    zero pivot, an Inf or a NaN, non-finite only where the reference is."""
+    run_case("case_trsm.py", "rltn", ps, finite)
+
+
 @pytest.mark.parametrize("ps", [4, 8])
 def test_potrf_global_kernel(emu_build, ps):
     """k_potrf (potrf_l for n > 256; 16-column panels at full height, the

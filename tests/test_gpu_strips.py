@@ -1,6 +1,6 @@
 """GPU parity of the kernels that keep 16-row strips in registers, at the edges of
 their strips, blocks and launches, against the CPU oracle: potrf_l(_mn) with one
-and with several waves per instance, syrk_dpotrf_ln."""
+and with several waves per instance, syrk_dpotrf_ln, trsm_rltn."""
 import numpy as np
 import pytest
 
@@ -9,6 +9,7 @@ import oracle
 from blasfeo_amd import autotune
 from helpers import Batch, run_both, compare_buffers
 import chol_cases
+import trsm_cases
 
 pytestmark = pytest.mark.gpu
 
@@ -88,4 +89,28 @@ def test_syrk_potrf(gpu, ps, bound):
 
     g, gd, rr, rd = run_both(b, b.host(), bfa.DSYRK_DPOTRF_ARG, recs, "dsyrk_dpotrf_ln", ocall, (bound, bound, 70))
     compare_buffers(b, g, rr, "syrk_dpotrf_ln")
+    assert (gd["use_dA"] == rd["use_dA"]).all()
+
+
+@pytest.mark.parametrize("finite", [True, False])
+@pytest.mark.parametrize("prec,ps", [(p, q) for p in "ds" for q in _panel_sizes(p)])
+def test_trsm_rltn(gpu, prec, ps, finite):
+    b = Batch(prec, ps, seed=6)
+    recs = chol_cases.to_batch(b, trsm_cases.rltn(ps, 100 + ps, finite))
+    f = oracle.fn(prec, "trsm_rltn")
+
+    def ocall(h, r):
+        f(ps, r["m"], r["n"], r["alpha"], h.desc_addr(r["sA"]), r["ai"], r["aj"], h.desc_addr(r["sB"]), r["bi"], r["bj"],
+          h.desc_addr(r["sD"]), r["di"], r["dj"])
+
+    with np.errstate(invalid="ignore"):
+        g, gd, rr, rd = run_both(b, b.host(), bfa.DTRSM_ARG if prec == "d" else bfa.STRSM_ARG, recs, prec + "trsm_rltn", ocall, (130, 256, 0))
+        if finite:
+            compare_buffers(b, g, rr, "trsm_rltn")
+        else:
+            for i in range(len(b.layout)):
+                x, y = b.layout.view(g, i), b.layout.view(rr, i)
+                tol = 1e-11 if prec == "d" else 9e-4
+                same = (x == y) | (np.isnan(x) & np.isnan(y)) | (np.abs(x - y) <= tol * (np.abs(x) + np.abs(y)) + tol)
+                assert same.all(), "matrix %d: %d differ" % (i, int((~same).sum()))
     assert (gd["use_dA"] == rd["use_dA"]).all()

@@ -34,3 +34,38 @@ def nonfinite(ps, op, seed):
         mats = {"sA": (ai + m, aj + m, Ad), "sB": (bi + m, bj + n, Bd), "sD": (di + m, dj + n, -1.0)}
         out.append((mats, dict(m=m, n=n, ai=ai, aj=aj, bi=bi, bj=bj, di=di, dj=dj, alpha=1.0)))
     return out
+
+
+RLTN_SIZES = [(1, 1), (15, 16), (16, 17), (17, 15), (64, 64), (65, 63), (129, 65), (127, 128), (33, 129), (80, 144), (16, 255), (130, 256)]
+
+
+def rltn(ps, seed, finite=True):
+    """trsm_rltn at the edges of its strips (16 rows), workgroups (64 and 128
+    rows), blocks (16 columns) and launches (64, 128, 256 columns), offsets, in
+    place on every fourth instance; finite=False: a zero on A's diagonal in
+    some, an Inf or a NaN in B in the others (the columns solved before it keep
+    their values, as in the reference)."""
+    rng = np.random.default_rng(seed)
+    out = []
+    for r, (m, n) in enumerate(RLTN_SIZES):
+        ai, bi, di = (int(x) for x in rng.integers(0, 2 * ps, 3))
+        aj, bj, dj = (int(x) for x in rng.integers(0, 3, 3))
+        if r % 3 == 0:
+            ai = aj = 0
+        T = np.tril(rng.standard_normal((n, n)) * (0.5 / np.sqrt(n)), -1) + np.diag(1.0 + rng.uniform(0, 1, n))
+        if not finite and r % 2 == 0:
+            z = int(rng.integers(0, n))
+            T[z, z] = 0.0
+        Ad = np.full((ai + n, aj + n), 1e3)
+        Ad[ai:, aj:] = T + 1e3 * np.triu(np.ones((n, n)), 1)
+        Bd = rng.standard_normal((bi + m, bj + n))
+        if not finite and r % 2 == 1:
+            Bd[bi + int(rng.integers(0, m)), bj + int(rng.integers(0, n))] = np.inf if r % 4 == 1 else np.nan
+        mats = {"sA": (ai + n, aj + n, Ad), "sB": (bi + m, bj + n, Bd)}
+        if r % 4 == 3:
+            mats["sD"] = "=sB"
+            di, dj = bi, bj
+        else:
+            mats["sD"] = (di + m, dj + n, -1.0)
+        out.append((mats, dict(m=m, n=n, ai=ai, aj=aj, bi=bi, bj=bj, di=di, dj=dj, alpha=[1.0, -0.5][r % 2])))
+    return out
