@@ -289,7 +289,7 @@ def run_riccati(args, torch, bfa):
         "roofline": {"bound": rbound, "achieved": rach, "peak": rpeak, "unit": runit,
                      "frac": rach / rpeak, "traffic": traffic,
                      "algorithmic_bytes": algo_bytes, "flops_per_launch": flops,
-                     "kernel": "k_ric_class<ps,256> + k_ric_class<ps,128> (the class launches of one batched call, run side by side)"},
+                     "kernel": "k_ric_coop<ps,NW> (the class launches of one batched call, run side by side)"},
         "cpu_baseline": cpu,
         "checks": checks,
     }
@@ -573,7 +573,7 @@ def run_ric_sv(args, torch, bfa):
            "roofline": {"bound": rbound, "achieved": rach, "peak": rpeak, "unit": runit,
                         "frac": rach / rpeak, "traffic": None,
                         "algorithmic_bytes": algo_bytes, "flops_per_launch": flops,
-                        "kernel": "k_ric_class<ps,NT,aug> class launches + k_ric_sv_fwd (factorisation flops only)"},
+                        "kernel": "k_ric_coop<ps,NW,NX,aug> class launches + k_ric_sv_fwd (factorisation flops only)"},
            "cpu_baseline": cpu, "checks": checks}
     print(json.dumps(out), flush=True)
 

@@ -26,15 +26,28 @@ _RT_SZ = 16 * 17
 
 
 def ric_footprint(nkmax, nxmax):
-    """LDS bytes of one instance in the resident Riccati sweep (the kernel's
-    rule: tiles, reciprocal pivots and the 16-byte work-queue slot)."""
+    """Bytes of one instance's stage matrices as lower and rectangular tiles of
+    doubles, reciprocal pivots and the 16-byte work-queue slot; the FP32 sweep
+    holds half of it in LDS."""
     nkt = (nkmax + 15) // 16
     nxt = (nxmax + 15) // 16
     return ((nkt * (nkt + 1) // 2 + nkt * nxt) * _RT_SZ + nkt * 16) * 8 + 16
 
 
+def ric_strip_class(nkmax, nxmax):
+    """Class of an instance of the FP64 sweep: the 16-row strips of its largest
+    stage, less one (0..7), or 8 for the global-memory sweep."""
+    return 8 if nxmax > 64 or nkmax > 128 else max(0, (nkmax + 15) // 16 - 1)
+
+
+def ric_strip_lds(cls, nt):
+    """LDS bytes of an instance of that class with nt threads."""
+    R, nx = cls + 1, 2 if nt == 64 else 4
+    return 8 * (2 + 128 + 128 + R * (R + 1) // 2 * _RT_SZ + cls * nx * 256)
+
+
 def ric_class(nkmax, nxmax):
-    """Footprint class of an instance (0..7), or 8 for the global-memory sweep."""
+    """Footprint class of an instance (0..7), or 8 where nothing holds it."""
     if nxmax > 64 or nkmax > 128:
         return 8
     f = ric_footprint(nkmax, nxmax)
@@ -104,15 +117,13 @@ def _time(torch, stream, fn, steps, warmup=1):
 
 
 def _ric_candidates(cls):
-    cap = RIC_CAPS[cls]
-    lds_fit = RIC_LDS // cap
     out = []
-    for nt in ((64, 128, 256) if cls <= 4 else (128, 256)):
-        # resident instances per CU: at most what LDS holds; more workgroups
-        # than that only queue behind the resident ones
-        waves_fit = 32 // (nt // 64)
-        top = max(1, min(lds_fit, waves_fit))
-        for pc in sorted({top, max(1, top // 2), max(1, (3 * top) // 4), min(top, 12), min(top, 8), min(top, 4)}):
+    # a wave holds two strips; the one-wave form serves two strips at most
+    for nt in [t for t in (64, 128, 256) if t // 64 * 2 >= cls + 1 and (t > 64 or cls < 2)]:
+        # resident instances per CU: at most what LDS and registers (two or
+        # three waves per SIMD) hold; more workgroups only queue behind them
+        top = max(1, min(RIC_LDS // ric_strip_lds(cls, nt), (12 if nt == 64 else 8) // (nt // 64)))
+        for pc in sorted({top, max(1, top // 2), max(1, (3 * top) // 4)}):
             out.append((nt, pc))
     return out
 
@@ -125,7 +136,7 @@ def tune_riccati(nxs, nus, N, ps_list=(4, 8), steps=3, seed=1, log=None):
     from .riccati import RiccatiBatch, DeviceRiccati
     nxs = np.asarray(nxs)
     nus = np.asarray(nus)
-    classes = np.array([ric_class(int(x + u), int(x)) for x, u in zip(nxs, nus)])
+    classes = np.array([ric_strip_class(int(x + u), int(x)) for x, u in zip(nxs, nus)])
     work = np.zeros(9)
     for c, x, u in zip(classes, nxs, nus):
         nk = x + u

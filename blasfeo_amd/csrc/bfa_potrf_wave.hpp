@@ -280,7 +280,7 @@ __device__ __forceinline__ void potrf_coop(int m, int n, int k, const StripView<
 		const int row = 16 * J + rid;
 		strip_store_diag(D, D.at(di + min(row, m - 1), dj + g), g, rid, 16 * J, n, row < m, l, dD, iv);
 	};
-	chol_coop<T, NW>(hi, lo, ih, il, R, Cb, lds, emit, emit_diag);
+	chol_coop<T, NW>(hi, lo, ih, il, Cb, CoopRing<T, NW>{lds, lane}, emit, emit_diag);
 }
 
 // Waves per SIMD that a kernel with NW waves per instance is compiled for.
@@ -294,7 +294,7 @@ template <typename T, int PS, int NW>
 __global__ __launch_bounds__(NW * WAVE, (coop_waves<T, NW>())) void k_potrf_coop(const typename FactArg<T>::type *__restrict__ args,
 	int mmax, bool mn)
 {
-	__shared__ T lds[coop_lds<T, NW>()];
+	__shared__ T lds[CoopRing<T, NW>::ELEMS];
 	const typename FactArg<T>::type &a = args[blockIdx.x];
 	const int m = __builtin_amdgcn_readfirstlane(a.m);
 	const int n = mn ? min(m, __builtin_amdgcn_readfirstlane(a.n)) : m;
@@ -310,7 +310,7 @@ __global__ __launch_bounds__(NW * WAVE, (coop_waves<T, NW>())) void k_potrf_coop
 template <typename T, int PS, int NW>
 __global__ __launch_bounds__(NW * WAVE, (coop_waves<T, NW>())) void k_syrk_potrf_coop(const typename SPArg<T>::type *__restrict__ args, int mmax)
 {
-	__shared__ T lds[coop_lds<T, NW>()];
+	__shared__ T lds[CoopRing<T, NW>::ELEMS];
 	const typename SPArg<T>::type &a = args[blockIdx.x];
 	const int m = __builtin_amdgcn_readfirstlane(a.m), k = __builtin_amdgcn_readfirstlane(a.k);
 	const int n = min(m, __builtin_amdgcn_readfirstlane(a.n));

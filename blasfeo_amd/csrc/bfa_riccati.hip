@@ -6,17 +6,18 @@
 //     W    = BAbt[k] * L[k+1](nu[k+1]:, nu[k+1]:)      (trmm_rlnn)
 //     L[k] = chol(RSQ[k] + W * W^T)                    (syrk_dpotrf_ln)
 //
-// Launch model (size-bucketed work queue):
-//   1. a plan kernel gives every instance an LDS footprint class from its
-//      largest stage and appends its index to that class's list;
-//   2. one persistent launch per class, largest first, the launches spread
-//      over the caller's stream and helper streams so that the classes run
-//      side by side; the workgroups of a launch pull instances from the
-//      class's atomic work queue.  Two or four waves per instance by default
-//      (one wave when the tuning knobs ask for it), a few instances per CU so
-//      that their latency chains overlap;
-//   3. instances too large for LDS (nx > 64 or footprint > 160 KB) take the
-//      general sweep, which keeps only a 16-column panel in LDS.
+// FP64 (trf, and sv with its augmented matrices): the stage matrix in registers,
+// one to four waves per instance (bfa_ric_coop.hpp).  FP32 (the mixed-precision
+// solve): the stage matrix in LDS (ric_sweep_lds).
+// Launch model where no single launch serves the batch (launch_ric_coop):
+//   1. a plan kernel gives every instance a class, its number of 16-row strips
+//      (FP32: its LDS footprint), and appends its index to that class's list;
+//   2. one persistent launch per class, spread over the caller's stream and helper
+//      streams so that the classes run side by side; the workgroups of a launch
+//      pull instances from the class's atomic work queue, a few instances per CU
+//      so that their latency chains overlap;
+//   3. FP64 instances too large for that (nx > 64 or nu+nx > 128) take the general
+//      sweep, which keeps only a 16-column panel in LDS.
 #include <mutex>
 #include <map>
 
@@ -27,22 +28,17 @@
 namespace bfa {
 
 constexpr int RIC_LDS_MAX = 163840;   // LDS bytes a workgroup may use on gfx950
-constexpr int RIC_NCLASS = 8;         // LDS-resident footprint classes
+constexpr int RIC_NCLASS = 8;         // classes: strips of the largest stage (FP32: LDS footprints)
 constexpr int RIC_GENERAL = RIC_NCLASS;
 constexpr int RIC_HEAD = 32;          // offset of the work-queue heads in the plan workspace
 static_assert(RIC_HEAD + RIC_NCLASS <= 64, "plan workspace header holds 64 ints");
-// class capacities in bytes: multiples of 1 KiB that divide the CU's LDS
+// FP32 class capacities in bytes: multiples of 1 KiB that divide the CU's LDS
 // into 20, 10, 6, 5, 4, 3, 2 and 1 resident instances
 __constant__ int c_ric_cap[RIC_NCLASS] = {8192, 16384, 24576, 32768, 40960, 54272, 81920, 163840};
 static const int h_ric_cap[RIC_NCLASS] = {8192, 16384, 24576, 32768, 40960, 54272, 81920, 163840};
 
-// LDS storage of the resident form: the stage matrix M as packed lower tiles
-// (TileLowerT, bfa_chol_core.hpp) and W as a rectangle of the same 16x17
-// tiles.  Against a square column-major M this keeps only the lower tiles,
-// so the largest stage (nu+nx = 80, nx = 64) needs 76,800 B and two
-// instances share a CU instead of one.
-typedef TileLowerT<double> TileLower;
-
+// LDS storage of the FP32 form: the stage matrix M as packed lower tiles
+// (TileLowerT, bfa_chol_core.hpp) and W as a rectangle of the same 16x17 tiles.
 template <typename T>
 struct TileRectT
 {
@@ -53,7 +49,6 @@ struct TileRectT
 		return p[((r >> 4) * nct + (c >> 4)) * RT_SZ + (c & 15) * RT_LD + (r & 15)];
 	}
 };
-typedef TileRectT<double> TileRect;
 
 // The first RIC_QSLOT bytes of a class kernel's dynamic LDS hold the work-queue
 // slot (bytes 0..3) and a 0.0 of the sweep's type (just before the sweep's M);
@@ -64,7 +59,7 @@ constexpr int RIC_QSLOT = 16;
 // LDS bytes of the resident form for an instance whose largest stage is
 // nkmax = max(nu+nx) and whose largest state is nxmax (queue slot included),
 // with esz-byte elements.
-__host__ __device__ __forceinline__ int ric_footprint(int nkmax, int nxmax, int esz = 8)
+__host__ __device__ __forceinline__ int ric_footprint(int nkmax, int nxmax, int esz)
 {
 	const int nkt = (nkmax + 15) / 16;
 	const int nxt = (nxmax + 15) / 16;
@@ -76,22 +71,6 @@ __host__ __device__ __forceinline__ int ric_footprint(int nkmax, int nxmax, int 
 //   M (packed lower tiles): L[k+1] at the start of stage k, then
 //     RSQ[k] + W W^T, then L[k]
 //   W (tile rectangle): BAbt[k], then W = BAbt[k] * L[k+1](nu1:, nu1:)
-// The two matrix-core stages of a Riccati step are inlined into the kernels
-// of two and four waves per instance.  The one-wave kernel calls them out of
-// line (inlined, their address arithmetic is hoisted across the whole sweep
-// and it needs 248 VGPRs + 64 AGPRs, one wave per SIMD), with the LDS base
-// passed opaquely (see lds_opaque).
-// An LDS address rebuilt from its 32-bit offset behind an empty asm: the
-// callee then keeps the base in a register instead of resolving the kernel's
-// dynamic-LDS variable through the offset table at every access.
-__device__ __forceinline__ double *lds_opaque(double *p)
-{
-	unsigned off = (unsigned)(size_t)(__attribute__((address_space(3))) double *)p;
-	asm volatile("" : "+v"(off));
-	off = __builtin_amdgcn_readfirstlane(off);
-	return (double *)(__attribute__((address_space(3))) double *)(size_t)off;
-}
-
 // ---------------------------------------------------------------------------
 // A value every lane holds, moved to a scalar register: loops and branches
 // that it controls are then uniform (scalar branches, no exec masking), so
@@ -209,35 +188,30 @@ struct RicChunk
 	typename Vec4<T>::type rq[4];
 };
 
-template <int NT, int PS, bool FROMG, bool AUG>
-__device__ __forceinline__ int ric_syrk_mine(int nkt, int nk)
+template <int NT>
+__device__ __forceinline__ int ric_syrk_mine(int nkt)
 {
 	constexpr int NW = NT / WAVE;
 	const int w = uni(wave_id());
-	const int mrt = AUG ? (nk + 1 + 15) / 16 : nkt;   // row tiles
-	int ntile = 0;
-	for (int bj = 0; bj < nkt; bj++)
-		ntile += mrt - bj;
+	const int ntile = nkt * (nkt + 1) / 2;
 	return (ntile - w + NW - 1) / NW;   // tiles w, w + NW, ...
 }
 
-template <int NT, int PS, bool FROMG, bool AUG, typename T>
+template <int NT, int PS, typename T>
 __device__ __forceinline__ void ric_syrk_chunk(RicChunk<T> &ch, int c0, int mine, int nkt, int nk,
 	const PM<double, PS> gR)
 {
 	constexpr int NW = NT / WAVE;
 	const int lane = lane_id();
 	const int w = uni(wave_id());
-	const int mrt = AUG ? (nk + 1 + 15) / 16 : nkt;
-	const int nrows = AUG ? nk + 1 : nk;
 	ch.cnt = min(4, mine - c0);
 #pragma unroll
 	for (int t = 0; t < 4; t++)
 	{
 		int q = w + NW * (c0 + min(t, ch.cnt - 1)), bj = 0;
-		while (q >= mrt - bj)
+		while (q >= nkt - bj)
 		{
-			q -= mrt - bj;
+			q -= nkt - bj;
 			bj++;
 		}
 		ch.I[t] = bj + q;
@@ -247,56 +221,45 @@ __device__ __forceinline__ void ric_syrk_chunk(RicChunk<T> &ch, int c0, int mine
 	for (int t = 0; t < 4; t++)
 	{
 		ch.rq[t] = typename Vec4<T>::type{0, 0, 0, 0};
-		if (FROMG && t < ch.cnt)
+		if (t < ch.cnt)
 		{
 			const int col = ch.J[t] * 16 + (lane & 15);
 #pragma unroll
 			for (int r = 0; r < 4; r++)
 			{
 				const int row = ch.I[t] * 16 + acc_row<T>(lane, r);
-				if (row < nrows && col < nk && row >= col)
+				if (row < nk && col < nk && row >= col)
 					ch.rq[t][r] = (T)gR.at(row, col);
 			}
 		}
 	}
 }
 
-// M += W W^T on the lower tiles (syrk_ln).  The lower tiles (I, J), I >= J,
-// numbered down the block columns, are dealt round-robin to the waves, which
+// M = lower(gR) + W W^T on the lower tiles (syrk_ln).  The lower tiles (I, J),
+// I >= J, numbered down the block columns, are dealt round-robin to the waves, which
 // take theirs four at a time, so the waves' shares differ by one tile at
-// most.  FROMG: M = lower(gR) + W W^T instead: the nk x nk lower triangle of
-// gR (global memory, zero elsewhere) is loaded into registers of its own
-// before the matrix-core steps and added after them, so that its latency
-// overlaps them and M needs no separate staging pass.
-// AUG: the (nk+1) x nk trapezoid of the fused sweep (one more row of W and
-// M, the linear-term row): row tiles of nk+1 rows, column tiles of nk
-// columns, and the columns from nk on written as zero (the Cholesky needs its
-// padding columns zero; W's row nk is not padding).
+// most.  The nk x nk lower triangle of gR (global memory, zero elsewhere) is
+// loaded into registers of its own before the matrix-core steps and added after
+// them, so that its latency overlaps them and M needs no separate staging pass.
 // W's columns from n1 on are zero (the trmm writes them so), so the inner
 // dimension runs over whole 16-column tiles.
-template <int NT, int PS = 4, bool FROMG = false, bool AUG = false, typename T = double>
+template <int NT, int PS, typename T>
 __device__ __forceinline__ void ric_syrk_m(const TileLowerT<T> M, const TileRectT<T> W, int nkt, int n1,
-	const PM<double, PS> gR = PM<double, PS>{}, int nk = 0)
+	const PM<double, PS> gR, int nk)
 {
 	typedef typename Vec4<T>::type V4;
 	const int lane = lane_id();
 	const int kt = (n1 + 15) / 16;
-	const int mine = ric_syrk_mine<NT, PS, FROMG, AUG>(nkt, nk);
+	const int mine = ric_syrk_mine<NT>(nkt);
 	for (int c0 = 0; c0 < mine; c0 += 4)
 	{
 		RicChunk<T> ch;
-		ric_syrk_chunk<NT, PS, FROMG, AUG, T>(ch, c0, mine, nkt, nk, gR);
+		ric_syrk_chunk<NT, PS, T>(ch, c0, mine, nkt, nk, gR);
 		const int cnt = ch.cnt;
 		V4 acc[4];
 #pragma unroll
 		for (int t = 0; t < 4; t++)
-		{
 			acc[t] = V4{0, 0, 0, 0};
-			if (!FROMG && t < cnt)
-#pragma unroll
-				for (int r = 0; r < 4; r++)
-					acc[t][r] = M(ch.I[t] * 16 + acc_row<T>(lane, r), ch.J[t] * 16 + (lane & 15));
-		}
 		if (cnt == 4)
 			ric_syrk_tiles<4, T>(W, ch.I, ch.J, kt, acc);
 		else if (cnt == 3)
@@ -313,54 +276,29 @@ __device__ __forceinline__ void ric_syrk_m(const TileLowerT<T> M, const TileRect
 				const int col = ch.J[t] * 16 + (lane & 15);
 #pragma unroll
 				for (int r = 0; r < 4; r++)
-				{
-					const T v = FROMG ? acc[t][r] + ch.rq[t][r] : acc[t][r];
-					M(ch.I[t] * 16 + acc_row<T>(lane, r), col) = (AUG && col >= nk) ? T(0) : v;
-				}
+					M(ch.I[t] * 16 + acc_row<T>(lane, r), col) = acc[t][r] + ch.rq[t][r];
 			}
 		}
 	}
 }
 
-// The one-wave kernels call the in-LDS Cholesky out of line: inlined it
-// would raise them above the 168 registers that three waves per SIMD allow.
-template <int NT>
-__device__ __attribute__((noinline)) void ric_trmm_call(const TileLower M, const TileRect W, int nkt, int n1, int n1t, int u1)
-{
-	ric_trmm_w<NT>(TileLower{lds_opaque(M.p)}, TileRect{lds_opaque(W.p), W.nct}, nkt, n1, n1t, u1);
-}
-
-template <int NT>
-__device__ __attribute__((noinline)) void ric_syrk_call(const TileLower M, const TileRect W, int nkt, int n1)
-{
-	ric_syrk_m<NT>(TileLower{lds_opaque(M.p)}, TileRect{lds_opaque(W.p), W.nct}, nkt, n1);
-}
-
-template <int NT, int NMAXC>
-__device__ __attribute__((noinline)) void ric_chol_call(const TileLower M, int nk, double *invd)
-{
-	chol_acc<double, NT, NMAXC, TileLower, false>(TileLower{lds_opaque(M.p)}, nk, nk, lds_opaque(invd));
-}
+// The argument record of the sweep: trf's, or the fused sweep's (AUG).
+template <bool AUG> struct RicArg { typedef blasfeo_amd_riccati_arg type; };
+template <> struct RicArg<true> { typedef blasfeo_amd_riccati_sv_arg type; };
 
 // the work matrix of a record: trf's `work`, the fused sweep's `work_mat`
 __device__ __forceinline__ blasfeo_dmat *ric_work(const blasfeo_amd_riccati_arg &a) { return a.work; }
 __device__ __forceinline__ blasfeo_dmat *ric_work(const blasfeo_amd_riccati_sv_arg &a) { return a.work_mat; }
 
-// AUG = true: the backward part of the fused sweep (d_back_ric_sv_libstr,
-// examples/example_d_riccati_recursion.c:58-79): every stage matrix has one
-// more row, the linear terms (BAbt[k]'s row nk = b^T, RSQrq[k]'s row nk =
-// [r; q]^T), carried through the trmm, the syrk and the trapezoid Cholesky
-// (L[k] is (nk+1) x nk); before the syrk the row of the previous factor is
-// added to W's last row (the reference's blasfeo_dgead).
-// T = float: the mixed-precision form -- the stage matrices and factors are
-// held and computed in FP32 (inputs converted on staging, factors written to
-// the FP64 outputs), multi-wave kernels only.
-template <int PS, int NT, bool AUG = false, typename ArgT = blasfeo_amd_riccati_arg, typename T = double>
-__device__ void ric_sweep_lds(const ArgT &a, T *smem)
+} // namespace bfa
+#include "bfa_ric_coop.hpp"
+namespace bfa {
+
+// The stage matrices and factors are held and computed in FP32 (inputs converted
+// on staging, factors written to the FP64 outputs).
+template <int PS, int NT, typename T>
+__device__ void ric_sweep_lds(const blasfeo_amd_riccati_arg &a, T *smem)
 {
-	static_assert(sizeof(T) == 8 || NT != WAVE, "the FP32 sweep runs on two or four waves per instance");
-	constexpr int NMAXC = (NT == WAVE) ? 64 : 128;
-	constexpr int XR = AUG ? 1 : 0;   // extra row of the augmented form
 	const int N = uni(a.N);
 	const int *nx = a.nx;
 	const int *nu = a.nu;
@@ -375,15 +313,14 @@ __device__ void ric_sweep_lds(const ArgT &a, T *smem)
 	}
 	nkmax = uni(nkmax);
 	nxmax = uni(nxmax);
-	const int nkt_max = (nkmax + XR + 15) / 16;
+	const int nkt_max = (nkmax + 15) / 16;
 	const int nxt_max = (nxmax + 15) / 16;
 	const int nlow = nkt_max * (nkt_max + 1) / 2;
 	const TileLowerT<T> M{smem};
 	const TileRectT<T> W{smem + (size_t)nlow * RT_SZ, nxt_max};
 	T *invd = smem + (size_t)(nlow + nkt_max * nxt_max) * RT_SZ;
 
-	// s = -1 is the last stage, L[N] = chol(Q_N) (potrf_l; potrf_l_mn of the
-	// (nx+1) x nx trapezoid when AUG); s >= 0 is stage k = N-1-s.  One call
+	// s = -1 is the last stage, L[N] = chol(Q_N); s >= 0 is stage k = N-1-s.  One call
 	// site of the in-LDS Cholesky.  Inlined, it addresses the kernel's dynamic
 	// LDS directly; out of line, every LDS access of the callee first loads
 	// the kernel's LDS offset from a table and waits for it.
@@ -392,8 +329,7 @@ __device__ void ric_sweep_lds(const ArgT &a, T *smem)
 		const bool last = s < 0;
 		const int k = last ? N : N - 1 - s;
 		const int nk = uni(last ? nx[N] : nu[k] + nx[k]);
-		const int nkt = (nk + 15) / 16;         // column tiles
-		const int mrt = (nk + XR + 15) / 16;    // row tiles
+		const int nkt = (nk + 15) / 16;
 		if (!last)
 		{
 			const int n1 = uni(nx[k + 1]);
@@ -405,66 +341,36 @@ __device__ void ric_sweep_lds(const ArgT &a, T *smem)
 			// M are complete at the Cholesky's barriers; without a barrier
 			// here the previous stage's stores of L (which only read M)
 			// overlap the trmm (which only reads M and writes W)
-			if constexpr (NT == WAVE)
-			{
-				g2s_acc<double, PS, NT, false>(view<double, PS>(&BAbt[k]), 0, 0, mrt * 16, n1t * 16, nk + XR, n1, W);
-				__syncthreads();
-			}
-			if constexpr (NT == WAVE)
-				ric_trmm_call<NT>(M, W, mrt, n1, n1t, u1);
-			else
-				ric_trmm_w<NT, T>(M, W, mrt, n1, n1t, u1);
+			ric_trmm_w<NT, T>(M, W, nkt, n1, n1t, u1);
 			__syncthreads();
-			if constexpr (AUG)
-			{
-				// W(nk, :) += L[k+1](nu1 + nx1, nu1:) (blasfeo_dgead): the linear
-				// term's row of the previous factor, still in M
-				for (int j = threadIdx.x; j < n1; j += NT)
-					W(nk, j) += M(u1 + n1, u1 + j);
-				__syncthreads();
-			}
 		}
 		// M <- lower(RSQ[k]) + W W^T (L[k+1] is no longer needed); the
 		// multi-wave kernels start the syrk accumulators from RSQ[k] itself
-		if (last || NT == WAVE)
-			g2s_acc<double, PS, NT, true>(view<double, PS>(&RSQ[k]), 0, 0, mrt * 16, nkt * 16, nk + XR, nk, M);
-		if (!last)
-		{
-			if constexpr (NT == WAVE)
-			{
-				__syncthreads();
-				ric_syrk_call<NT>(M, W, nkt, uni(nx[k + 1]));
-			}
-			else
-				ric_syrk_m<NT, PS, true, AUG, T>(M, W, nkt, uni(nx[k + 1]), view<double, PS>(&RSQ[k]), nk);
-		}
+		if (last)
+			g2s_acc<double, PS, NT, true>(view<double, PS>(&RSQ[k]), 0, 0, nkt * 16, nkt * 16, nk, nk, M);
+		else
+			ric_syrk_m<NT, PS, T>(M, W, nkt, uni(nx[k + 1]), view<double, PS>(&RSQ[k]), nk);
 		// L[k] = chol(M); W is free (the syrk has read it), so the waves
 		// other than 0 load the next stage's BAbt into it meanwhile
-		if constexpr (NT == WAVE)
-			ric_chol_call<NT, NMAXC>(M, nk, invd);
-		else
-		{
-			const int kn = k - 1;   // next stage (k = N for the last stage: kn = N - 1)
-			auto side = [&]() {
-				if (kn >= 0)
-				{
-					const int nkn = uni(nu[kn] + nx[kn]), n1n = uni(nx[kn + 1]);
-					g2s_acc<double, PS, NT, false, TileRectT<T>, 1>(view<double, PS>(&BAbt[kn]), 0, 0,
-						(nkn + XR + 15) / 16 * 16, (n1n + 15) / 16 * 16, nkn + XR, n1n, W);
-				}
-			};
-			chol_acc<T, NT, NMAXC, TileLowerT<T>, true, decltype(side)>(M, nk + XR, nk, invd, side);
-		}
-		s2g_acc<double, PS, NT, true>(view<double, PS>(&L[k]), 0, 0, nk + XR, nk, M, 0);
+		const int kn = k - 1;   // next stage (k = N for the last stage: kn = N - 1)
+		auto side = [&]() {
+			if (kn >= 0)
+			{
+				const int nkn = uni(nu[kn] + nx[kn]), n1n = uni(nx[kn + 1]);
+				g2s_acc<double, PS, NT, false, TileRectT<T>, 1>(view<double, PS>(&BAbt[kn]), 0, 0,
+					(nkn + 15) / 16 * 16, (n1n + 15) / 16 * 16, nkn, n1n, W);
+			}
+		};
+		chol_acc<T, NT, 128, TileLowerT<T>, true, decltype(side)>(M, nk, nk, invd, side);
+		s2g_acc<double, PS, NT, true>(view<double, PS>(&L[k]), 0, 0, nk, nk, M, 0);
 		for (int j = threadIdx.x; j < nk; j += NT)
 			L[k].dA[j] = invd[j];
 		if (threadIdx.x == 0)
 		{
-			// potrf_l marks the whole diagonal cached; syrk_dpotrf_ln and the
-			// trapezoid forms (potrf_l_mn, syrk_dpotrf_ln_mn) one entry
-			L[k].use_dA = (last && !AUG) ? nk : 1;
+			// potrf_l marks the whole diagonal cached, syrk_dpotrf_ln one entry
+			L[k].use_dA = last ? nk : 1;
 			if (!last)
-				ric_work(a)->use_dA = 0;
+				a.work->use_dA = 0;
 		}
 	}
 	__syncthreads();
@@ -533,21 +439,18 @@ __global__ void k_ric_zero(int *counts)
 		counts[threadIdx.x] = 0;
 }
 
-// The argument record of the sweep: trf's, or the fused sweep's (AUG).
-template <bool AUG> struct RicArg { typedef blasfeo_amd_riccati_arg type; };
-template <> struct RicArg<true> { typedef blasfeo_amd_riccati_sv_arg type; };
-
-// The plan: one thread per instance takes the size class of its largest
+// The plan: one thread per instance takes the class of its largest
 // stage (ric_class, -1 for none) and the workgroup appends to the class
 // lists.  Instances with a negative horizon or size are dropped (the
 // reference has no defined behaviour for them); those larger than mmax are
 // dropped from the general class, which cannot hold them.
 // AUG: stage matrices have one more row; no global-memory sweep serves them,
-// so instances that fit no LDS class are dropped (the entry refuses size
-// bounds that allow them).  T = float: the classes of the FP32 sweep (half
-// the bytes per element); it has no global-memory form either.
+// so instances that fit no class are dropped (the entry refuses size
+// bounds that allow them).  T = float: the LDS classes of the FP32 sweep; it
+// has no global-memory form either.  rmax: the strips that the hint allows;
+// larger instances join the last class, whose launch holds any of them.
 template <bool AUG = false, typename T = double>
-__device__ __forceinline__ int ric_class(const typename RicArg<AUG>::type &a, int mmax)
+__device__ __forceinline__ int ric_class(const typename RicArg<AUG>::type &a, int mmax, int rmax)
 {
 	constexpr int XR = AUG ? 1 : 0;
 	constexpr bool NOGEN = AUG || sizeof(T) != 8;
@@ -566,9 +469,14 @@ __device__ __forceinline__ int ric_class(const typename RicArg<AUG>::type &a, in
 	if (bad)
 		return -1;
 	int cls = RIC_GENERAL;
-	if (nxmax <= 64 && nkmax + XR <= 128)
+	if (sizeof(T) == 8 && nxmax <= 64 && nkmax + XR <= 128)
 	{
-		// one-wave classes (cap <= 40960) factor with one panel row per lane: nkmax <= 64
+		// the strips of its largest stage; more than the hint allows: the last class
+		const int R = max(1, (nkmax + XR + 15) / 16);
+		cls = R <= rmax ? R - 1 : RIC_NCLASS - 1;
+	}
+	else if (nxmax <= 64 && nkmax + XR <= 128)
+	{
 		const int f = ric_footprint(nkmax + XR, nxmax, (int)sizeof(T));
 		for (int c = RIC_NCLASS - 1; c >= 0; c--)
 			if (f <= c_ric_cap[c] && (c_ric_cap[c] > 40960 || nkmax + XR <= 64))
@@ -580,11 +488,11 @@ __device__ __forceinline__ int ric_class(const typename RicArg<AUG>::type &a, in
 }
 
 template <bool AUG = false, typename T = double>
-__global__ void k_ric_plan(const typename RicArg<AUG>::type *__restrict__ args, int batch, int mmax,
+__global__ void k_ric_plan(const typename RicArg<AUG>::type *__restrict__ args, int batch, int mmax, int rmax,
 	int *counts, int *lists)
 {
 	const int i = blockIdx.x * blockDim.x + threadIdx.x;
-	plan_bucket<RIC_GENERAL + 1>(i, i < batch ? ric_class<AUG, T>(args[i], mmax) : -1, batch, counts, lists);
+	plan_bucket<RIC_GENERAL + 1>(i, i < batch ? ric_class<AUG, T>(args[i], mmax, rmax) : -1, batch, counts, lists);
 }
 
 // Next instance of the class for this workgroup from the class's work-queue
@@ -593,56 +501,26 @@ __global__ void k_ric_plan(const typename RicArg<AUG>::type *__restrict__ args, 
 // the class size.  Several waves share the value through the LDS slot, which
 // is rewritten only after the sweep's last barrier, which every thread passes
 // after reading it.
-template <int NT>
 __device__ __forceinline__ int ric_next(int *head, int *slot)
 {
-	if constexpr (NT == WAVE)
-	{
-		int t = 0;
-		if (threadIdx.x == 0)
-			t = atomicAdd(head, 1);
-		return __shfl(t, 0, WAVE);
-	}
-	else
-	{
-		if (threadIdx.x == 0)
-			*slot = atomicAdd(head, 1);
-		__syncthreads();
-		return *slot;
-	}
+	if (threadIdx.x == 0)
+		*slot = atomicAdd(head, 1);
+	__syncthreads();
+	return *slot;
 }
 
-template <int PS, int NT, bool AUG = false, typename T = double>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_ric_class(const typename RicArg<AUG>::type *__restrict__ args,
+template <int PS, int NT, typename T>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_ric_class(const blasfeo_amd_riccati_arg *__restrict__ args,
 	const int *__restrict__ count, const int *__restrict__ list, int *head)
 {
-	static_assert(!(AUG && NT == WAVE), "the fused sweep runs on two or four waves per instance");
 	extern __shared__ double smem_d[];
 	int *slot = reinterpret_cast<int *>(smem_d);
 	T *work = reinterpret_cast<T *>(smem_d) + RIC_QSLOT / sizeof(T);
 	if (threadIdx.x == 0)
 		work[-1] = T(0);   // the trmm's zero operand (ric_trmm_w)
 	const int cnt = *count;
-	for (int t = ric_next<NT>(head, slot); t < cnt; t = ric_next<NT>(head, slot))
-		ric_sweep_lds<PS, NT, AUG, typename RicArg<AUG>::type, T>(args[list[t]], work);
-}
-
-// one wave per instance (selected by the tuning knobs, not by default):
-// registers capped at 168 so that three instances share each SIMD.  Only
-// classes of at most 40960 B can use it, whose stages have nu+nx <= 64 (the
-// plan's rule), so the Cholesky keeps one panel row per lane.
-template <int PS>
-__global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(3))) void k_ric_class1(
-	const blasfeo_amd_riccati_arg *__restrict__ args, const int *__restrict__ count, const int *__restrict__ list,
-	int *head)
-{
-	extern __shared__ double smem_d[];
-	double *work = smem_d + RIC_QSLOT / sizeof(double);
-	if (threadIdx.x == 0)
-		work[-1] = 0.0;   // the trmm's zero operand (ric_trmm_w)
-	const int cnt = *count;
-	for (int t = ric_next<WAVE>(head, nullptr); t < cnt; t = ric_next<WAVE>(head, nullptr))
-		ric_sweep_lds<PS, WAVE>(args[list[t]], work);
+	for (int t = ric_next(head, slot); t < cnt; t = ric_next(head, slot))
+		ric_sweep_lds<PS, NT, T>(args[list[t]], work);
 }
 
 template <int PS>
@@ -661,33 +539,15 @@ __global__ __launch_bounds__(NT3) void k_ric_general(const blasfeo_amd_riccati_a
 		ric_sweep_general<PS>(args[list[t]], P, LDP, mmax, As, Bs, L11, invs);
 }
 
-template <int PS, int NT, bool AUG = false, typename T = double>
-static int launch_class(int cls, int grid, const typename RicArg<AUG>::type *args, int *counts, const int *lists,
+template <int PS, int NT, typename T>
+static int launch_class(int cls, int grid, const blasfeo_amd_riccati_arg *args, int *counts, const int *lists,
 	int batch, hipStream_t st, const char *name)
 {
-	if constexpr (AUG || sizeof(T) != 8)
-	{
-		static_assert(NT != WAVE, "the fused and FP32 sweeps run on two or four waves per instance");
-		if (const int rc = lds_check(reinterpret_cast<const void *>(&k_ric_class<PS, NT, AUG, T>), h_ric_cap[cls], name))
-			return rc;
-		hipLaunchKernelGGL((k_ric_class<PS, NT, AUG, T>), dim3(grid), dim3(NT), h_ric_cap[cls], st, args,
-			counts + cls, lists + (size_t)cls * batch, counts + RIC_HEAD + cls);
-		return check_launch(name);
-	}
-	else
-	{
-		const void *fn = NT == WAVE ? reinterpret_cast<const void *>(&k_ric_class1<PS>)
-		                            : reinterpret_cast<const void *>(&k_ric_class<PS, NT>);
-		if (const int rc = lds_check(fn, h_ric_cap[cls], name))
-			return rc;
-		if (NT == WAVE)
-			hipLaunchKernelGGL((k_ric_class1<PS>), dim3(grid), dim3(WAVE), h_ric_cap[cls], st, args,
-				counts + cls, lists + (size_t)cls * batch, counts + RIC_HEAD + cls);
-		else
-			hipLaunchKernelGGL((k_ric_class<PS, NT>), dim3(grid), dim3(NT), h_ric_cap[cls], st, args,
-				counts + cls, lists + (size_t)cls * batch, counts + RIC_HEAD + cls);
-		return check_launch(name);
-	}
+	if (const int rc = lds_check(reinterpret_cast<const void *>(&k_ric_class<PS, NT, T>), h_ric_cap[cls], name))
+		return rc;
+	hipLaunchKernelGGL((k_ric_class<PS, NT, T>), dim3(grid), dim3(NT), h_ric_cap[cls], st, args,
+		counts + cls, lists + (size_t)cls * batch, counts + RIC_HEAD + cls);
+	return check_launch(name);
 }
 
 // Helper streams (default priority) on which the class launches run side by
@@ -726,30 +586,22 @@ static RicFork *ric_fork_state()
 	return f;
 }
 
-// ws: the plan workspace, (RIC_NCLASS + 1) * batch + 64 ints.  fork: run the
-// class launches side by side on helper streams (else all on st, in order).
-template <int PS, bool AUG = false, typename T = double>
-static int launch_ric(int batch, const typename RicArg<AUG>::type *args, int mmax, int maxfoot, int *ws, bool fork,
-	hipStream_t st, const char *name)
+// The fork of the caller's stream to the helpers and the join back, RAII: the
+// helpers are joined also after a launch error, so that the caller's stream never
+// runs ahead of them.
+struct RicStreams
 {
-	int *counts = ws;
-	int *lists = ws + 64;
-	hipLaunchKernelGGL(k_ric_zero, dim3(1), dim3(64), 0, st, counts);
-	hipLaunchKernelGGL((k_ric_plan<AUG, T>), dim3((batch + 255) / 256), dim3(256), 0, st, args, batch, mmax, counts, lists);
-	int rc = check_launch(name);
-	if (rc)
-		return rc;
-	const int cus = num_cus() > 0 ? num_cus() : 256;
 	RicFork *fk = nullptr;
 	std::unique_lock<std::mutex> lock;
-	hipStream_t ss[1 + RIC_AUX] = {st, st, st, st};
-	if (fork)
+	hipStream_t ss[1 + RIC_AUX];
+	explicit RicStreams(hipStream_t st) { for (hipStream_t &s : ss) s = st; }
+	int fork(const char *name)
 	{
 		fk = ric_fork_state();
 		if (!fk)
 			return set_error(BLASFEO_AMD_ELAUNCH, "%s: cannot create the helper streams", name);
 		lock = std::unique_lock<std::mutex>(fk->mu);
-		if (hipEventRecord(fk->fork, st) != hipSuccess)
+		if (hipEventRecord(fk->fork, ss[0]) != hipSuccess)
 			return check_launch(name);
 		for (int i = 0; i < RIC_AUX; i++)
 		{
@@ -757,93 +609,150 @@ static int launch_ric(int batch, const typename RicArg<AUG>::type *args, int mma
 			if (hipStreamWaitEvent(fk->aux[i], fk->fork, 0) != hipSuccess)
 				return check_launch(name);
 		}
+		return BLASFEO_AMD_OK;
 	}
-	// Launch schedule: (class, stream) in launch order; stream 0 is the
-	// caller's, 1..3 the helpers.  The general launch and the 40, 16 and
-	// 32 KB classes run one after another on the caller's stream; the 160,
-	// 80 and 54 KB classes start at once on the helpers, the 24 and 8 KB
-	// classes after the 80 KB one.  Measured on the 8192 x N=20 batch (nx ~
-	// U{8..64}, nu ~ U{2..16}) against other orders on MI355X: 5.52 ms
-	// replayed in a graph and 5.49 ms eager, against 5.85 and 5.96 ms for
-	// largest-first dealt round-robin over the four streams (the 16 and
-	// 32 KB classes started only after the 80 and 54 KB ones and ran alone
-	// at the end; an empty class launch holds its stream while its
-	// workgroups wait for LDS).
-	static const int sched[RIC_NCLASS + 1][2] = {
-		{RIC_GENERAL, 0}, {7, 1}, {6, 2}, {5, 3}, {4, 0}, {1, 0}, {3, 0}, {2, 2}, {0, 2}};
+	int join(const char *name)
+	{
+		for (int i = 0; fk && i < RIC_AUX; i++)
+			if (hipEventRecord(fk->join[i], fk->aux[i]) != hipSuccess ||
+				hipStreamWaitEvent(ss[0], fk->join[i], 0) != hipSuccess)
+				return check_launch(name);
+		return BLASFEO_AMD_OK;
+	}
+};
+
+// One launch of k_ric_coop: the class of R strips (its list), or every instance
+// (lists == nullptr).
+template <int PS, int NW, bool AUG>
+static int launch_coop(int R, int grid, const typename RicArg<AUG>::type *args, int *counts, const int *lists, int batch,
+	hipStream_t st, const char *name)
+{
+	constexpr int NX = NW == 1 ? 2 : 4;
+	const size_t shm = sizeof(double) * ric_coop_elems(R, NX);
+	if (const int rc = lds_check(reinterpret_cast<const void *>(&k_ric_coop<PS, NW, NX, AUG>), shm, name))
+		return rc;
+	const int cls = R - 1;
+	hipLaunchKernelGGL((k_ric_coop<PS, NW, NX, AUG>), dim3(grid), dim3(NW * WAVE), shm, st, args, R,
+		lists ? counts + cls : (const int *)nullptr, lists ? lists + (size_t)cls * batch : (const int *)nullptr,
+		lists ? counts + RIC_HEAD + cls : (int *)nullptr);
+	return check_launch(name);
+}
+
+// The FP64 sweep.  nxmax: the hint's bound of nx.
+template <int PS, bool AUG>
+static int launch_ric_coop(int batch, const typename RicArg<AUG>::type *args, int mmax, int nxmax, int *ws, bool fork,
+	hipStream_t st, const char *name)
+{
+	constexpr int XR = AUG ? 1 : 0;
+	const int cus = num_cus() > 0 ? num_cus() : 256;
+	const bool resident = mmax + XR <= 128 && nxmax <= 64;   // the hint admits no larger instance
+	const int rmax = resident ? max(1, (mmax + XR + 15) / 16) : RIC_NCLASS;
+	// No plan where one launch serves every instance: a batch that gives no CU
+	// more than one (four waves each, the LDS of the largest size), and sizes of
+	// up to 32 rows (one wave each, their LDS differs little).  The tuning knobs
+	// shape the class launches.
+	bool tuned = false;
+	for (int c = 0; c < RIC_NCLASS; c++)
+		tuned = tuned || tune_value(TUNE_RIC_THREADS, c) || tune_value(TUNE_RIC_PER_CU, c);
+	const bool direct = resident && !tuned;
+	if (direct && rmax <= 2)
+		return launch_coop<PS, 1, AUG>(rmax, batch, args, nullptr, nullptr, batch, st, name);
+	if (direct && batch <= cus)
+		return launch_coop<PS, 4, AUG>(RIC_NCLASS, batch, args, nullptr, nullptr, batch, st, name);
+	int *counts = ws;
+	int *lists = ws + 64;
+	hipLaunchKernelGGL(k_ric_zero, dim3(1), dim3(64), 0, st, counts);
+	hipLaunchKernelGGL((k_ric_plan<AUG>), dim3((batch + 255) / 256), dim3(256), 0, st, args, batch, mmax, rmax, counts, lists);
+	int rc = check_launch(name);
+	if (rc)
+		return rc;
+	RicStreams str(st);
+	if (fork && (rc = str.fork(name)))
+		return rc;
+	// Launch schedule: (strips, stream) in launch order; stream 0 is the caller's.
+	// The classes up to 80 rows, most of the work of the batches measured, start
+	// side by side.  One wave per instance up to two strips, two up to four, four
+	// above: on 8192 x N = 20, nx ~ U{8..64}, nu ~ U{2..16} (MI355X, 4.29 ms) four
+	// waves for three strips take 4.64, for four strips 4.65, two for two 4.35 ms.
+	static const int sched[RIC_NCLASS][2] = {{8, 1}, {5, 2}, {4, 0}, {3, 3}, {7, 1}, {6, 1}, {2, 2}, {1, 1}};
+	if constexpr (!AUG)
+	{
+		const size_t shm = sizeof(double) * PW * ((mmax + 15) / 16 * 16 + 1);
+		rc = lds_check(reinterpret_cast<const void *>(&k_ric_general<PS>), shm, name);
+		if (!rc)
+		{
+			hipLaunchKernelGGL((k_ric_general<PS>), dim3(min(batch, cus)), dim3(NT3), shm, str.ss[0], args,
+				counts + RIC_GENERAL, lists + (size_t)RIC_GENERAL * batch, mmax);
+			rc = check_launch(name);
+		}
+	}
+	for (int e = 0; e < RIC_NCLASS && !rc; e++)
+	{
+		const int R = sched[e][0];
+		hipStream_t sc = str.ss[sched[e][1]];
+		if (R > rmax && R < RIC_NCLASS)
+			continue;
+		int nw = R <= 2 ? 1 : R <= 4 ? 2 : 4;
+		if (const int v = tune_value(TUNE_RIC_THREADS, R - 1))
+			if (v / WAVE * 2 >= R)
+				nw = v / WAVE;
+		// as many workgroups as the registers and the LDS of a CU hold
+		const int lds = (int)sizeof(double) * ric_coop_elems(R, nw == 1 ? 2 : 4);
+		int per_cu = max(1, min(4 * ric_coop_waves(nw) / nw, RIC_LDS_MAX / lds));
+		if (const int v = tune_value(TUNE_RIC_PER_CU, R - 1))
+			per_cu = v;
+		const int grid = min(batch, R > rmax ? 16 : cus * per_cu);
+		if (nw == 1)
+			rc = launch_coop<PS, 1, AUG>(R, grid, args, counts, lists, batch, sc, name);
+		else if (nw == 2)
+			rc = launch_coop<PS, 2, AUG>(R, grid, args, counts, lists, batch, sc, name);
+		else
+			rc = launch_coop<PS, 4, AUG>(R, grid, args, counts, lists, batch, sc, name);
+	}
+	const int rj = str.join(name);
+	return rc ? rc : rj;
+}
+
+// The FP32 sweep.  ws: the plan workspace, (RIC_NCLASS + 1) * batch + 64 ints.
+template <int PS>
+static int launch_ric_f32(int batch, const blasfeo_amd_riccati_arg *args, int mmax, int *ws, hipStream_t st, const char *name)
+{
+	int *counts = ws;
+	int *lists = ws + 64;
+	hipLaunchKernelGGL(k_ric_zero, dim3(1), dim3(64), 0, st, counts);
+	hipLaunchKernelGGL((k_ric_plan<false, float>), dim3((batch + 255) / 256), dim3(256), 0, st, args, batch, mmax, 0, counts, lists);
+	int rc = check_launch(name);
+	if (rc)
+		return rc;
+	const int cus = num_cus() > 0 ? num_cus() : 256;
+	RicStreams str(st);
+	if ((rc = str.fork(name)))
+		return rc;
+	// Launch schedule: (class, stream) in launch order; stream 0 is the caller's,
+	// 1..3 the helpers.  The 40, 16 and 32 KB classes run one after another on
+	// the caller's stream; the 160, 80 and 54 KB classes start at once on the
+	// helpers, the 24 and 8 KB classes after the 80 KB one.
+	static const int sched[RIC_NCLASS][2] = {{7, 1}, {6, 2}, {5, 3}, {4, 0}, {1, 0}, {3, 0}, {2, 2}, {0, 2}};
 	static_assert(RIC_NCLASS == 8 && RIC_AUX == 3, "the launch schedule lists 8 classes on 4 streams");
-	(void)maxfoot;
-	for (int e = 0; e <= RIC_NCLASS && !rc; e++)
+	for (int e = 0; e < RIC_NCLASS && !rc; e++)
 	{
 		const int cls = sched[e][0];
-		hipStream_t sc = ss[sched[e][1]];
-		if (cls == RIC_GENERAL)
-		{
-			if constexpr (!AUG && sizeof(T) == 8)
-			{
-				const size_t shm = sizeof(double) * PW * ((mmax + 15) / 16 * 16 + 1);
-				const int grid = min(batch, cus);
-				rc = lds_check(reinterpret_cast<const void *>(&k_ric_general<PS>), shm, name);
-				if (!rc)
-				{
-					hipLaunchKernelGGL((k_ric_general<PS>), dim3(grid), dim3(NT3), shm, sc, args,
-						counts + RIC_GENERAL, lists + (size_t)RIC_GENERAL * batch, mmax);
-					rc = check_launch(name);
-				}
-			}
-			continue;
-		}
-		// built-in launch shape per class (threads per instance, resident
-		// instances per CU), from autotuner runs on the 8192 x N=20 batch
-		// (nx ~ U{8..64}, nu ~ U{2..16}) on MI355X: two waves per instance up
-		// to 24 KB (4 per CU up to 8 KB, 8 above: fewer resident instances
-		// spread a small class over more CUs), four waves and 3 per CU at
-		// 32 KB, four waves and 2 per CU above.  The tuning knobs override
-		// both.
-		int per_cu, nt;
-		if (h_ric_cap[cls] <= 24576)
-		{
-			nt = 128;
-			per_cu = h_ric_cap[cls] <= 8192 ? 4 : min(RIC_LDS_MAX / h_ric_cap[cls], 8);
-		}
-		else if (h_ric_cap[cls] == 32768)
-		{
-			nt = 256;
-			per_cu = 3;
-		}
-		else
-		{
-			nt = 256;
-			per_cu = max(1, min(2, RIC_LDS_MAX / h_ric_cap[cls]));
-		}
-		if constexpr (sizeof(T) != 8)
-		{
-			// FP32 sweep: as many resident instances as LDS and three waves
-			// per SIMD allow
-			per_cu = min(nt == 128 ? 6 : 3, RIC_LDS_MAX / h_ric_cap[cls]);
-		}
+		hipStream_t sc = str.ss[sched[e][1]];
+		// two waves per instance up to 24 KB, four above; as many resident
+		// instances as LDS and three waves per SIMD allow.  The tuning knobs
+		// override both.
+		int nt = h_ric_cap[cls] <= 24576 ? 128 : 256;
+		int per_cu = min(nt == 128 ? 6 : 3, RIC_LDS_MAX / h_ric_cap[cls]);
 		if (const int v = tune_value(TUNE_RIC_PER_CU, cls))
 			per_cu = v;
 		if (const int v = tune_value(TUNE_RIC_THREADS, cls))
 			nt = v;
 		const int grid = min(batch, cus * per_cu);
-		constexpr bool ONEWAVE = !AUG && sizeof(T) == 8;
-		if (nt == 64 && ONEWAVE)
-			rc = launch_class<PS, ONEWAVE ? 64 : 128, AUG, T>(cls, grid, args, counts, lists, batch, sc, name);
-		else if (nt <= 128)
-			rc = launch_class<PS, 128, AUG, T>(cls, grid, args, counts, lists, batch, sc, name);
-		else
-			rc = launch_class<PS, 256, AUG, T>(cls, grid, args, counts, lists, batch, sc, name);
-		if (rc)
-			break;
+		rc = nt <= 128 ? launch_class<PS, 128, float>(cls, grid, args, counts, lists, batch, sc, name)
+		               : launch_class<PS, 256, float>(cls, grid, args, counts, lists, batch, sc, name);
 	}
-	// join back whatever was launched (also after a launch error, so that
-	// the caller's stream never runs ahead of the helpers)
-	for (int i = 0; fork && i < RIC_AUX; i++)
-		if (hipEventRecord(fk->join[i], fk->aux[i]) != hipSuccess ||
-			hipStreamWaitEvent(st, fk->join[i], 0) != hipSuccess)
-			return check_launch(name);
-	return rc ? rc : check_launch(name);
+	const int rj = str.join(name);
+	return rc ? rc : rj;
 }
 
 // ---------------------------------------------------------------------------
@@ -900,14 +809,13 @@ extern "C" int blasfeo_amd_d_back_ric_trf_batched(int ps, int batch, const blasf
 	if (mmax > fact_mmax<double>())
 		return set_error(BLASFEO_AMD_ETOOBIG, "%s: nu+nx up to %d supported, got %d", name, fact_mmax<double>(), mmax);
 	const int nxmax = hint->max_n > 0 ? hint->max_n : mmax;
-	const int maxfoot = ric_footprint(mmax, min(nxmax, mmax));
 	hipStream_t st = (hipStream_t)stream;
 	const size_t wsbytes = sizeof(int) * ((size_t)(RIC_NCLASS + 1) * batch + 64);
 	int *ws = (int *)workspace(wsbytes, st);
 	if (!ws)
 		return set_error(BLASFEO_AMD_ENOMEM, "%s: cannot allocate the %zu-byte plan workspace", name, wsbytes);
-	return ps == 4 ? launch_ric<4>(batch, args, mmax, maxfoot, ws, true, st, name)
-	               : launch_ric<8>(batch, args, mmax, maxfoot, ws, true, st, name);
+	return ps == 4 ? launch_ric_coop<4, false>(batch, args, mmax, nxmax, ws, true, st, name)
+	               : launch_ric_coop<8, false>(batch, args, mmax, nxmax, ws, true, st, name);
 }
 
 extern "C" int blasfeo_amd_d_back_ric_trf_batched_noalloc(int ps, int batch, const blasfeo_amd_riccati_arg *args, const blasfeo_amd_hint *hint, blasfeo_amd_stream_t stream)
@@ -930,13 +838,12 @@ extern "C" int blasfeo_amd_d_back_ric_trf_batched_noalloc(int ps, int batch, con
 	if (mmax > fact_mmax<double>())
 		return set_error(BLASFEO_AMD_ETOOBIG, "%s: nu+nx up to %d supported, got %d", name, fact_mmax<double>(), mmax);
 	const int nxmax = hint->max_n > 0 ? hint->max_n : mmax;
-	const int maxfoot = ric_footprint(mmax, min(nxmax, mmax));
 	int *ws = noalloc_scratch();
 	if (!ws)
 		return set_error(BLASFEO_AMD_ELAUNCH, "%s: no device address for the scratch array", name);
 	hipStream_t st = (hipStream_t)stream;
-	return ps == 4 ? launch_ric<4>(batch, args, mmax, maxfoot, ws, false, st, name)
-	               : launch_ric<8>(batch, args, mmax, maxfoot, ws, false, st, name);
+	return ps == 4 ? launch_ric_coop<4, false>(batch, args, mmax, nxmax, ws, false, st, name)
+	               : launch_ric_coop<8, false>(batch, args, mmax, nxmax, ws, false, st, name);
 }
 
 // ---------------------------------------------------------------------------
@@ -1120,9 +1027,8 @@ extern "C" int blasfeo_amd_d_back_ric_sv_batched(int ps, int batch, const blasfe
 	int *ws = (int *)workspace(wsbytes, st);
 	if (!ws)
 		return set_error(BLASFEO_AMD_ENOMEM, "%s: cannot allocate the %zu-byte plan workspace", name, wsbytes);
-	const int maxfoot = ric_footprint(mmax + 1, min(nxmax, mmax));
-	int rc = ps == 4 ? launch_ric<4, true>(batch, args, mmax, maxfoot, ws, true, st, name)
-	                 : launch_ric<8, true>(batch, args, mmax, maxfoot, ws, true, st, name);
+	int rc = ps == 4 ? launch_ric_coop<4, true>(batch, args, mmax, nxmax, ws, true, st, name)
+	                 : launch_ric_coop<8, true>(batch, args, mmax, nxmax, ws, true, st, name);
 	if (rc)
 		return rc;
 	if (ps == 4)
@@ -1337,10 +1243,8 @@ extern "C" int blasfeo_amd_d_ric_solve_mixed_batched(int ps, int batch, const bl
 	hipLaunchKernelGGL(k_mix_setup, g256, dim3(256), 0, st, args, batch, ra, tm, tc);
 	int rc = check_launch(name);
 	// FP32 factorisation, solve on it
-	const int foot32 = ric_footprint(mmax, min(nxmax, mmax), 4);
 	if (!rc)
-		rc = ps == 4 ? launch_ric<4, false, float>(batch, ra, mmax, foot32, pws, true, st, name)
-		             : launch_ric<8, false, float>(batch, ra, mmax, foot32, pws, true, st, name);
+		rc = ps == 4 ? launch_ric_f32<4>(batch, ra, mmax, pws, st, name) : launch_ric_f32<8>(batch, ra, mmax, pws, st, name);
 	blasfeo_amd_hint th{mmax, nxmax, 0};
 	if (!rc)
 		rc = blasfeo_amd_d_back_ric_trs_batched(ps, batch, tm, &th, stream);
@@ -1366,10 +1270,9 @@ extern "C" int blasfeo_amd_d_ric_solve_mixed_batched(int ps, int batch, const bl
 		hipLaunchKernelGGL(k_mix_fallback, g256, dim3(256), 0, st, args, batch, ra, tm, tc);
 		rc = check_launch(name);
 	}
-	const int foot64 = ric_footprint(mmax, min(nxmax, mmax));
 	if (!rc)
-		rc = ps == 4 ? launch_ric<4>(batch, ra, mmax, foot64, pws, true, st, name)
-		             : launch_ric<8>(batch, ra, mmax, foot64, pws, true, st, name);
+		rc = ps == 4 ? launch_ric_coop<4, false>(batch, ra, mmax, nxmax, pws, true, st, name)
+		             : launch_ric_coop<8, false>(batch, ra, mmax, nxmax, pws, true, st, name);
 	if (!rc)
 		rc = blasfeo_amd_d_back_ric_trs_batched(ps, batch, tm, &th, stream);
 	if (!rc)

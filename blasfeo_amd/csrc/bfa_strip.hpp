@@ -435,55 +435,66 @@ __device__ __forceinline__ void strip_solve2(typename Vec4<T>::type acc0, typena
 // finished strips are read back for every later one, which above 64 rows
 // misses L2 and bounds the launch (8192 x 128 rows: 1.9 GB read for 0.55 GB of
 // input).
-// lds: 2 (2 NW * 256 + 256) values: two columns of operand tiles, two diagonal
-// blocks (3 steps and the 4 x 4 triangles).
+// LAY says where in LDS the tiles are passed on: tile(I, j) the base of tile (I, j)
+// of the current column, at(s) this lane's offset in it for step s, diag(j) and
+// tri(j) the diagonal block and its 4 x 4 triangles.
 // ---------------------------------------------------------------------------
+// Two columns of operand tiles and two diagonal blocks, used in turn.
 template <typename T, int NW>
-constexpr int coop_lds() { return 2 * (2 * NW * 256 + 256); }
+struct CoopRing
+{
+	static constexpr int ELEMS = 2 * (2 * NW * 256 + 256);
+	static constexpr int DSTEPS = 3;   // steps of a diagonal block that are passed on
+	T *p;
+	int lane;
+	__device__ __forceinline__ T *tile(int I, int j) const { return p + (j & 1) * (2 * NW * 256) + 256 * I; }
+	__device__ __forceinline__ int at(int s) const { return 64 * s + lane; }
+	__device__ __forceinline__ T *diag(int j) const { return p + 2 * 2 * NW * 256 + (j & 1) * 256; }
+	__device__ __forceinline__ T *tri(int j) const { return diag(j) + 192; }
+};
 
-template <typename T, int NW, typename EMIT, typename EMITD>
+template <typename T, int NW, typename LAY, typename EMIT, typename EMITD>
 __device__ __forceinline__ void chol_coop(typename Vec4<T>::type (&hi)[2 * NW], typename Vec4<T>::type (&lo)[NW],
-	int ih, int il, int R, int Cb, T *lds, const EMIT &emit, const EMITD &emit_diag)
+	int ih, int il, int Cb, const LAY &lay, const EMIT &emit, const EMITD &emit_diag)
 {
 	typedef typename Vec4<T>::type V4;
 	const int lane = lane_id();
-	T *diag = lds + 2 * 2 * NW * 256;
 	// factors the diagonal tile of block column j and passes it on
 	auto factor = [&](V4 acc, int j) {
 		T l[4], iv[4];
 		strip_chol16<T>(acc, l, iv);
-		T *db = diag + (j & 1) * 256;
+		T *db = lay.diag(j);
 #pragma unroll
-		for (int s = 0; s < 3; s++)
-			db[64 * s + lane] = l[s];
-		strip_put_tri<T>(db + 192, l, iv);
+		for (int s = 0; s < LAY::DSTEPS; s++)
+			db[lay.at(s)] = l[s];
+		strip_put_tri<T>(lay.tri(j), l, iv);
 		emit_diag(j, l, iv);
 	};
-	if (ih == 0)
+	if (Cb > 0 && ih == 0)
 		factor(hi[0], 0);
-	else if (il == 0)
+	else if (Cb > 0 && il == 0)
 		factor(lo[0], 0);
 	__syncthreads();
 #pragma unroll 1
 	for (int j = 0; j < Cb; j++)
 	{
-		T *col = lds + (j & 1) * (2 * NW * 256);
-		const T *db = diag + (j & 1) * 256;
+		const T *db = lay.diag(j), *tb = lay.tri(j);
 		V4 yh = V4{0, 0, 0, 0}, yl = V4{0, 0, 0, 0};   // -X of this column
 		{
 			T lk[3], d[4];
 #pragma unroll
 			for (int s = 0; s < 3; s++)
-				lk[s] = db[64 * s + lane];
+				lk[s] = db[lay.at(s)];
 #pragma unroll
 			for (int s = 0; s < 4; s++)
-				d[s] = db[192 + 16 * s + (lane & 15)];
+				d[s] = tb[16 * s + (lane & 15)];
 			auto done = [&](const T (&x)[4], int I, V4 &y) {
 				emit(I, j, x);
+				T *t = lay.tile(I, j);
 #pragma unroll
 				for (int s = 0; s < 4; s++)
 				{
-					col[256 * I + 64 * s + lane] = x[s];
+					t[lay.at(s)] = x[s];
 					y[s] = -x[s];
 				}
 			};
@@ -522,7 +533,7 @@ __device__ __forceinline__ void chol_coop(typename Vec4<T>::type (&hi)[2 * NW], 
 				T a[4];
 #pragma unroll
 				for (int s = 0; s < 4; s++)
-					a[s] = col[256 * J + 64 * s + lane];
+					a[s] = lay.tile(J, j)[lay.at(s)];
 #pragma unroll
 				for (int s = 0; s < 4; s++)
 					hi[J] = mfma16(a[s], yh[s], hi[J]);
