@@ -41,6 +41,24 @@ __device__ __forceinline__ unsigned xcd_local_index(unsigned g, unsigned total)
 }
 
 // (instance, slot) of this workgroup in a 1-D launch of batch * slots
+// workgroups (rounded up to a multiple of XCDS): the slots of an instance
+// consecutive on one XCD; inst >= batch for the rounding workgroups.  The order of
+// an instance's slots is turned by its index: workgroups go to the shader
+// engines and CUs of an XCD in turn, so with 4, 8 or 16 slots in the same order
+// slot 0, which every instance has, would always come to the same ones and
+// the last slots, which few of an uneven batch have, leave the others idle
+// (32768 dgemm_nt + dsyrk_ln of U{4..128}: 4 slots 2182 -> 1747 us, 16 slots 1762
+// -> 1690; 8192 dtrsm_rltn of U{16..256} 2151 -> 1690 us).  spread: the slots of
+// an instance over all XCDs, for batches so small that whole instances would
+// load the XCDs unevenly.
+__device__ __forceinline__ void xcd_inst_slot(int slots, int &inst, int &slot, bool spread = false)
+{
+	const unsigned li = spread ? blockIdx.x : xcd_local_index(blockIdx.x, gridDim.x);
+	inst = (int)(li / (unsigned)slots);
+	slot = (int)((li + (unsigned)inst) % (unsigned)slots);
+}
+
+// (instance, slot) of this workgroup in a 1-D launch of batch * slots
 // workgroups (rounded up to a multiple of XCDS): XCD-aware (the slots of an
 // instance consecutive on one XCD) or instance-fastest (slot s of every
 // instance, then slot s + 1); inst >= batch for the rounding workgroups.
@@ -48,9 +66,7 @@ __device__ __forceinline__ void batch_slot(bool xcd, int batch, int slots, int &
 {
 	if (xcd)
 	{
-		const unsigned li = xcd_local_index(blockIdx.x, gridDim.x);
-		inst = (int)(li / (unsigned)slots);
-		slot = (int)(li % (unsigned)slots);
+		xcd_inst_slot(slots, inst, slot);
 	}
 	else
 	{

@@ -12,7 +12,8 @@
 // Measured (MI355X, 8192 FP64 solves, ps = 4; before: the row block in LDS, one of
 // four waves solving the diagonal blocks): m = n = 32 125 -> 54 us, 64 235 -> 159,
 // 128 1608 -> 795, 256 15.3 -> 4.4 ms (31 TFLOP/s; 6.2 ms with every wave reading
-// A for itself); m, n ~ U{16..256} 4.61 -> 2.15 ms.  Bound by memory up to 64
+// A for itself); m, n ~ U{16..256} 4.61 -> 1.69 ms (2.15 before the slots of an
+// instance were turned, xcd_inst_slot).  Bound by memory up to 64
 // columns, then by the matrix cores and the substitution's vector instructions,
 // with two waves per SIMD.
 #pragma once
@@ -53,8 +54,8 @@ __global__ __launch_bounds__(NT3, (trsm_waves<T, NB>())) void k_trsm_rltn(const 
 	extern __shared__ unsigned char smem_raw[];
 	T *tiles = reinterpret_cast<T *>(smem_raw);
 	__shared__ T inv_s[16 * NB];
-	const unsigned li = xcd_local_index(blockIdx.x, gridDim.x);
-	const int inst = (int)(li / (unsigned)slots), slot = (int)(li % (unsigned)slots);
+	int inst, slot;
+	xcd_inst_slot(slots, inst, slot);
 	if (inst >= batch)
 		return;
 	const typename TrsmArg<T>::type &a = args[inst];
