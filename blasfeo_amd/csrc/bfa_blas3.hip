@@ -4,13 +4,10 @@
 // Launch model: one workgroup per (instance, tile slot), `slots` slots per
 // instance (tile t of an instance goes to slot t mod slots), so a batch of
 // small instances uses one workgroup each and a batch of large ones spreads
-// its 64x64 tiles over several (tile engine: bfa_gemm_core.hpp).  The gemm
-// and trmm launches are 1-D (batch_slot): in XCD-aware order when an
-// instance has more than four slots (the slots of one instance run together
-// on one XCD and share its L2: 4000 gemm_nt of U{64..512} 7.68 -> 6.41 ms,
-// 20000 of U{4..300} 7.62 -> 6.34 ms on MI355X), instance-fastest otherwise
-// (100000 of U{4..128} on this engine: 5.35 against 8.07 ms in XCD order).
-// trsm keeps a 2-D grid (x the instance, y the slot).
+// its tiles over several.  gemm and syrk: one wavefront per tile
+// (bfa_gemm_wave.hpp); trmm: 64 x 64 tiles by four waves through LDS
+// (bfa_gemm_core.hpp), in XCD-aware order when an instance has more than four slots
+// and instance-fastest otherwise (batch_slot); trsm: bfa_trsm_strip.hpp.
 #include "bfa_gemm_core.hpp"
 #include "bfa_gemm_wave.hpp"
 #include "bfa_chol_core.hpp"
@@ -18,28 +15,6 @@
 #include "bfa_internal.hpp"
 
 namespace bfa {
-
-template <typename T, int PS, int OP>
-__global__ __launch_bounds__(NT3) __attribute__((amdgpu_waves_per_eu(3))) void k_gemm(const typename GemmArg<T>::type *__restrict__ args,
-	int batch, int slots)
-{
-	__shared__ T As[KC * LDT];
-	__shared__ T Bs[KC * LDT];
-	int inst, slot;
-	batch_slot(slots > 4, batch, slots, inst, slot);
-	if (inst >= batch)
-		return;
-	const typename GemmArg<T>::type &a = args[inst];
-	const int m = a.m;
-	const int n = (OP == OP_SYRK) ? a.m : a.n;
-	if (m <= 0 || n <= 0)
-		return;
-	if (threadIdx.x == 0 && slot == 0)
-		a.sD->use_dA = 0;
-	gemm_core<T, PS, OP>(As, Bs, m, n, a.k, a.alpha, a.beta,
-		view<T, PS>(a.sA), a.ai, a.aj, view<T, PS>(a.sB), a.bi, a.bj,
-		view<T, PS>(a.sC), a.ci, a.cj, view<T, PS>(a.sD), a.di, a.dj, slot, slots);
-}
 
 // D = alpha * B * A, A lower n x n (blasfeo_ref/x_blas3_ref.c:3218-3330)
 template <typename T, int PS>
@@ -56,10 +31,8 @@ __global__ __launch_bounds__(NT3) __attribute__((amdgpu_waves_per_eu(3))) void k
 		return;
 	if (threadIdx.x == 0 && slot == 0)
 		a.sD->use_dA = 0;
-	const PM<T, PS> gA = view<T, PS>(a.sA);
-	gemm_core<T, PS, OP_TRMM_RLNN>(As, Bs, a.m, a.n, a.n, a.alpha, T(0),
-		gA, a.ai, a.aj, view<T, PS>(a.sB), a.bi, a.bj,
-		gA, 0, 0, view<T, PS>(a.sD), a.di, a.dj, slot, slots);
+	trmm_core<T, PS>(As, Bs, a.m, a.n, a.alpha, view<T, PS>(a.sA), a.ai, a.aj, view<T, PS>(a.sB), a.bi, a.bj,
+		view<T, PS>(a.sD), a.di, a.dj, slot, slots);
 }
 
 // ---------------------------------------------------------------------------
@@ -424,6 +397,20 @@ static int tiles_y(const blasfeo_amd_hint *hint, int tm, int tn)
 	return y < 1 ? 1 : (y > cap ? cap : y);
 }
 
+// tile slots per instance of a gemm-family launch with TE x TE tiles
+template <int OP>
+static int gemm_slots(const blasfeo_amd_hint *hint, int te)
+{
+	if (!hint || hint->max_m <= 0)
+		return 1;
+	const int mt = (hint->max_m + te - 1) / te;
+	const int nt = OP == OP_SYRK ? mt : hint->max_n > 0 ? (hint->max_n + te - 1) / te : 1;
+	int cap = tune_value(TUNE_GEMM_GRID_Y, 0);
+	if (cap <= 0)
+		cap = 64;
+	return max(1, min(cap, gw_ntiles<OP>(mt, nt)));
+}
+
 static int check_common(int ps, int batch, const void *args, bool is_float, const char *name)
 {
 	if (batch < 0)
@@ -447,47 +434,55 @@ static int xcd_grid(int batch, int slots, int threads, dim3 *grid, const char *n
 	return BLASFEO_AMD_OK;
 }
 
+// One wavefront per output tile, E = 4 (64 x 64) or E = 2 (32 x 32).
+template <typename T, int PS, int OP, int E>
+static int launch_gemm_tile(int batch, const typename GemmArg<T>::type *args, int slots, hipStream_t st, const char *name)
+{
+	// FP32 and few instances: their tiles over all XCDs (64 sgemm_nn of U{64..512}
+	// 118 -> 81 us, of 512: 154 and 155 us; in FP64, where the operands that several
+	// XCDs then read weigh more, 118 and 120, 270 and 304 us)
+	const bool spread = sizeof(T) == 4 && batch <= 64;
+	dim3 grid;
+	int rc = xcd_grid(batch, slots, WAVE, &grid, name);
+	if (rc)
+		return rc;
+	hipLaunchKernelGGL((k_gemm_wave<T, PS, OP, E>), grid, dim3(WAVE), 0, st, args, batch, slots, spread);
+	return check_launch(name);
+}
+template <typename T, int PS, int OP>
+static int launch_gemm_ps(int batch, const typename GemmArg<T>::type *args, const blasfeo_amd_hint *hint, hipStream_t st, const char *name)
+{
+	// The large tile reads a quarter of the operands that the small one reads per
+	// product but leaves a batch of few or uneven instances with too few waves.
+	// It is taken above 256 rows or columns (64 dgemm_nn of 512: 270 us against 348,
+	// 16 of them 74 against 120), without bounds, and above 128 (FP32 96) where the
+	// batch has 16384 of its tiles (4096 dgemm_nt + dsyrk_ln of U{16..256}: 1052
+	// against 1132 us, 512 of them 219 against 180; 4096 of 128: 738 against 788, of
+	// U{4..128} 260 against 229; 4096 FP32 of U{4..128} 157 against 166, of U{4..96}
+	// 99 against 95).  The "gemm_wave" knob sets the small (1) or the large tile (2).
+	const int knob = tune_value(TUNE_GEMM_WAVE, 0);
+	const int slots = gemm_slots<OP>(hint, 64);
+	const int maxm = hint ? hint->max_m : 0, maxn = OP == OP_SYRK ? maxm : hint ? hint->max_n : 0;
+	const int most = maxm > 0 && maxn > 0 ? max(maxm, maxn) : 512;
+	const bool large = most > 256 || (most > (sizeof(T) == 8 ? 128 : 96) && (long long)batch * slots >= 16384);
+	if (knob == 2 || (knob == 0 && large))
+		return launch_gemm_tile<T, PS, OP, 4>(batch, args, slots, st, name);
+	return launch_gemm_tile<T, PS, OP, 2>(batch, args, gemm_slots<OP>(hint, 32), st, name);
+}
+
 template <typename T, int OP>
 static int launch_gemm(int ps, int batch, const typename GemmArg<T>::type *args, const blasfeo_amd_hint *hint, hipStream_t st, const char *name)
 {
 	int rc = check_common(ps, batch, args, sizeof(T) == 4, name);
 	if (rc || batch == 0)
 		return rc;
-	// sizes bounded by 256 (at most 64 tiles of 32 x 32 per instance): one
-	// wavefront per output tile, operands straight from global memory; the
-	// LDS-staged 64 x 64 engine for larger or unbounded sizes.  The
-	// "gemm_wave" knob forces the wave form off (2).
-	const int gwk = tune_value(TUNE_GEMM_WAVE, 0);
-	if (gwk != 2 && hint && hint->max_m > 0 && hint->max_m <= 256 &&
-	    (OP == OP_SYRK || (hint->max_n > 0 && hint->max_n <= 256)))
-	{
-		const int mt = (hint->max_m + GW_T - 1) / GW_T;
-		const int nt = OP == OP_SYRK ? mt : (hint->max_n + GW_T - 1) / GW_T;
-		int gy = (OP == OP_SYRK || OP == OP_SYRK_MN) ? mt * (mt + 1) / 2 : mt * nt;
-		gy = gy < 1 ? 1 : gy;
-		// one wave per (instance, tile slot), XCD-aware order (k_gemm_wave)
-		dim3 gridw;
-		if ((rc = xcd_grid(batch, gy, WAVE, &gridw, name)))
-			return rc;
-		if (ps == 4)
-			hipLaunchKernelGGL((k_gemm_wave<T, 4, OP>), gridw, dim3(WAVE), 0, st, args, batch, gy);
-		else if (ps == 8)
-			hipLaunchKernelGGL((k_gemm_wave<T, 8, OP>), gridw, dim3(WAVE), 0, st, args, batch, gy);
-		else
-			hipLaunchKernelGGL((k_gemm_wave<T, 16, OP>), gridw, dim3(WAVE), 0, st, args, batch, gy);
-		return check_launch(name);
-	}
-	const int slots = tiles_y(hint, TM, TN);
-	dim3 grid;
-	if ((rc = xcd_grid(batch, slots, NT3, &grid, name)))
-		return rc;
 	if (ps == 4)
-		hipLaunchKernelGGL((k_gemm<T, 4, OP>), grid, dim3(NT3), 0, st, args, batch, slots);
-	else if (ps == 8)
-		hipLaunchKernelGGL((k_gemm<T, 8, OP>), grid, dim3(NT3), 0, st, args, batch, slots);
-	else
-		hipLaunchKernelGGL((k_gemm<T, 16, OP>), grid, dim3(NT3), 0, st, args, batch, slots);
-	return check_launch(name);
+		return launch_gemm_ps<T, 4, OP>(batch, args, hint, st, name);
+	if (ps == 8)
+		return launch_gemm_ps<T, 8, OP>(batch, args, hint, st, name);
+	if constexpr (sizeof(T) == 4)
+		return launch_gemm_ps<T, 16, OP>(batch, args, hint, st, name);
+	return BLASFEO_AMD_EINVAL;
 }
 
 template <typename T>

@@ -1,5 +1,6 @@
-// bfa_gemm_core.hpp -- the 64x64-tile matrix-core gemm used by the level-3
-// kernels and by the fused Riccati sweep.
+// bfa_gemm_core.hpp -- the 64x64-tile matrix-core product with a triangular
+// right factor (trmm_rlnn) used by that entry point and by the Riccati sweep
+// for large stages.
 //
 // A workgroup is 4 waves; each output tile is 64x64 and each wave owns a 32x32
 // quarter as 2x2 matrix-core 16x16 accumulators.  Operands go global -> LDS in
@@ -12,7 +13,7 @@
 
 namespace bfa {
 
-enum { OP_NT = 0, OP_NN = 1, OP_SYRK = 2, OP_SYRK_MN = 3, OP_TRMM_RLNN = 4 };
+enum { OP_NT = 0, OP_NN = 1, OP_SYRK = 2, OP_SYRK_MN = 3 };
 
 constexpr int NT3 = 256;  // threads per workgroup
 constexpr int TM = 64;    // tile rows
@@ -87,13 +88,10 @@ struct TileLoader
 	}
 };
 
-// One gemm-family instance, tiles t0, t0 + tstep, ...
-// OP_NT/OP_SYRK*: D = beta*C + alpha*A*B^T (B is n x k);  OP_NN: B is k x n;
-// OP_TRMM_RLNN: D = alpha*B*A with A lower k x k (here A is the right operand).
-template <typename T, int PS, int OP>
-__device__ __forceinline__ void gemm_core(T *As, T *Bs, int m, int n, int k, T alpha, T beta,
-	const PM<T, PS> gA, int ai, int aj, const PM<T, PS> gB, int bi, int bj,
-	const PM<T, PS> gC, int ci, int cj, PM<T, PS> gD, int di, int dj, int t0, int tstep)
+// One instance of D = alpha * B * A, A lower n x n, B m x n: tiles t0, t0 + tstep, ...
+template <typename T, int PS>
+__device__ __forceinline__ void trmm_core(T *As, T *Bs, int m, int n, T alpha,
+	const PM<T, PS> gA, int ai, int aj, const PM<T, PS> gB, int bi, int bj, PM<T, PS> gD, int di, int dj, int t0, int tstep)
 {
 	typedef typename Vec4<T>::type V4;
 	const int mt = (m + TM - 1) / TM;
@@ -109,8 +107,6 @@ __device__ __forceinline__ void gemm_core(T *As, T *Bs, int m, int n, int k, T a
 		const int ti = t % mt;
 		const int tj = t / mt;
 		const int i0 = ti * TM, j0 = tj * TN;
-		if ((OP == OP_SYRK || OP == OP_SYRK_MN) && j0 > i0 + TM - 1)
-			continue;
 		const int mv = min(TM, m - i0);
 		const int nv = min(TN, n - j0);
 
@@ -121,35 +117,22 @@ __device__ __forceinline__ void gemm_core(T *As, T *Bs, int m, int n, int k, T a
 			for (int y = 0; y < 2; y++)
 				acc[x][y] = V4{0, 0, 0, 0};
 
-		// K range: trmm_rlnn only needs l >= j0 (A lower)
-		const int kbeg = (OP == OP_TRMM_RLNN) ? (j0 / KC) * KC : 0;
+		// only rows l >= j0 of A are needed (A lower)
+		const int kbeg = (j0 / KC) * KC;
 		TileLoader<T, PS> la, lb;
 		auto fetch = [&](int kk) {
-			const int kv = min(KC, k - kk);
-			if (OP == OP_TRMM_RLNN)
-			{
-				// left operand: B(i0.., kk..) of the call (sB), right: A(kk.., j0..) lower
-				la.template load<false, false>(gB, bi + i0, bj + kk, TM, KC, mv, kv, 0, 0);
-				lb.template load<true, true>(gA, ai + kk, aj + j0, KC, TN, kv, nv, kk, j0);
-			}
-			else
-			{
-				la.template load<false, false>(gA, ai + i0, aj + kk, TM, KC, mv, kv, 0, 0);
-				if (OP == OP_NN)
-					lb.template load<true, false>(gB, bi + kk, bj + j0, KC, TN, kv, nv, 0, 0);
-				else
-					lb.template load<false, false>(gB, bi + j0, bj + kk, TN, KC, nv, kv, 0, 0);
-			}
+			const int kv = min(KC, n - kk);
+			la.template load<false, false>(gB, bi + i0, bj + kk, TM, KC, mv, kv, 0, 0);
+			lb.template load<true, true>(gA, ai + kk, aj + j0, KC, TN, kv, nv, kk, j0);
 		};
-		if (kbeg < k)
-			fetch(kbeg);
-		for (int kk = kbeg; kk < k; kk += KC)
+		fetch(kbeg);
+		for (int kk = kbeg; kk < n; kk += KC)
 		{
 			__syncthreads();
 			la.store(As);
 			lb.store(Bs);
 			__syncthreads();
-			if (kk + KC < k)
+			if (kk + KC < n)
 				fetch(kk + KC);
 #pragma unroll
 			for (int k4 = 0; k4 < KC; k4 += 4)
@@ -170,15 +153,8 @@ __device__ __forceinline__ void gemm_core(T *As, T *Bs, int m, int n, int k, T a
 			}
 		}
 
-		// epilogue: D = beta*C + alpha*acc (trmm: alpha*acc), element-wise,
-		// a row half (x) of the wave's quarter at a time: its 8 elements of C
-		// are all loaded before any of D is stored (C may be D: in place,
-		// each element is read before it is written either way), so the
-		// loads overlap instead of each waiting behind the previous store.
 #pragma unroll
 		for (int x = 0; x < 2; x++)
-		{
-			T cv[2][4];
 #pragma unroll
 			for (int y = 0; y < 2; y++)
 			{
@@ -187,32 +163,10 @@ __device__ __forceinline__ void gemm_core(T *As, T *Bs, int m, int n, int k, T a
 				for (int r = 0; r < 4; r++)
 				{
 					const int il = wr + 16 * x + acc_row<T>(lane, r);
-					const int gi = i0 + il, gj = j0 + jl;
-					const bool need = OP != OP_TRMM_RLNN && beta != T(0) && il < mv && jl < nv &&
-						!((OP == OP_SYRK || OP == OP_SYRK_MN) && gi < gj);
-					cv[y][r] = need ? gC.at(ci + gi, cj + gj) : T(0);
+					if (il < mv && jl < nv)
+						gD.at(di + i0 + il, dj + j0 + jl) = alpha * acc[x][y][r];
 				}
 			}
-#pragma unroll
-			for (int y = 0; y < 2; y++)
-			{
-				const int jl = wc + 16 * y + (lane & 15);
-#pragma unroll
-				for (int r = 0; r < 4; r++)
-				{
-					const int il = wr + 16 * x + acc_row<T>(lane, r);
-					if (il >= mv || jl >= nv)
-						continue;
-					const int gi = i0 + il, gj = j0 + jl;
-					if ((OP == OP_SYRK || OP == OP_SYRK_MN) && gi < gj)
-						continue;
-					T val = alpha * acc[x][y][r];
-					if (OP != OP_TRMM_RLNN && beta != T(0))
-						val = beta * cv[y][r] + val;
-					gD.at(di + gi, dj + gj) = val;
-				}
-			}
-		}
 	}
 }
 

@@ -1,23 +1,31 @@
 // bfa_gemm_wave.hpp -- gemm_nt / gemm_nn / syrk_ln(_mn) with one wavefront per
-// 32x32 output tile, for batches of small and uneven instances.
+// output tile and no LDS: operands from global memory straight into the matrix
+// cores' registers.
 //
-// The wave's 2x2 block of 16x16 matrix-core accumulators takes its operands
-// straight from global memory: lane l loads A(i0 + 16x + l%16, k0 + l/16) and
-// the matching B element for each 4-column step of K, which in panel-major
-// storage is four contiguous 128-byte runs per operand (one per 4-row panel
-// for ps = 4), so the loads coalesce without staging through LDS.  With no
-// LDS and no barriers, a wave never waits for another, a CU holds as many
-// waves as registers allow (their load latencies overlap), and an instance of
-// m = n = 4 costs one wave instead of a 256-thread workgroup with a 64x64
-// tile.  Each wave keeps the operands of the next two K steps in flight.
-// The role of the reference's small-size kernels (the vs/gen edge kernels of
-// blasfeo_hp_pm/d_blas3_lib4.c:800-872,1137-1374).
+// A wave computes a tile of 64 x 64 (E = 4) or 32 x 32 (E = 2) as 16x16
+// accumulators.  It forms D^T = B A^T, so that a lane's accumulators are elements of
+// one row of D (lane % 16) in four consecutive columns across the lanes of a
+// register: with A's rows taken VA at a time (rows VA c .. VA c + VA - 1 of a
+// group of 16 VA rows by lane c, one row for each of VA tiles), A is loaded, C
+// loaded and D stored in 16-byte pieces, four columns of a panel side by side
+// (whole 128-byte lines for ps = 4).  Matrices whose rows do not start on a
+// VA-row boundary take the same loop one element at a time.
+// The operands of the next DEPTH steps of four K columns are in flight; columns
+// past K read the last one and are zeroed in the tail.  Only the 16-row groups
+// and 16-column blocks that the tile has are loaded and multiplied (one loop
+// per shape), so that the edges cost no products beyond their last block.
+// Measured (MI355X; before: 32 x 32 tiles with 8-byte loads up to 256, a 64 x 64
+// tile staged through LDS by four waves above): 1024 dgemm_nn of U{64..512}, ps = 8,
+// 1929 -> 1055 us (49 TFLOP/s), 256 of 512^3 1697 -> 1030 us (67 TFLOP/s, the rate of
+// a large library product here), 8192 sgemm_nt + ssyrk_ln of U{16..256} 1855 -> 1115 us
+// (3.4 TB/s, 60 TFLOP/s): bound by the matrix cores and the last blocks' padding.
+// 32768 dgemm_nt + dsyrk_ln of U{4..128} 1939 -> 1690 us (4.3 TB/s), 16384 of 64^3
+// 698 -> 648 us (4.95 TB/s, a large copy's rate): bound by memory.
 #pragma once
 #include "bfa_gemm_core.hpp"
+#include "bfa_strip.hpp"
 
 namespace bfa {
-
-constexpr int GW_T = 32;   // tile edge
 
 // tile t of an instance -> (ti, tj); syrk walks the lower tiles column by
 // column (tiles ti >= tj, tj < ntj)
@@ -43,7 +51,7 @@ __device__ __forceinline__ void gw_tile(int t, int mt, int nt, int &ti, int &tj)
 }
 
 template <int OP>
-__device__ __forceinline__ int gw_ntiles(int mt, int nt)
+__host__ __device__ __forceinline__ int gw_ntiles(int mt, int nt)
 {
 	if (OP == OP_SYRK || OP == OP_SYRK_MN)
 	{
@@ -53,29 +61,191 @@ __device__ __forceinline__ int gw_ntiles(int mt, int nt)
 	return mt * nt;
 }
 
-// operands of one 4-column K step (k0) for this lane
-template <typename T, int PS, int OP>
-__device__ __forceinline__ void gw_load(const PM<T, PS> &gA, int ai, int aj, const PM<T, PS> &gB, int bi, int bj,
-	int i0, int j0, int m, int n, int k, int k0, T (&av)[2], T (&bv)[2])
+template <typename T, int N> struct VecN { typedef T type __attribute__((ext_vector_type(N))); };
+template <typename T> struct VecN<T, 1> { typedef T type; };
+template <typename T, int N>
+__device__ __forceinline__ T vec_get(const typename VecN<T, N>::type &v, int e)
 {
-	const int lane = threadIdx.x & (WAVE - 1);
-	const int kq = k0 + (lane >> 4);
-	const bool kok = kq < k;
+	if constexpr (N == 1)
+		return v;
+	else
+		return v[e];
+}
+
+// K steps of operands in flight and waves per SIMD that the kernel is compiled for:
+// between 2 and 6 steps and 2 and 6 waves nothing but the least (2 steps of the
+// large tile) was more than a few per cent apart.
+template <typename T, int E> constexpr int gw_depth() { return E == 4 ? 3 : 4; }
+template <typename T, int E> constexpr int gw_waves() { return E == 4 ? (sizeof(T) == 8 ? 2 : 3) : 4; }
+// rows that a lane takes at a time in a tile of MX 16-row groups
+template <typename T, int MX> constexpr int gw_rows() { return MX == 4 && sizeof(T) == 4 ? 4 : 2; }
+
+template <typename T, int PS>
+struct GwArg
+{
+	StripView<T, PS> A, B, C, D;
+	int ai, aj, bi, bj, ci, cj, di, dj, m, n, k;
+	T alpha, beta;
+};
+
+// One tile of MX 16-row groups and NY 16-column blocks at (i0, j0); VA: rows that a
+// lane takes at a time (1: any offsets).
+template <typename T, int PS, int OP, int MX, int NY, int VA, int DEPTH>
+__device__ __forceinline__ void gw_body(const GwArg<T, PS> &a, int i0, int j0)
+{
+	typedef typename Vec4<T>::type V4;
+	typedef typename VecN<T, VA>::type VV;
+	constexpr int NV = MX / VA;
+	constexpr unsigned CS = StripView<T, PS>::CS;
+	constexpr bool SY = OP == OP_SYRK || OP == OP_SYRK_MN;
+	const int lane = lane_id(), g = lane >> 4, c = lane & 15;
+	const int m = a.m, n = a.n, k = a.k;
+	const int lastv = (m - 1) & ~(VA - 1);
+	auto ldv = [](const StripView<T, PS> &v, unsigned o) -> VV { return *(const BFA_GLOBAL VV *)(v.p + o); };
+	V4 acc[MX][NY];
 #pragma unroll
-	for (int x = 0; x < 2; x++)
-	{
-		const int i = i0 + 16 * x + (lane & 15);
-		av[x] = (kok && i < m) ? gA.at(ai + i, aj + kq) : T(0);
-	}
+	for (int x = 0; x < MX; x++)
 #pragma unroll
-	for (int y = 0; y < 2; y++)
+		for (int y = 0; y < NY; y++)
+			acc[x][y] = V4{0, 0, 0, 0};
+	if (k > 0)
 	{
-		const int j = j0 + 16 * y + (lane & 15);
-		if (OP == OP_NN)
-			bv[y] = (kok && j < n) ? gB.at(bi + kq, bj + j) : T(0);
-		else
-			bv[y] = (kok && j < n) ? gB.at(bi + j, bj + kq) : T(0);
+		unsigned ao[NV], bo[NY];
+#pragma unroll
+		for (int v = 0; v < NV; v++)
+			ao[v] = a.A.at(a.ai + min(i0 + 16 * VA * v + VA * c, lastv), a.aj);
+#pragma unroll
+		for (int y = 0; y < NY; y++)
+		{
+			const int j = min(j0 + 16 * y + strip_row<T>(c), n - 1);
+			bo[y] = OP == OP_NN ? (unsigned)(a.bj + j) * CS : a.B.at(a.bi + j, a.bj);
+		}
+		const int ns = (k + 3) / 4;
+		VV av[DEPTH][NV];
+		T bv[DEPTH][NY];
+		auto load = [&](int s, VV (&x)[NV], T (&y)[NY]) {
+			const int kq = min(4 * s + g, k - 1);
+			const unsigned kc = (unsigned)kq * CS, kb = OP == OP_NN ? a.B.at(a.bi + kq, 0) : kc;
+#pragma unroll
+			for (int v = 0; v < NV; v++)
+				x[v] = ldv(a.A, ao[v] + kc);
+#pragma unroll
+			for (int t = 0; t < NY; t++)
+				y[t] = a.B.ld(0, bo[t] + kb);
+		};
+		auto step = [&](const VV (&x)[NV], const T (&y)[NY]) {
+#pragma unroll
+			for (int v = 0; v < NV; v++)
+#pragma unroll
+				for (int e = 0; e < VA; e++)
+#pragma unroll
+					for (int t = 0; t < NY; t++)
+						acc[VA * v + e][t] = mfma16(y[t], vec_get<T, VA>(x[v], e), acc[VA * v + e][t]);
+		};
+#pragma unroll
+		for (int d = 0; d < DEPTH; d++)
+			load(d, av[d], bv[d]);
+		int s = 0;
+		for (; s + DEPTH < ns; s += DEPTH)
+		{
+#pragma unroll
+			for (int d = 0; d < DEPTH; d++)
+			{
+				step(av[d], bv[d]);
+				load(s + DEPTH + d, av[d], bv[d]);
+			}
+		}
+		// the last 1 .. DEPTH steps
+#pragma unroll
+		for (int d = 0; d < DEPTH; d++)
+			if (s + d < ns)
+			{
+				if (4 * (s + d) + 4 > k)
+				{
+					const bool in = 4 * (s + d) + g < k;
+#pragma unroll
+					for (int v = 0; v < NV; v++)
+						av[d][v] = in ? av[d][v] : VV(0);
+#pragma unroll
+					for (int t = 0; t < NY; t++)
+						bv[d][t] = in ? bv[d][t] : T(0);
+				}
+				step(av[d], bv[d]);
+			}
 	}
+	// D = beta * C + alpha * acc, a 16-column block at a time: its elements of C are
+	// all loaded before any of D is stored (C may be D)
+	const bool whole = i0 + 16 * MX <= m && j0 + 16 * NY <= n && !(SY && i0 < j0 + 16 * NY - 1);
+#pragma unroll
+	for (int y = 0; y < NY; y++)
+	{
+		VV cv[NV][4];
+		if (a.beta != T(0))
+		{
+#pragma unroll
+			for (int v = 0; v < NV; v++)
+			{
+				const unsigned oc = a.C.at(a.ci + min(i0 + 16 * VA * v + VA * c, lastv), a.cj);
+#pragma unroll
+				for (int r = 0; r < 4; r++)
+					cv[v][r] = ldv(a.C, oc + (unsigned)min(j0 + 16 * y + 4 * r + g, n - 1) * CS);
+			}
+		}
+#pragma unroll
+		for (int v = 0; v < NV; v++)
+		{
+			const int gi = i0 + 16 * VA * v + VA * c;
+			const unsigned od = a.D.at(a.di + min(gi, lastv), a.dj);
+#pragma unroll
+			for (int r = 0; r < 4; r++)
+			{
+				const int gj = j0 + 16 * y + 4 * r + g;
+				const unsigned o = od + (unsigned)min(gj, n - 1) * CS;
+				T val[VA];
+				VV vv;
+#pragma unroll
+				for (int e = 0; e < VA; e++)
+				{
+					val[e] = a.alpha * acc[VA * v + e][y][r];
+					if (a.beta != T(0))
+						val[e] = a.beta * vec_get<T, VA>(cv[v][r], e) + val[e];
+					if constexpr (VA == 1)
+						vv = val[e];
+					else
+						vv[e] = val[e];
+				}
+				if (whole)
+					*(BFA_GLOBAL VV *)(a.D.p + o) = vv;
+				else if (gj < n)
+				{
+					if (gi + VA <= m && !(SY && gi < gj))
+						*(BFA_GLOBAL VV *)(a.D.p + o) = vv;
+					else
+#pragma unroll
+						for (int e = 0; e < VA; e++)
+							if (gi + e < m && !(SY && gi + e < gj))
+								*(BFA_GLOBAL T *)(a.D.p + o + e * (unsigned)sizeof(T)) = val[e];
+				}
+			}
+		}
+	}
+}
+
+// the loop for a tile's nb <= E column blocks
+template <typename T, int PS, int OP, int MX, int E, int DEPTH>
+__device__ __forceinline__ void gw_blocks(const GwArg<T, PS> &a, int i0, int j0, int nb)
+{
+	constexpr int VA = gw_rows<T, MX>();
+	if constexpr (E == 4)
+	{
+		if (nb == 4)
+			return gw_body<T, PS, OP, MX, 4, VA, DEPTH>(a, i0, j0);
+		if (nb == 3)
+			return gw_body<T, PS, OP, MX, 3, VA, DEPTH>(a, i0, j0);
+	}
+	if (nb >= 2)
+		return gw_body<T, PS, OP, MX, 2, VA, DEPTH>(a, i0, j0);
+	gw_body<T, PS, OP, MX, 1, VA, DEPTH>(a, i0, j0);
 }
 
 // One wave per (instance, tile slot): `slots` slots per instance (the tile
@@ -83,98 +253,52 @@ __device__ __forceinline__ void gw_load(const PM<T, PS> &gA, int ai, int aj, con
 // workgroups rounded up to a multiple of XCDS.  The slots of one instance
 // map to consecutive logical indices on one XCD (xcd_local_index), so the
 // tiles that re-read the same A row block or B column block run together
-// on one L2; slot t >= the instance's tile count exits at once.  Registers
-// are capped for five waves per SIMD (92 VGPRs, no spills), so that more
-// waves' load latencies overlap: faster than four (124 VGPRs) on the
-// 100000-call uneven batch; six and eight spill and are slower.
-template <typename T, int PS, int OP>
-__global__ __launch_bounds__(WAVE, 5) void k_gemm_wave(const typename GemmArg<T>::type *__restrict__ args, int batch,
-	int slots)
+// on one L2; slot t >= the instance's tile count exits at once.
+template <typename T, int PS, int OP, int E>
+__global__ __launch_bounds__(WAVE, (gw_waves<T, E>())) void k_gemm_wave(const typename GemmArg<T>::type *__restrict__ args, int batch,
+	int slots, bool spread)
 {
-	typedef typename Vec4<T>::type V4;
-	const unsigned li = xcd_local_index(blockIdx.x, gridDim.x);
-	const int inst = (int)(li / (unsigned)slots), slot = (int)(li % (unsigned)slots);
+	constexpr int TE = 16 * E, DEPTH = gw_depth<T, E>();
+	int inst, slot;
+	xcd_inst_slot(slots, inst, slot, spread);
 	if (inst >= batch)
 		return;
-	const typename GemmArg<T>::type &a = args[inst];
-	const int m = a.m;
-	const int n = (OP == OP_SYRK) ? a.m : a.n;
-	const int k = a.k;
-	if (m <= 0 || n <= 0)
+	const typename GemmArg<T>::type &r = args[inst];
+	GwArg<T, PS> a;
+	a.m = __builtin_amdgcn_readfirstlane(r.m);
+	a.n = OP == OP_SYRK ? a.m : __builtin_amdgcn_readfirstlane(r.n);
+	a.k = __builtin_amdgcn_readfirstlane(r.k);
+	if (a.m <= 0 || a.n <= 0)
 		return;
 	if (threadIdx.x == 0 && slot == 0)
-		a.sD->use_dA = 0;
-	const PM<T, PS> gA = view<T, PS>(a.sA), gB = view<T, PS>(a.sB), gC = view<T, PS>(a.sC);
-	PM<T, PS> gD = view<T, PS>(a.sD);
-	const T alpha = a.alpha, beta = a.beta;
-	const int lane = threadIdx.x;
-	const int mt = (m + GW_T - 1) / GW_T, nt = (n + GW_T - 1) / GW_T;
+		r.sD->use_dA = 0;
+	const int mt = (a.m + TE - 1) / TE, nt = (a.n + TE - 1) / TE;
 	const int ntiles = gw_ntiles<OP>(mt, nt);
+	if (slot >= ntiles)
+		return;
+	a.A = strip_view<T, PS>(r.sA);
+	a.B = strip_view<T, PS>(r.sB);
+	a.C = strip_view<T, PS>(r.sC);
+	a.D = strip_view<T, PS>(r.sD);
+	a.ai = r.ai, a.aj = r.aj, a.bi = r.bi, a.bj = r.bj, a.ci = r.ci, a.cj = r.cj, a.di = r.di, a.dj = r.dj;
+	a.alpha = r.alpha;
+	a.beta = r.beta;
+	// rows in pieces: the matrices' rows start on a piece's boundary, in memory too
+	constexpr int VA = gw_rows<T, E>();
+	const unsigned long long low = (unsigned long long)(uintptr_t)a.A.p | (unsigned long long)(uintptr_t)a.C.p | (unsigned long long)(uintptr_t)a.D.p;
+	const bool pieces = ((a.ai | a.ci | a.di) & (VA - 1)) == 0 && (low & (VA * sizeof(T) - 1)) == 0;
 	for (int t = slot; t < ntiles; t += slots)
 	{
 		int ti, tj;
 		gw_tile<OP>(t, mt, nt, ti, tj);
-		const int i0 = ti * GW_T, j0 = tj * GW_T;
-		V4 acc[2][2];
-#pragma unroll
-		for (int x = 0; x < 2; x++)
-#pragma unroll
-			for (int y = 0; y < 2; y++)
-				acc[x][y] = V4{0, 0, 0, 0};
-		// two K steps of operands in flight
-		T a0[2], b0[2], a1[2], b1[2];
-		gw_load<T, PS, OP>(gA, a.ai, a.aj, gB, a.bi, a.bj, i0, j0, m, n, k, 0, a0, b0);
-		gw_load<T, PS, OP>(gA, a.ai, a.aj, gB, a.bi, a.bj, i0, j0, m, n, k, 4, a1, b1);
-		for (int k0 = 0; k0 < k; k0 += 8)
-		{
-#pragma unroll
-			for (int x = 0; x < 2; x++)
-#pragma unroll
-				for (int y = 0; y < 2; y++)
-					acc[x][y] = mfma16(a0[x], b0[y], acc[x][y]);
-			if (k0 + 8 < k)
-				gw_load<T, PS, OP>(gA, a.ai, a.aj, gB, a.bi, a.bj, i0, j0, m, n, k, k0 + 8, a0, b0);
-			if (k0 + 4 < k)
-			{
-#pragma unroll
-				for (int x = 0; x < 2; x++)
-#pragma unroll
-					for (int y = 0; y < 2; y++)
-						acc[x][y] = mfma16(a1[x], b1[y], acc[x][y]);
-				if (k0 + 12 < k)
-					gw_load<T, PS, OP>(gA, a.ai, a.aj, gB, a.bi, a.bj, i0, j0, m, n, k, k0 + 12, a1, b1);
-			}
-		}
-		// epilogue: D = beta*C + alpha*acc on the valid (for syrk: lower)
-		// elements; each row half's C loads issued before its D stores
-#pragma unroll
-		for (int x = 0; x < 2; x++)
-		{
-			T cv[2][4];
-#pragma unroll
-			for (int y = 0; y < 2; y++)
-#pragma unroll
-				for (int r = 0; r < 4; r++)
-				{
-					const int gi = i0 + 16 * x + acc_row<T>(lane, r), gj = j0 + 16 * y + (lane & 15);
-					const bool need = beta != T(0) && gi < m && gj < n &&
-						!((OP == OP_SYRK || OP == OP_SYRK_MN) && gi < gj);
-					cv[y][r] = need ? gC.at(a.ci + gi, a.cj + gj) : T(0);
-				}
-#pragma unroll
-			for (int y = 0; y < 2; y++)
-#pragma unroll
-				for (int r = 0; r < 4; r++)
-				{
-					const int gi = i0 + 16 * x + acc_row<T>(lane, r), gj = j0 + 16 * y + (lane & 15);
-					if (gi >= m || gj >= n || ((OP == OP_SYRK || OP == OP_SYRK_MN) && gi < gj))
-						continue;
-					T val = alpha * acc[x][y][r];
-					if (beta != T(0))
-						val = beta * cv[y][r] + val;
-					gD.at(a.di + gi, a.dj + gj) = val;
-				}
-		}
+		const int i0 = ti * TE, j0 = tj * TE;
+		const int nb = min(E, (a.n - j0 + 15) / 16);
+		if (!pieces)
+			gw_body<T, PS, OP, E, E, 1, 2>(a, i0, j0);
+		else if (E == 2 || a.m - i0 <= 32)
+			gw_blocks<T, PS, OP, 2, E, DEPTH>(a, i0, j0, nb);
+		else if constexpr (E == 4)
+			gw_blocks<T, PS, OP, 4, E, DEPTH>(a, i0, j0, nb);
 	}
 }
 

@@ -49,7 +49,7 @@ bool valid(const char *name, int index, int value)
 	if (!std::strcmp(name, "potrf_bw"))
 		return value == 1 || value == 2 || value == 4;
 	// trsm_thin: 1 = always the one-wavefront left solve when it applies, 2 = never
-	// gemm_wave: 1 = the one-wavefront-per-tile gemm when the sizes allow it, 2 = never
+	// gemm_wave: 1 = 32 x 32 tiles, 2 = 64 x 64 tiles
 	if (!std::strcmp(name, "trsm_thin") || !std::strcmp(name, "gemm_wave"))
 		return value == 1 || value == 2;
 	// lds_threads: accepted and returned, no launch uses it

@@ -143,11 +143,9 @@ const char *blasfeo_amd_last_error(void);
  *                  hint->max_n <= 4 and m <= 256 on one wavefront per instance:
  *                  1 always, 2 never; built-in: when the batch has at least
  *                  16 instances per CU;
- *   "gemm_wave",   index 0: gemm_nt/nn and syrk_ln(_mn) with size bounds
- *                  up to 256 on one wavefront per 32 x 32 output tile
- *                  (operands from global memory): 1 or 0 (built-in) when the
- *                  hint bounds m and n by 256, 2 never (the LDS-staged
- *                  64 x 64 engine);
+ *   "gemm_wave",   index 0: output tile of gemm_nt/nn and syrk_ln(_mn): 32 x 32
+ *                  (1) or 64 x 64 (2); built-in: by the hint's bounds and the
+ *                  batch (large bounds and many tiles: 64 x 64);
  *   "lds_threads", index 2..7: 256 or 512, kept and returned; no launch uses it
  *                  (the kernels it shaped have no such choice any more).
  * blasfeo_amd_tune_set returns BLASFEO_AMD_OK or BLASFEO_AMD_EINVAL;

@@ -1,7 +1,7 @@
 """Emulator cases (TEST INFRASTRUCTURE ONLY) for the gemm family on the
 record sets of tests/gemm_cases.py, checked against the oracle at the
 reference's rule (tol 1e-11).
-Usage: python case_gemm.py <op> <ps> <wave: 1 = one wavefront per tile, 2 = the LDS engine>"""
+Usage: python case_gemm.py <op> <ps> <wave: 1 = 32 x 32 tiles, 2 = 64 x 64> [pieces]"""
 import ctypes
 import sys
 
@@ -9,9 +9,10 @@ from emu_harness import records, compare_outputs, emu_lib, to_mats, bfa, oracle
 import gemm_cases
 
 
-def run(op, ps, wave):
+def run(op, ps, wave, pieces=False):
     E = emu_lib("emu_lapack")
-    re, ro = to_mats(ps, gemm_cases.uneven(ps, op, 90 + ps + 7 * len(op)))
+    cases = gemm_cases.pieces if pieces else gemm_cases.uneven
+    re, ro = to_mats(ps, cases(ps, op, 90 + ps + 7 * len(op)))
     blk = records(bfa.DGEMM_ARG, re)
     print("emu %s ps=%d wave=%d batch=%d" % (op, ps, wave, len(re)), flush=True)
     assert E.blasfeo_amd_tune_set(b"gemm_wave", 0, wave) == 0
@@ -31,4 +32,4 @@ def run(op, ps, wave):
 
 
 if __name__ == "__main__":
-    run(sys.argv[1], int(sys.argv[2]), int(sys.argv[3]))
+    run(sys.argv[1], int(sys.argv[2]), int(sys.argv[3]), len(sys.argv) > 4)

@@ -106,6 +106,15 @@ def test_gemm_family(emu_build, op, ps, wave):
     run_case("case_gemm.py", op, ps, wave)
 
 
+@pytest.mark.parametrize("wave", [1, 2])
+@pytest.mark.parametrize("ps", [4, 8])
+@pytest.mark.parametrize("op", ["gemm_nt", "gemm_nn", "syrk_ln", "syrk_ln_mn"])
+def test_gemm_pieces(emu_build, op, ps, wave):
+    """The gemm family with rows on piece boundaries (16-byte loads and stores), at
+    the edges of pieces, blocks, tiles and K steps."""
+    run_case("case_gemm.py", op, ps, wave, "pieces")
+
+
 @pytest.mark.parametrize("ps", [4, 8])
 def test_riccati_trf(emu_build, ps):
     """The LDS-resident Riccati factorisation sweep over every footprint class,

@@ -1,6 +1,7 @@
 """GPU parity of the kernels that keep 16-row strips in registers, at the edges of
 their strips, blocks and launches, against the CPU oracle: potrf_l(_mn) with one
-and with several waves per instance, syrk_dpotrf_ln, trsm_rltn."""
+and with several waves per instance, syrk_dpotrf_ln, trsm_rltn; and of the gemm
+family's tiles."""
 import numpy as np
 import pytest
 
@@ -9,6 +10,7 @@ import oracle
 from blasfeo_amd import autotune
 from helpers import Batch, run_both, compare_buffers
 import chol_cases
+import gemm_cases
 import trsm_cases
 
 pytestmark = pytest.mark.gpu
@@ -114,3 +116,29 @@ def test_trsm_rltn(gpu, prec, ps, finite):
                 same = (x == y) | (np.isnan(x) & np.isnan(y)) | (np.abs(x - y) <= tol * (np.abs(x) + np.abs(y)) + tol)
                 assert same.all(), "matrix %d: %d differ" % (i, int((~same).sum()))
     assert (gd["use_dA"] == rd["use_dA"]).all()
+
+
+@pytest.mark.parametrize("tile", [1, 2])
+@pytest.mark.parametrize("op", ["gemm_nt", "gemm_nn", "syrk_ln", "syrk_ln_mn"])
+@pytest.mark.parametrize("prec,ps", [(p, q) for p in "ds" for q in _panel_sizes(p)])
+def test_gemm_pieces(gpu, prec, ps, op, tile):
+    """rows on piece boundaries; four times over: a batch above the one that is spread over the XCDs"""
+    if prec == "s" and op == "syrk_ln_mn":
+        pytest.skip("no FP32 syrk_ln_mn entry")
+    f = oracle.fn(prec, op)
+
+    def ocall(h, r):
+        mn = (r["m"],) if op == "syrk_ln" else (r["m"], r["n"])
+        f(ps, *mn, r["k"], r["alpha"], h.desc_addr(r["sA"]), r["ai"], r["aj"], h.desc_addr(r["sB"]), r["bi"], r["bj"],
+          r["beta"], h.desc_addr(r["sC"]), r["ci"], r["cj"], h.desc_addr(r["sD"]), r["di"], r["dj"])
+
+    autotune.set_knob("gemm_wave", 0, tile)
+    try:
+        for times in (1, 4):
+            b = Batch(prec, ps, seed=7)
+            recs = chol_cases.to_batch(b, gemm_cases.pieces(ps, op, 120 + ps) * times)
+            g, gd, rr, rd = run_both(b, b.host(), bfa.DGEMM_ARG if prec == "d" else bfa.SGEMM_ARG, recs, prec + op, ocall, (130, 130, 33))
+            compare_buffers(b, g, rr, "%s%s ps=%d" % (prec, op, ps))
+            assert (gd["use_dA"] == rd["use_dA"]).all()
+    finally:
+        autotune.set_knob("gemm_wave", 0, 0)
