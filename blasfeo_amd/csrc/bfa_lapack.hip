@@ -2,7 +2,7 @@
 // syrk_dpotrf_ln(_mn) and getrf_rp on panel-major matrices.
 //
 // potrf and syrk_dpotrf up to 256 columns: 16-row strips in registers
-// (bfa_potrf_wave.hpp).  potrf above 256 columns and getrf: one workgroup
+// (bfa_potrf_wave.hpp), getrf up to 256 rows: bfa_getrf_wg.hpp.  Above: one workgroup
 // (4 waves) per instance, left-looking over 16-column panels held in LDS at full
 // height (the role of the reference's 12x4 / 8x8 register blocks,
 // blasfeo_hp_pm/d_lapack_lib4.c:954-985 and :2443-2634):
@@ -100,6 +100,11 @@ __device__ __forceinline__ int getrf_order(int t, int batch, const int *counts, 
 	return -1;
 }
 
+} // namespace bfa
+#include "bfa_getrf_wg.hpp"
+namespace bfa {
+
+// instances of more than 256 rows
 template <typename T, int PS, bool PIV = true>
 __global__ __launch_bounds__(NTL) __attribute__((amdgpu_waves_per_eu(4))) void k_getrf(const typename FactArg<T>::type *__restrict__ args, int mmax,
 	int batch = 0, const int *__restrict__ counts = nullptr, const int *__restrict__ lists = nullptr)
@@ -608,6 +613,18 @@ static int launch_potrf(int ps, int batch, const typename FactArg<T>::type *args
 	return check_launch(name);
 }
 
+template <typename T, bool PIV, int NW>
+static void launch_getrf_wg(int ps, int batch, const typename FactArg<T>::type *args, int mmax, const int *counts, const int *lists, hipStream_t st)
+{
+	constexpr size_t shm = sizeof(T) * 16 * (NW * WAVE + 1);
+	if (ps == 4)
+		hipLaunchKernelGGL((k_getrf_wg<T, 4, PIV, NW>), dim3(batch), dim3(NW * WAVE), shm, st, args, mmax, batch, counts, lists);
+	else if (ps == 8)
+		hipLaunchKernelGGL((k_getrf_wg<T, 8, PIV, NW>), dim3(batch), dim3(NW * WAVE), shm, st, args, mmax, batch, counts, lists);
+	else if constexpr (sizeof(T) == 4)
+		hipLaunchKernelGGL((k_getrf_wg<T, 16, PIV, NW>), dim3(batch), dim3(NW * WAVE), shm, st, args, mmax, batch, counts, lists);
+}
+
 template <typename T, bool PIV = true>
 static int launch_getrf(int ps, int batch, const typename FactArg<T>::type *args, const blasfeo_amd_hint *hint, hipStream_t st, const char *name)
 {
@@ -625,6 +642,20 @@ static int launch_getrf(int ps, int batch, const typename FactArg<T>::type *args
 	int *counts = ws, *lists = ws + 64;
 	hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(64), 0, st, counts, 64);
 	hipLaunchKernelGGL((k_getrf_plan<T>), dim3((batch + 255) / 256), dim3(256), 0, st, args, batch, counts, lists);
+	if (mmax <= GLU_M)
+	{
+		// the waves of a workgroup by the bound of the rows, so that small instances
+		// come with as many workgroups per CU as there are registers for; a launch
+		// for each range of rows was no faster on mixed batches (8192 LU solves of
+		// U{16..256} 3916 against 3925 us) and slower on small ones (512: 600, 806)
+		if (mmax <= 64)
+			launch_getrf_wg<T, PIV, 1>(ps, batch, args, mmax, counts, lists, st);
+		else if (mmax <= 128)
+			launch_getrf_wg<T, PIV, 2>(ps, batch, args, mmax, counts, lists, st);
+		else
+			launch_getrf_wg<T, PIV, 4>(ps, batch, args, mmax, counts, lists, st);
+		return check_launch(name);
+	}
 	if (ps == 4)
 		hipLaunchKernelGGL((k_getrf<T, 4, PIV>), dim3(batch), dim3(NTL), shm, st, args, mmax, batch, counts, lists);
 	else if (ps == 8)

@@ -122,6 +122,19 @@ uint64_t exch(uint64_t v, int src)
 	return r;
 }
 
+// the wave's predicates, every lane of it taking part
+uint64_t ballot(bool p)
+{
+	Wave &w = g_waves[t_wave];
+	w.slot[t_lane] = p;
+	wave_bar();
+	uint64_t r = 0;
+	for (int l = 0; l < 64; l++)
+		r |= (w.slot[l] & 1) << l;
+	wave_bar();
+	return r;
+}
+
 uint64_t exch_dpp(uint64_t old, uint64_t v, int ctrl, int row_mask, int bank_mask, bool bound_ctrl)
 {
 	Wave &w = g_waves[t_wave];

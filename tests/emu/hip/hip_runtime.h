@@ -76,6 +76,7 @@ uint64_t exch_dpp(uint64_t old, uint64_t v, int ctrl, int row_mask, int bank_mas
 void mfma_f64(double a, double b, double acc[4]);
 void mfma_f32(float a, float b, float acc[4]);
 int lane();
+uint64_t ballot(bool p);
 typedef void (*block_fn)(void *);
 void run_grid(dim3 grid, dim3 block, size_t shm, block_fn fn, void *ctx);
 }
@@ -136,6 +137,8 @@ inline emu_f4 emu_mfma_f(float a, float b, emu_f4 acc)
 }
 #define __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, x, y, z) emu_mfma_d((a), (b), (acc))
 #define __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc, x, y, z) emu_mfma_f((a), (b), (acc))
+
+inline uint64_t __ballot(bool p) { return emu::ballot(p); }
 
 template <typename T>
 inline T __shfl(T v, int src, int width = 64)

@@ -106,6 +106,15 @@ def test_gemm_family(emu_build, op, ps, wave):
     run_case("case_gemm.py", op, ps, wave)
 
 
+@pytest.mark.parametrize("bound", [64, 128, 256])
+@pytest.mark.parametrize("ps", [4, 8])
+@pytest.mark.parametrize("op", ["getrf_rp", "getrf_np"])
+def test_getrf(emu_build, op, ps, bound):
+    """LU with one, two and four waves per instance: edges of blocks, lane slots and
+    workgroups, tall and wide, in place, ties, zero columns, NaN and Inf."""
+    run_case("case_lu.py", op, ps, bound)
+
+
 @pytest.mark.parametrize("wave", [1, 2])
 @pytest.mark.parametrize("ps", [4, 8])
 @pytest.mark.parametrize("op", ["gemm_nt", "gemm_nn", "syrk_ln", "syrk_ln_mn"])
