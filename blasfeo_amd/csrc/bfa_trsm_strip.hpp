@@ -3,8 +3,9 @@
 // (bfa_strip.hpp).
 //
 // A wave holds S strips from their first block column to the last: block K is
-// alpha B_K minus the products of the finished blocks with the row block A_K, then
-// the solve with A_KK.  The four waves of a workgroup walk the block columns
+// alpha B_K minus the products of the finished blocks with the row block A_K (summed
+// before B_K is added, which keeps the rounding of the sum at the size of the
+// products), then the solve with A_KK.  The four waves of a workgroup walk the block columns
 // together: the tiles of row block A_K are brought to LDS once for all of them, as
 // operand tiles, dealt to the waves and loaded one block column ahead (read by
 // every wave for itself they came from L2 at a rate that bound the kernel).
@@ -12,8 +13,8 @@
 // Measured (MI355X, 8192 FP64 solves, ps = 4; before: the row block in LDS, one of
 // four waves solving the diagonal blocks): m = n = 32 125 -> 54 us, 64 235 -> 159,
 // 128 1608 -> 795, 256 15.3 -> 4.4 ms (31 TFLOP/s; 6.2 ms with every wave reading
-// A for itself); m, n ~ U{16..256} 4.61 -> 1.69 ms (2.15 before the slots of an
-// instance were turned, xcd_inst_slot).  Bound by memory up to 64
+// A for itself); m, n ~ U{16..256} 4.61 -> 1.80 ms (1.69 with the sum begun at B_K,
+// whose error was 2.4 times as large).  Bound by memory up to 64
 // columns, then by the matrix cores and the substitution's vector instructions,
 // with two waves per SIMD.
 #pragma once
@@ -140,9 +141,9 @@ __global__ __launch_bounds__(NT3, (trsm_waves<T, NB>())) void k_trsm_rltn(const 
 					V4 acc[S];
 #pragma unroll
 					for (int t = 0; t < S; t++)
-						acc[t] = alpha * nx[t][K];
+						acc[t] = V4{0, 0, 0, 0};
 #pragma unroll
-					for (int p = 0; p < K; p++)
+					for (int p = K - 1; p >= 0; p--)
 					{
 						T l[4];
 #pragma unroll
@@ -154,6 +155,9 @@ __global__ __launch_bounds__(NT3, (trsm_waves<T, NB>())) void k_trsm_rltn(const 
 							for (int t = 0; t < S; t++)
 								acc[t] = mfma16(l[s], nx[t][p][s], acc[t]);
 					}
+#pragma unroll
+					for (int t = 0; t < S; t++)
+						acc[t] += alpha * nx[t][K];
 					T x[S][4];
 					if constexpr (S == 2)
 						strip_solve2<T>(acc[0], acc[1], lk, d, x[0], x[1]);
@@ -213,14 +217,9 @@ __global__ __launch_bounds__(NT3, (trsm_waves<T, NB>())) void k_trsm_rltn(const 
 			V4 acc[S];
 #pragma unroll
 			for (int t = 0; t < S; t++)
-				acc[t] = alpha * cn[t];
+				acc[t] = V4{0, 0, 0, 0};
 			if (K + 1 < nb)
-			{
 				fetch(K + 1);
-#pragma unroll
-				for (int t = 0; t < S; t++)
-					strip_load<4>(B, ob[t], g, 16 * (K + 1), n, cn[t]);
-			}
 			T lk[3], d[4];
 #pragma unroll
 			for (int s = 0; s < 3; s++)
@@ -229,7 +228,7 @@ __global__ __launch_bounds__(NT3, (trsm_waves<T, NB>())) void k_trsm_rltn(const 
 			for (int s = 0; s < 4; s++)
 				d[s] = tr == tc ? inv_s[16 * K + 4 * s + tc] : buf[256 * K + trio[s]];
 #pragma unroll
-			for (int p = 0; p < NB - 1; p++)
+			for (int p = NB - 2; p >= 0; p--)
 				if (p < K)
 				{
 					T l[4];
@@ -242,6 +241,14 @@ __global__ __launch_bounds__(NT3, (trsm_waves<T, NB>())) void k_trsm_rltn(const 
 						for (int t = 0; t < S; t++)
 							acc[t] = mfma16(l[s], nx[t][p][s], acc[t]);
 				}
+#pragma unroll
+			for (int t = 0; t < S; t++)
+			{
+				acc[t] += alpha * cn[t];
+				// needed after the next block column's products
+				if (K + 1 < nb)
+					strip_load<4>(B, ob[t], g, 16 * (K + 1), n, cn[t]);
+			}
 			T x[S][4];
 			if constexpr (S == 2)
 				strip_solve2<T>(acc[0], acc[1], lk, d, x[0], x[1]);
