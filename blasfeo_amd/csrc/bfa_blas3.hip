@@ -211,139 +211,145 @@ __global__ __launch_bounds__(NT3) void k_trsm_left(const typename TrsmArg<T>::ty
 // ---------------------------------------------------------------------------
 // The same four left-side solves for few right-hand sides (chosen when the hint
 // bounds n by 4) and m <= 256: one wavefront per instance, row i of X in lane
-// i % 64 (slot i / 64), four columns of X at a time in registers.  Column j of the solve is taken in order (top-down for llnn
-// and llnu, bottom-up for lltn and lunn): row j's values are scaled by the
-// reciprocal diagonal and broadcast with v_readlane, and every row still to
-// be solved drops its multiple of them.  No barriers; the elements of A for
-// the next column are loaded while the current one is applied.
+// i % 64 (slot i / 64), four columns of X at a time in registers.  The columns j of
+// the solve are taken in order (top-down for llnn and llnu, bottom-up for lltn and
+// lunn): row j's values are scaled by the reciprocal diagonal and broadcast with
+// v_readlane, and every row still to be solved drops its multiple of them.  No
+// barriers.  The elements of A are loaded four columns at a time (a 128-byte line
+// holds four columns of a panel's rows for ps = 4), the next four while the
+// current ones are applied.
+// Measured (MI355X, 4 right-hand sides; before: a column at a time): 8192 LU solves
+// (factorisation included) of U{16..256} 3922 -> 3829 us, of U{16..64} 355 -> 326.
 // ---------------------------------------------------------------------------
 constexpr int THIN_RHS = 4;
 constexpr int THIN_Q = 4;
 
 template <typename T, int PS, int MODE>
-__device__ __forceinline__ void thin_coef(const PM<T, PS> gA, int ai, int aj, int m, int j, T (&e)[THIN_Q])
-{
-	constexpr bool BACK = tl_back(MODE);
-	const int lane = threadIdx.x & (WAVE - 1);
-#pragma unroll
-	for (int q = 0; q < THIN_Q; q++)
-	{
-		const int i = lane + q * WAVE;
-		T v = T(0);
-		if (BACK ? (i < j) : (i > j && i < m))
-			v = MODE == TL_LLTN ? gA.at(ai + j, aj + i) : gA.at(ai + i, aj + j);
-		e[q] = v;
-	}
-}
-
-template <typename T, int PS, int MODE>
-__global__ __launch_bounds__(WAVE) void k_trsm_left_thin(const typename TrsmArg<T>::type *__restrict__ args)
+__global__ __launch_bounds__(WAVE, 4) void k_trsm_left_thin(const typename TrsmArg<T>::type *__restrict__ args)
 {
 	constexpr bool BACK = tl_back(MODE);
 	constexpr bool UNIT = MODE == TL_LLNU;
+	constexpr unsigned CS = StripView<T, PS>::CS;
 	const typename TrsmArg<T>::type &a = args[blockIdx.x];
-	const int m = a.m;
-	if (m <= 0 || a.n <= 0 || m > THIN_Q * WAVE)
+	const int m = __builtin_amdgcn_readfirstlane(a.m), nrhs = __builtin_amdgcn_readfirstlane(a.n);
+	if (m <= 0 || nrhs <= 0 || m > THIN_Q * WAVE)
 		return;
-	const PM<T, PS> gA = view_flat<T, PS>(a.sA);
-	const PM<T, PS> gB = view_flat<T, PS>(a.sB);
-	PM<T, PS> gD = view_flat<T, PS>(a.sD);
+	const StripView<T, PS> A = strip_view<T, PS>(a.sA), B = strip_view<T, PS>(a.sB), D = strip_view<T, PS>(a.sD);
 	const int ai = a.ai, aj = a.aj;
 	const int lane = threadIdx.x;
 	const bool cached = !UNIT && ai == 0 && aj == 0 && a.sD != a.sA && a.sA->use_dA >= m;
-	const T *dA = a.sA->dA;
-	// right-hand sides in groups of THIN_RHS (one group when n <= 4)
-	for (int c0 = 0; c0 < a.n; c0 += THIN_RHS)
-	{
-	const int n = min(THIN_RHS, a.n - c0);
-	T x[THIN_Q][THIN_RHS];
+	const BFA_GLOBAL T *dA = (const BFA_GLOBAL T *)a.sA->dA;
+	// this lane's rows of A (lltn: columns; rows past the end read the last one)
+	// and their reciprocal diagonals
+	unsigned oa[THIN_Q];
+	T rd[THIN_Q];
 #pragma unroll
 	for (int q = 0; q < THIN_Q; q++)
-#pragma unroll
-		for (int c = 0; c < THIN_RHS; c++)
+		if (q * WAVE < m)
 		{
-			const int i = lane + q * WAVE;
-			x[q][c] = (i < m && c < n) ? a.alpha * gB.at(a.bi + i, a.bj + c0 + c) : T(0);
+			const int i = min(lane + q * WAVE, m - 1);
+			oa[q] = MODE == TL_LLTN ? (unsigned)(aj + i) * CS : A.at(ai + i, aj);
+			rd[q] = UNIT ? T(1) : cached ? dA[i] : T(1) / A.ld(0, A.at(ai + i, aj + i));
 		}
-	T e[THIN_Q];
-	thin_coef<T, PS, MODE>(gA, ai, aj, m, BACK ? m - 1 : 0, e);
-	// the reciprocal diagonal of column j, also loaded one column ahead
-	auto recip = [&](int jj) -> T {
-		return UNIT ? T(1) : (cached ? dA[jj] : T(1) / gA.at(ai + jj, aj + jj));
-	};
-	T d = recip(BACK ? m - 1 : 0);
-	// the solve's columns j in order, grouped by the register slot qb = j / 64
-	// that holds row j (unrolled, so every register index is a constant)
+	// columns j0 .. j0+3 of the solve, slots q0 .. q1-1
+	auto coef = [&](int j0, int q0, int q1, T (&e)[THIN_Q][4]) {
 #pragma unroll
-	for (int qq = 0; qq < THIN_Q; qq++)
+		for (int q = 0; q < THIN_Q; q++)
+			if (q >= q0 && q < q1 && q * WAVE < m)
+#pragma unroll
+				for (int t = 0; t < 4; t++)
+				{
+					const int j = max(0, min(j0 + t, m - 1));
+					e[q][t] = A.ld(MODE == TL_LLTN ? A.at(ai + j, 0) : (unsigned)j * CS, oa[q]);
+				}
+	};
+	// right-hand sides in groups of THIN_RHS (one group when n <= 4)
+	for (int c0 = 0; c0 < nrhs; c0 += THIN_RHS)
 	{
-		const int qb = BACK ? THIN_Q - 1 - qq : qq;
-		for (int ll = 0; ll < WAVE; ll++)
-		{
-			const int lj = BACK ? WAVE - 1 - ll : ll;
-			const int j = qb * WAVE + lj;
-			if (j >= m)
-			{
-				if (BACK)
-					continue;
-				break;
-			}
-			const int jn = BACK ? j - 1 : j + 1;          // the next column
-			const bool more = BACK ? jn >= 0 : jn < m;
-			T en[THIN_Q];
-			T dn = T(1);
-			if (more)
-			{
-				thin_coef<T, PS, MODE>(gA, ai, aj, m, jn, en);
-				dn = recip(jn);
-			}
-			T xj[THIN_RHS];
+		const int n = min(THIN_RHS, nrhs - c0);
+		T x[THIN_Q][THIN_RHS];
+#pragma unroll
+		for (int q = 0; q < THIN_Q; q++)
 #pragma unroll
 			for (int c = 0; c < THIN_RHS; c++)
-				xj[c] = readlane(x[qb][c], lj) * d;
-#pragma unroll
-			for (int q = 0; q < THIN_Q; q++)
 			{
-				// slots whose rows are all solved already (before qb on the way
-				// down, after it on the way up) or all past m are left alone
-				if (BACK ? q > qb : q < qb)
-					continue;
-				if (q * WAVE >= m)
-					continue;
 				const int i = lane + q * WAVE;
-				// only the rows still to be solved take the update (a solved
-				// row is never touched again, so an Inf or NaN in xj cannot
-				// reach it through a zero coefficient); row j itself keeps its
-				// unscaled value, scaled by its reciprocal after the sweep
-				const bool open = BACK ? i < j : i > j;
-#pragma unroll
-				for (int c = 0; c < THIN_RHS; c++)
-					x[q][c] = open ? x[q][c] - e[q] * xj[c] : x[q][c];
+				x[q][c] = (i < m && c < n) ? a.alpha * B.ld(0, B.at(a.bi + i, a.bj + c0 + c)) : T(0);
 			}
-			if (more)
+		T e[THIN_Q][4];
+		coef(BACK ? (m - 1) & ~3 : 0, 0, THIN_Q, e);
+		// grouped by the register slot qb = j / 64 that holds row j (unrolled, so
+		// that every register index is a constant)
+#pragma unroll
+		for (int qq = 0; qq < THIN_Q; qq++)
+		{
+			const int qb = BACK ? THIN_Q - 1 - qq : qq;
+#pragma unroll 1
+			for (int l4 = 0; l4 < WAVE; l4 += 4)
 			{
+				const int lb = BACK ? WAVE - 4 - l4 : l4;   // first lane of the group
+				const int j0 = qb * WAVE + lb;
+				if (j0 >= m)
+				{
+					if (BACK)
+						continue;
+					break;
+				}
+				T en[THIN_Q][4];
+				if (BACK ? j0 > 0 : j0 + 4 < m)
+					coef(BACK ? j0 - 4 : j0 + 4, BACK ? 0 : qb, BACK ? qb + 1 : THIN_Q, en);
+#pragma unroll
+				for (int tt = 0; tt < 4; tt++)
+				{
+					const int t = BACK ? 3 - tt : tt;
+					const int j = j0 + t;
+					if (j < m)
+					{
+						const T d = UNIT ? T(1) : readlane(rd[qb], lb + t);
+						T xj[THIN_RHS];
+#pragma unroll
+						for (int c = 0; c < THIN_RHS; c++)
+							xj[c] = readlane(x[qb][c], lb + t) * d;
+						// only the rows still to be solved take the update (a
+						// solved row is never touched again, so an Inf or NaN in
+						// xj cannot reach it); row j itself keeps its unscaled
+						// value, scaled by its reciprocal after the sweep
+						const bool open = BACK ? lane < lb + t : lane > lb + t;
+#pragma unroll
+						for (int q = 0; q < THIN_Q; q++)
+						{
+							if (BACK ? q > qb : q < qb)
+								continue;
+							if (q * WAVE >= m)
+								continue;
+#pragma unroll
+							for (int c = 0; c < THIN_RHS; c++)
+							{
+								const T y = x[q][c] - e[q][t] * xj[c];
+								x[q][c] = q != qb || open ? y : x[q][c];
+							}
+						}
+					}
+				}
 #pragma unroll
 				for (int q = 0; q < THIN_Q; q++)
-					e[q] = en[q];
-				d = dn;
+#pragma unroll
+					for (int t = 0; t < 4; t++)
+						e[q][t] = en[q][t];
 			}
 		}
-	}
-	// row i's solved value is its unscaled value times the reciprocal the
-	// sweep used for column i (the same product the broadcast formed)
+		// row i's solved value is its unscaled value times the reciprocal the
+		// sweep used for column i (the same product the broadcast formed)
 #pragma unroll
-	for (int q = 0; q < THIN_Q; q++)
-	{
-		const int i = lane + q * WAVE;
-		if (i < m)
+		for (int q = 0; q < THIN_Q; q++)
 		{
-			const T di = recip(i);
+			const int i = lane + q * WAVE;
+			if (i < m)
 #pragma unroll
-			for (int c = 0; c < THIN_RHS; c++)
-				if (c < n)
-					gD.at(a.di + i, a.dj + c0 + c) = UNIT ? x[q][c] : x[q][c] * di;
+				for (int c = 0; c < THIN_RHS; c++)
+					if (c < n)
+						D.st(0, D.at(a.di + i, a.dj + c0 + c), UNIT ? x[q][c] : x[q][c] * rd[q]);
 		}
-	}
 	}
 }
 
@@ -595,15 +601,16 @@ static int launch_trsml(int ps, int batch, const typename TrsmArg<T>::type *args
 	const int gy = hint->max_n > 0 ? min(64, (hint->max_n + LNC - 1) / LNC) : 1;
 	dim3 grid(batch, gy);
 	// few right-hand sides (hint->max_n <= 4), m <= 256 and a batch that fills
-	// the GPU by itself (16 instances per CU): one wavefront per instance with X
+	// the GPU by itself (8 instances per CU): one wavefront per instance with X
 	// in registers.  Smaller batches keep the four-wave block sweep, whose
-	// per-instance chain is shorter (2048 solves of n = 256 with 4 right-hand
-	// sides: 1.34 ms against 1.48 ms one wavefront each).
+	// per-instance chain is shorter (SPD solves, factorisation included, 4
+	// right-hand sides: 2048 of 256 1037 us with one wavefront against 1066, 512 of
+	// 256 389 against 357, 1000 of U{100..200} 332 against 300).
 	// The "trsm_thin" knob forces it on (1) or off (2) where it applies.
 	const int cus = num_cus() > 0 ? num_cus() : 256;
 	const int knob = tune_value(TUNE_TRSM_THIN, 0);
 	const bool thin = sizeof(T) == 8 && hint->max_n > 0 && hint->max_n <= THIN_RHS && mmax <= THIN_Q * WAVE
-	                  && (knob == 1 || (knob == 0 && batch >= 16 * cus));
+	                  && (knob == 1 || (knob == 0 && batch >= 8 * cus));
 	if (ps == 4)
 		return launch_trsml_ps<T, 4, MODE>(batch, args, grid, shm, mmax, thin, st, name);
 	if (ps == 8)

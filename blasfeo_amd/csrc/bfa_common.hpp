@@ -167,18 +167,6 @@ __device__ __forceinline__ PM<T, PS> view(const typename MatOf<T>::type *s)
 	return v;
 }
 
-// The same with the descriptor read through the generic pointer, for the
-// one-wavefront left solve: there the global form was slower (16384 LU
-// solves, two such launches: 1.31 -> 1.40 ms).
-template <typename T, int PS>
-__device__ __forceinline__ PM<T, PS> view_flat(const typename MatOf<T>::type *s)
-{
-	PM<T, PS> v;
-	v.p = s->pA;
-	v.cn = s->cn;
-	return v;
-}
-
 // Walks the elements of the R x C block at absolute (r0, c0) of a panel-major
 // matrix that this thread copies: the waves take the covering panels in turn
 // and the lanes of a wave walk one panel's contiguous run of C*PS elements, so

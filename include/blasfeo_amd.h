@@ -142,7 +142,7 @@ const char *blasfeo_amd_last_error(void);
  *   "trsm_thin",   index 0: left-side solves (llnn, lltn, llnu, lunn) with
  *                  hint->max_n <= 4 and m <= 256 on one wavefront per instance:
  *                  1 always, 2 never; built-in: when the batch has at least
- *                  16 instances per CU;
+ *                  8 instances per CU;
  *   "gemm_wave",   index 0: output tile of gemm_nt/nn and syrk_ln(_mn): 32 x 32
  *                  (1) or 64 x 64 (2); built-in: by the hint's bounds and the
  *                  batch (large bounds and many tiles: 64 x 64);
