@@ -11,7 +11,11 @@ nx = 64, every matrix and every vector in its own exactly-sized block:
             solve, the FP64 refinement): ux and pi against the oracle's
             d_back_ric_trf + d_back_ric_trs, and every instance's backward
             error at or below the tolerance.
-Usage: python case_ric.py sv|trf|mixed <ps>"""
+  trs <ps>  blasfeo_amd_d_back_ric_trs_batched on the oracle's factors, stages of at
+            most 32 rows (the form of small stages), without and with valid
+            reciprocals, one instance beyond the bound given: ux, pi, Pb, the
+            reciprocals and their flags.
+Usage: python case_ric.py sv|trf|mixed|trs <ps>"""
 import ctypes
 import sys
 
@@ -180,6 +184,56 @@ def vec_blocks(rs, buf):
     return blocks, tab
 
 
+def run_trs(ps):
+    from blasfeo_amd.riccati import HostRiccati, RiccatiSolve
+    E = emu_lib("emu_lapack")
+    for N, nxs, nus, bound in ((4, [1, 3, 8, 8, 17, 31, 24, 12, 32, 20], [0, 2, 3, 5, 15, 1, 6, 0, 0, 12], 32),
+                               (1, [5, 12], [2, 0], 12), (0, [6], [2], 8), (3, [8, 9, 4], [3, 3, 2], 11)):
+        rb = RiccatiBatch(nxs, nus, N=N, ps=ps)
+        rs = RiccatiSolve(rb)
+        rng = np.random.default_rng(980 + ps + N)
+        inp, sin = rb.fill_inputs(rng), rs.fill_inputs(rng)
+        for valid in (0, 1):
+            host = HostRiccati(rb, inp)
+            oracle.lib().or_dric_trf_batch(ps, rb.batch, host.argv.ctypes.data)
+            hb, hr, hL, hw, hnx, hnu = host.t
+            hL["use_dA"] = valid
+            in_blocks, fix_in = split(rb.inp, inp, ("mem", "pA", "dA"))
+            out_blocks, fix_out = split(rb.out, host.outbuf, ("mem", "pA", "dA"))
+            babt, rsq, L, work, nx, nu = rb.tables(0, 0)
+            fix_in(babt), fix_out(L)
+            L["use_dA"] = valid
+            vblocks, vtab = vec_blocks(rs, sin)
+            tbl = {k: Block(v.nbytes) for k, v in (("babt", babt), ("L", L), ("nx", nx), ("nu", nu), ("v", vtab))}
+            for k, v in (("babt", babt), ("L", L), ("nx", nx), ("nu", nu), ("v", vtab)):
+                tbl[k].write(v)
+            a = rs.args(tbl["v"].addr, tbl["babt"].addr, tbl["L"].addr, tbl["nx"].addr, tbl["nu"].addr)
+            ablk = Block(a.nbytes)
+            ablk.write(a)
+            print("emu d_back_ric_trs ps=%d batch=%d N=%d bound=%d use_dA=%d" % (ps, rb.batch, N, bound, valid), flush=True)
+            rc = E.blasfeo_amd_d_back_ric_trs_batched(ps, rb.batch, ctypes.c_void_p(ablk.addr),
+                                                      ctypes.byref(HINT(bound, 1, 0)), None)
+            assert rc == 0, E.emu_last_error()
+            hsol = sin.copy()
+            htab = rs.table(hsol.ctypes.data)
+            targs = rs.args(htab.ctypes.data, hb.ctypes.data, hL.ctypes.data, hnx.ctypes.data, hnu.ctypes.data)
+            oracle.lib().or_dric_trs_batch(ps, rb.batch, targs.ctypes.data)
+            Lout = tbl["L"].read(bfa.DMAT)
+            assert (Lout["use_dA"] == hL["use_dA"]).all(), (Lout["use_dA"], hL["use_dA"])
+            for i in range(rb.batch):
+                for kind, ks in (("ux", range(N + 1)), ("pi", range(N)), ("Pb", range(N))):
+                    for k in ks:
+                        j = rs.index(i, kind, k)
+                        compare(vblocks[j].read(np.float64, int(rs.sizes[j])), rs.vec(hsol, i, kind, k), 1e-11,
+                                "%s[%d] instance %d" % (kind, k, i))
+                for k in range(N + 1):
+                    j = rb.i_L[i][k]
+                    m, n, pm, cn = rb.out.geom(j)
+                    want = np.frombuffer(host.outbuf[rb.out.offsets[j]: rb.out.offsets[j] + out_blocks[j].nbytes], np.float64)
+                    compare(out_blocks[j].read(np.float64)[pm * cn: pm * cn + n], want[pm * cn: pm * cn + n], 1e-11, "dA[%d] instance %d" % (k, i))
+    print("ok", flush=True)
+
+
 def run_mixed(ps):
     from blasfeo_amd.riccati import HostRiccati, RiccatiSolve
     nxs = NXS + [2, 12]
@@ -266,4 +320,4 @@ def run_mixed_once(E, ps, rb, rs, N, ablk, info, tol, rule, vblocks, inp, sin):
 
 
 if __name__ == "__main__":
-    {"sv": run, "trf": run_trf, "mixed": run_mixed}[sys.argv[1]](int(sys.argv[2]))
+    {"sv": run, "trf": run_trf, "mixed": run_mixed, "trs": run_trs}[sys.argv[1]](int(sys.argv[2]))

@@ -132,6 +132,13 @@ def test_riccati_trf(emu_build, ps):
 
 
 @pytest.mark.parametrize("ps", [4, 8])
+def test_riccati_trs(emu_build, ps):
+    """The Riccati solve of stages of at most 32 rows: N = 0, 1, 3 and 4, no inputs,
+    reciprocals valid or not, an instance beyond the bound."""
+    run_case("case_ric.py", "trs", ps)
+
+
+@pytest.mark.parametrize("ps", [4, 8])
 def test_riccati_sv(emu_build, ps):
     """The fused Riccati factorisation and solve over every LDS footprint class
     up to nu+nx = 127, nx = 64, each matrix and vector in its own block."""
