@@ -266,7 +266,7 @@ def run_riccati(args, torch, bfa):
         log("checked %d instances: stage backward error <= %.2f n eps, L_0 rel diff vs oracle %.1e"
             % (nchk, berr, fdiff))
 
-    traffic = read_traffic("k_ric_class", "riccati-%dx%d" % (args.batch, args.horizon))
+    traffic = read_traffic("k_ric_coop", "riccati-%dx%d" % (args.batch, args.horizon))
     rbound, rach, rpeak, runit = roof(flops, algo_bytes, ms, FP64_PEAK_TFLOPS)
     out = {
         "metric": METRIC,
@@ -1051,9 +1051,8 @@ def run_blas3_extra(args, torch, bfa):
         flops = float((mf ** 3 / 3).sum())
         algo = float((8 * (mf * (mf + 1) + mf)).sum())
         unit = "factorizations/s (dpotrf_l calls)"
-        kernel = ("k_potrf_lds_q<double,%d,64|256,false> (one persistent launch per 16-row bucket, "
-                  "packed lower tiles in LDS sized for the bucket)" % ps)
-        traffic = read_traffic("k_potrf_lds", "potrf-var-65536")
+        kernel = "k_potrf_wave<double,%d,8> (one wave per instance, 16-row strips in registers)" % ps
+        traffic = read_traffic("k_potrf_wave", "potrf-var-65536")
         cfg = {"workload": "dpotrf_l_batched", "batch": batch, "n": "U{8..128}"}
     else:
         base = bufs["C"].data_ptr()
@@ -1068,9 +1067,8 @@ def run_blas3_extra(args, torch, bfa):
         flops = float((mf * (mf + 1) * kf + mf ** 3 / 3).sum())
         algo = float((8 * (mf * kf + mf * (mf + 1) + mf)).sum())
         unit = "factorizations/s (dsyrk_dpotrf_ln calls)"
-        kernel = ("k_syrk_potrf_lds_q<double,%d,64|256> (one persistent launch per 16-row "
-                  "bucket, packed lower tiles in LDS sized for the bucket)" % ps)
-        traffic = read_traffic("k_syrk_potrf_lds", "syrk-potrf-65536")
+        kernel = "k_syrk_potrf_coop<double,%d> (16-row strips in registers, shared by the waves)" % ps
+        traffic = read_traffic("k_syrk_potrf_coop", "syrk-potrf-65536")
         cfg = {"workload": "dsyrk_dpotrf_ln_batched", "batch": batch, "m,k": "U{8..128}"}
     drec = to_device(rec)
     fn = lambda: bfa.call(call, ps, batch, drec.data_ptr(), hint, sh)
@@ -1183,8 +1181,8 @@ def run_other(args, torch, bfa):
         value = batch / (ms * 1e-3)
         unit = "factorizations/s"
         bound, achieved, peak, punit = roof(flops, algo, ms, FP64_PEAK_TFLOPS)
-        traffic = read_traffic("k_potrf_lds", "potrf-4096x32")
-        kernel = "k_potrf_lds<double,%d,64>" % ps
+        traffic = read_traffic("k_potrf_wave", "potrf-4096x32")
+        kernel = "k_potrf_wave<double,%d,2>" % ps
         wl = {"workload": "dpotrf_l_batched", "batch": batch, "n": n, "ps": ps, "precision": "fp64"}
         # check: backward error of every factor
         L = bufD.view(torch.float64).view(batch, stride)[:, : pm * n].view(batch, pm // ps, n, ps)
@@ -1300,8 +1298,8 @@ def run_other(args, torch, bfa):
         value = batch / (ms * 1e-3)
         unit = "factorizations/s"
         bound, achieved, peak, punit = roof(flops, algo, ms, FP64_PEAK_TFLOPS if prec == "d" else 157.3)
-        traffic = read_traffic("k_getrf", "getrf-16384") if args.workload == "getrf" else None
-        kernel = "k_getrf<%s,%d%s>" % ("double" if prec == "d" else "float", ps,
+        traffic = read_traffic("k_getrf_wg", "getrf-16384") if args.workload == "getrf" else None
+        kernel = "k_getrf_wg<%s,%d%s>" % ("double" if prec == "d" else "float", ps,
                                        ",PIV=false" if args.workload == "getrf_np" else "")
         if args.workload == "getrf_np":
             # the first 64 factors against the oracle's getrf_np on the same blocks

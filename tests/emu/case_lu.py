@@ -1,6 +1,7 @@
 """Emulator cases (TEST INFRASTRUCTURE ONLY) for the LU factorisations on the record
 sets of tests/lu_cases.py, checked against the oracle: pivots exactly, factors at
 the reference's rule, NaN and Inf included.
+The instances of more than half the bound (all of them for 64).
 Usage: python case_lu.py <getrf_rp | getrf_np> <ps> <bound of the rows>"""
 import ctypes
 import sys
@@ -13,7 +14,7 @@ import lu_cases
 
 def run(op, ps, bound):
     E = emu_lib("emu_lapack")
-    re, ro = to_mats(ps, [c for c in lu_cases.lu(ps, 60 + ps, op == "getrf_rp") if c[1]["m"] <= bound])
+    re, ro = to_mats(ps, [c for c in lu_cases.lu(ps, 60 + ps, op == "getrf_rp") if bound // 2 * (bound > 64) < c[1]["m"] <= bound])
     piv = [[Block(4 * min(r["m"], r["n"])) for r in s] for s in (re, ro)]
     for s, p in zip((re, ro), piv):
         for r, b in zip(s, p):

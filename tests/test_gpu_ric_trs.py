@@ -81,6 +81,35 @@ def test_riccati_trs_parity(gpu, ps, N):
             np.testing.assert_array_equal(rs.vec(gbuf, i, "rq", k), rs.vec(sin, i, "rq", k))
 
 
+@pytest.mark.parametrize("valid", [1, 0])
+@pytest.mark.parametrize("most", [16, 32])
+@pytest.mark.parametrize("ps,N", [(4, 7), (8, 1)])
+def test_riccati_trs_small(gpu, ps, N, most, valid):
+    """Stages of at most 16 and 32 rows, on LDS copies: the largest and the smallest
+    sizes, no inputs, with valid reciprocals and without."""
+    import torch
+    rng = np.random.default_rng(710 + ps + most)
+    nxs = [most, most - 1, 1, 2, most // 2 + 1, most - 5, 8, 3]
+    nus = [0, 1, most - 1, 0, most // 2 - 1, 5, 3, 2]
+    rb = RiccatiBatch(nxs, nus, N=N, ps=ps)
+    inp = rb.fill_inputs(rng)
+    dev = DeviceRiccati(rb, inp)
+    dev.run()
+    torch.cuda.synchronize()
+    Ltab = dev.t_dev[2]
+    Lh = Ltab.cpu().numpy().view(DMAT).copy()
+    Lh["use_dA"] = valid
+    Ltab.copy_(torch.from_numpy(Lh.view(np.uint8).reshape(Ltab.shape)))
+    rs = RiccatiSolve(rb)
+    sin = rs.fill_inputs(rng)
+    ds = DeviceRiccatiSolve(dev, rs, sin)
+    ds.run()
+    torch.cuda.synchronize()
+    rbuf, L, _ = _oracle_on_gpu_factors(rb, inp, dev, rs, sin, use_dA=valid)
+    _compare(rb, rs, ds.host(), rbuf)
+    np.testing.assert_array_equal(Ltab.cpu().numpy().view(DMAT)["use_dA"].reshape(-1), L["use_dA"].reshape(-1))
+
+
 def test_riccati_trs_forms_reciprocals(gpu):
     """use_dA = 0 in every factor's descriptor and NaN in dA: the solve forms
     1/L(j,j) for the columns its trsv uses (nu[k] on stages k >= 1, all on
