@@ -562,15 +562,19 @@ static int launch_potrf(int ps, int batch, const typename FactArg<T>::type *args
 		// sizes up to 128 are bounded to whole strips
 		if (mmax <= 128)
 			mmax = (mmax + 15) / 16 * 16;
-		// One wave per instance once the batch gives every CU more than two
-		// instances, NW waves per instance below: n = 64, 128 and 256 in batches
-		// of 256 take 16, 59 and 311 us against 14, 41 and 114 us, in batches of
-		// 8192 88, 489 and 2715 us against 106, 597 and 3431 us (MI355X; they
-		// cross between 512 and 1000 instances).  The "potrf_bw" knob forces the
-		// first (1) or the second (2, 4).
+		// One wave per instance once the batch gives every CU more than three
+		// instances (four up to 64 columns, two in FP32 above), NW waves per
+		// instance below: n = 64, 128 and 256 in batches of 256 take 16, 59 and 311 us
+		// against 14, 41 and 114 us, in batches of 8192 88, 489 and 2715 us against
+		// 106, 597 and 3431 us (MI355X); at 558 instances of 128, 256 and U{199..245}
+		// 65, 354 and 334 us against 54, 315 and 266, at 1024 of the first two 72 and
+		// 419 against 86 and 447; of 64 at 1024 17.8 against 17.5; FP32 of 128 at 558
+		// 56 and 56, at 1024 61 and 74.  The "potrf_bw" knob forces the first (1) or
+		// the second (2, 4).
 		const int cus = num_cus() > 0 ? num_cus() : 256;
 		const int knob = tune_value(TUNE_POTRF_BW, 0);
-		const bool wave = knob == 1 || (knob == 0 && batch > 2 * cus);
+		const int few = mmax <= 64 ? 4 : sizeof(T) == 8 ? 3 : 2;
+		const bool wave = knob == 1 || (knob == 0 && batch > few * cus);
 #define BFA_POTRF(PS_, NB_, NW_)                                                                                           \
 	do                                                                                                                     \
 	{                                                                                                                      \

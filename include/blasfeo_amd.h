@@ -138,7 +138,7 @@ const char *blasfeo_amd_last_error(void);
  *   "gemm_grid_y", index 0: most workgroups per gemm/syrk/trmm instance (1..64);
  *   "potrf_bw",    index 0: potrf_l(_mn) up to 256 columns with one wave per
  *                  instance (1) or with several (2, 4); built-in: one when the
- *                  batch gives every CU more than two instances;
+ *                  batch gives every CU more than two to four instances;
  *   "trsm_thin",   index 0: left-side solves (llnn, lltn, llnu, lunn) with
  *                  hint->max_n <= 4 and m <= 256 on one wavefront per instance:
  *                  1 always, 2 never; built-in: when the batch has at least
