@@ -224,31 +224,28 @@ __global__ __launch_bounds__(NT3) void k_trsm_left(const typename TrsmArg<T>::ty
 constexpr int THIN_RHS = 4;
 constexpr int THIN_Q = 4;
 
-template <typename T, int PS, int MODE>
-__global__ __launch_bounds__(WAVE, 4) void k_trsm_left_thin(const typename TrsmArg<T>::type *__restrict__ args)
+template <typename T, int PS, int MODE, typename O>
+__device__ __forceinline__ void trsm_thin(const typename TrsmArg<T>::type &a, int m, int nrhs, const StripView<T, PS> &vA,
+	const StripView<T, PS> &vB, const StripView<T, PS> &vD)
 {
 	constexpr bool BACK = tl_back(MODE);
 	constexpr bool UNIT = MODE == TL_LLNU;
-	constexpr unsigned CS = StripView<T, PS>::CS;
-	const typename TrsmArg<T>::type &a = args[blockIdx.x];
-	const int m = __builtin_amdgcn_readfirstlane(a.m), nrhs = __builtin_amdgcn_readfirstlane(a.n);
-	if (m <= 0 || nrhs <= 0 || m > THIN_Q * WAVE)
-		return;
-	const StripView<T, PS> A = strip_view<T, PS>(a.sA), B = strip_view<T, PS>(a.sB), D = strip_view<T, PS>(a.sD);
-	const int ai = a.ai, aj = a.aj;
+	constexpr unsigned CS = PS * sizeof(T);
+	int ai = a.ai, aj = a.aj, bi = a.bi, bj = a.bj, di = a.di, dj = a.dj;
+	const StripView<T, PS, O> A = vA.template block<O>(ai, aj), B = vB.template block<O>(bi, bj), D = vD.template block<O>(di, dj);
 	const int lane = threadIdx.x;
-	const bool cached = !UNIT && ai == 0 && aj == 0 && a.sD != a.sA && a.sA->use_dA >= m;
+	const bool cached = !UNIT && a.ai == 0 && a.aj == 0 && a.sD != a.sA && a.sA->use_dA >= m;
 	const BFA_GLOBAL T *dA = (const BFA_GLOBAL T *)a.sA->dA;
 	// this lane's rows of A (lltn: columns; rows past the end read the last one)
 	// and their reciprocal diagonals
-	unsigned oa[THIN_Q];
+	O oa[THIN_Q];
 	T rd[THIN_Q];
 #pragma unroll
 	for (int q = 0; q < THIN_Q; q++)
 		if (q * WAVE < m)
 		{
 			const int i = min(lane + q * WAVE, m - 1);
-			oa[q] = MODE == TL_LLTN ? (unsigned)(aj + i) * CS : A.at(ai + i, aj);
+			oa[q] = MODE == TL_LLTN ? (O)(aj + i) * CS : A.at(ai + i, aj);
 			rd[q] = UNIT ? T(1) : cached ? dA[i] : T(1) / A.ld(0, A.at(ai + i, aj + i));
 		}
 	// columns j0 .. j0+3 of the solve, slots q0 .. q1-1
@@ -260,7 +257,7 @@ __global__ __launch_bounds__(WAVE, 4) void k_trsm_left_thin(const typename TrsmA
 				for (int t = 0; t < 4; t++)
 				{
 					const int j = max(0, min(j0 + t, m - 1));
-					e[q][t] = A.ld(MODE == TL_LLTN ? A.at(ai + j, 0) : (unsigned)j * CS, oa[q]);
+					e[q][t] = A.ld(MODE == TL_LLTN ? A.at(ai + j, 0) : (O)j * CS, oa[q]);
 				}
 	};
 	// right-hand sides in groups of THIN_RHS (one group when n <= 4)
@@ -274,7 +271,7 @@ __global__ __launch_bounds__(WAVE, 4) void k_trsm_left_thin(const typename TrsmA
 			for (int c = 0; c < THIN_RHS; c++)
 			{
 				const int i = lane + q * WAVE;
-				x[q][c] = (i < m && c < n) ? a.alpha * B.ld(0, B.at(a.bi + i, a.bj + c0 + c)) : T(0);
+				x[q][c] = (i < m && c < n) ? a.alpha * B.ld(0, B.at(bi + i, bj + c0 + c)) : T(0);
 			}
 		T e[THIN_Q][4];
 		coef(BACK ? (m - 1) & ~3 : 0, 0, THIN_Q, e);
@@ -348,9 +345,23 @@ __global__ __launch_bounds__(WAVE, 4) void k_trsm_left_thin(const typename TrsmA
 #pragma unroll
 				for (int c = 0; c < THIN_RHS; c++)
 					if (c < n)
-						D.st(0, D.at(a.di + i, a.dj + c0 + c), UNIT ? x[q][c] : x[q][c] * rd[q]);
+						D.st(0, D.at(di + i, dj + c0 + c), UNIT ? x[q][c] : x[q][c] * rd[q]);
 		}
 	}
+}
+
+template <typename T, int PS, int MODE>
+__global__ __launch_bounds__(WAVE, 4) void k_trsm_left_thin(const typename TrsmArg<T>::type *__restrict__ args)
+{
+	const typename TrsmArg<T>::type &a = args[blockIdx.x];
+	const int m = __builtin_amdgcn_readfirstlane(a.m), nrhs = __builtin_amdgcn_readfirstlane(a.n);
+	if (m <= 0 || nrhs <= 0 || m > THIN_Q * WAVE)
+		return;
+	const StripView<T, PS> A = strip_view<T, PS>(a.sA), B = strip_view<T, PS>(a.sB), D = strip_view<T, PS>(a.sD);
+	if (__builtin_expect(strip_fits<T, PS>(max(A.cn, max(B.cn, D.cn))), 1))
+		trsm_thin<T, PS, MODE, unsigned>(a, m, nrhs, A, B, D);
+	else
+		trsm_thin<T, PS, MODE, size_t>(a, m, nrhs, A, B, D);
 }
 
 // Cache update after trsm_rltn / trsm_llnn / trsm_lltn, in the reference's

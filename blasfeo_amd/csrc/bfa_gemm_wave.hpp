@@ -24,6 +24,7 @@
 #pragma once
 #include "bfa_gemm_core.hpp"
 #include "bfa_strip.hpp"
+#include <type_traits>
 
 namespace bfa {
 
@@ -76,32 +77,38 @@ __device__ __forceinline__ T vec_get(const typename VecN<T, N>::type &v, int e)
 // between 2 and 6 steps and 2 and 6 waves nothing but the least (2 steps of the
 // large tile) was more than a few per cent apart.
 template <typename T, int E> constexpr int gw_depth() { return E == 4 ? 3 : 4; }
-template <typename T, int E> constexpr int gw_waves() { return E == 4 ? (sizeof(T) == 8 ? 2 : 3) : 4; }
+template <typename T, int E> constexpr int gw_waves() { return E == 4 ? (sizeof(T) == 8 ? 2 : 4) : sizeof(T) == 8 ? 5 : 8; }
 // rows that a lane takes at a time in a tile of MX 16-row groups
 template <typename T, int MX> constexpr int gw_rows() { return MX == 4 && sizeof(T) == 4 ? 4 : 2; }
 
-template <typename T, int PS>
+// A tile and what is right of and below it: m rows, n columns; the views start at the
+// tile (B's of gemm_nn at its columns), low is how far it lies below the diagonal.
+template <typename T, int PS, typename O>
 struct GwArg
 {
-	StripView<T, PS> A, B, C, D;
-	int ai, aj, bi, bj, ci, cj, di, dj, m, n, k;
+	StripView<T, PS, O> A, B, C, D;
+	int ai, aj, bi, bj, ci, cj, di, dj, m, n, k, low;
 	T alpha, beta;
 };
 
-// One tile of MX 16-row groups and NY 16-column blocks at (i0, j0); VA: rows that a
-// lane takes at a time (1: any offsets).
-template <typename T, int PS, int OP, int MX, int NY, int VA, int DEPTH>
-__device__ __forceinline__ void gw_body(const GwArg<T, PS> &a, int i0, int j0)
+// The tile's MX 16-row groups and NY 16-column blocks; VA: rows that a lane takes at a
+// time (1: any offsets).
+template <typename T, int PS, int OP, int MX, int NY, int VA, int DEPTH, typename O>
+__device__ __forceinline__ void gw_body(const GwArg<T, PS, O> &a)
 {
 	typedef typename Vec4<T>::type V4;
 	typedef typename VecN<T, VA>::type VV;
 	constexpr int NV = MX / VA;
-	constexpr unsigned CS = StripView<T, PS>::CS;
+	constexpr unsigned CS = PS * sizeof(T);
 	constexpr bool SY = OP == OP_SYRK || OP == OP_SYRK_MN;
-	const int lane = lane_id(), g = lane >> 4, c = lane & 15;
+	// (pinned: the columns and rows of the lane's elements, the same for every tile, would
+	// be kept in registers across the tiles)
+	int lane = lane_id();
+	BFA_PIN(lane);
+	const int g = lane >> 4, c = lane & 15;
 	const int m = a.m, n = a.n, k = a.k;
 	const int lastv = (m - 1) & ~(VA - 1);
-	auto ldv = [](const StripView<T, PS> &v, unsigned o) -> VV { return *(const BFA_GLOBAL VV *)(v.p + o); };
+	auto ldv = [](const StripView<T, PS, O> &v, O o) -> VV { return *(const BFA_GLOBAL VV *)(v.p + o); };
 	V4 acc[MX][NY];
 #pragma unroll
 	for (int x = 0; x < MX; x++)
@@ -110,28 +117,37 @@ __device__ __forceinline__ void gw_body(const GwArg<T, PS> &a, int i0, int j0)
 			acc[x][y] = V4{0, 0, 0, 0};
 	if (k > 0)
 	{
-		unsigned ao[NV], bo[NY];
+		O ao[NV], bo[NY];
 #pragma unroll
 		for (int v = 0; v < NV; v++)
-			ao[v] = a.A.at(a.ai + min(i0 + 16 * VA * v + VA * c, lastv), a.aj);
+			ao[v] = a.A.at(a.ai + min(16 * VA * v + VA * c, lastv), a.aj);
 #pragma unroll
 		for (int y = 0; y < NY; y++)
 		{
-			const int j = min(j0 + 16 * y + strip_row<T>(c), n - 1);
-			bo[y] = OP == OP_NN ? (unsigned)(a.bj + j) * CS : a.B.at(a.bi + j, a.bj);
+			const int j = min(16 * y + strip_row<T>(c), n - 1);
+			bo[y] = OP == OP_NN ? (O)(a.bj + j) * CS : a.B.at(a.bi + j, a.bj);
 		}
 		const int ns = (k + 3) / 4;
 		VV av[DEPTH][NV];
 		T bv[DEPTH][NY];
 		auto load = [&](int s, VV (&x)[NV], T (&y)[NY]) {
+			s = min(s, ns - 1);
 			const int kq = min(4 * s + g, k - 1);
-			const unsigned kc = (unsigned)kq * CS, kb = OP == OP_NN ? a.B.at(a.bi + kq, 0) : kc;
+			const O kc = (O)kq * CS;
+			// gemm_nn: the rows of B from the panel of row 4 s on
+			StripView<T, PS, O> B = a.B;
+			O kb = kc;
+			if constexpr (OP == OP_NN)
+			{
+				B.p += (size_t)((unsigned)(4 * s) / PS) * B.cn * CS;
+				kb = B.at(a.bi + kq - ((4 * s) & ~(PS - 1)), 0);
+			}
 #pragma unroll
 			for (int v = 0; v < NV; v++)
 				x[v] = ldv(a.A, ao[v] + kc);
 #pragma unroll
 			for (int t = 0; t < NY; t++)
-				y[t] = a.B.ld(0, bo[t] + kb);
+				y[t] = B.ld(0, bo[t] + kb);
 		};
 		auto step = [&](const VV (&x)[NV], const T (&y)[NY]) {
 #pragma unroll
@@ -175,7 +191,7 @@ __device__ __forceinline__ void gw_body(const GwArg<T, PS> &a, int i0, int j0)
 	}
 	// D = beta * C + alpha * acc, a 16-column block at a time: its elements of C are
 	// all loaded before any of D is stored (C may be D)
-	const bool whole = i0 + 16 * MX <= m && j0 + 16 * NY <= n && !(SY && i0 < j0 + 16 * NY - 1);
+	const bool whole = 16 * MX <= m && 16 * NY <= n && !(SY && a.low < 16 * NY - 1);
 #pragma unroll
 	for (int y = 0; y < NY; y++)
 	{
@@ -185,22 +201,22 @@ __device__ __forceinline__ void gw_body(const GwArg<T, PS> &a, int i0, int j0)
 #pragma unroll
 			for (int v = 0; v < NV; v++)
 			{
-				const unsigned oc = a.C.at(a.ci + min(i0 + 16 * VA * v + VA * c, lastv), a.cj);
+				const O oc = a.C.at(a.ci + min(16 * VA * v + VA * c, lastv), a.cj);
 #pragma unroll
 				for (int r = 0; r < 4; r++)
-					cv[v][r] = ldv(a.C, oc + (unsigned)min(j0 + 16 * y + 4 * r + g, n - 1) * CS);
+					cv[v][r] = ldv(a.C, oc + (O)min(16 * y + 4 * r + g, n - 1) * CS);
 			}
 		}
 #pragma unroll
 		for (int v = 0; v < NV; v++)
 		{
-			const int gi = i0 + 16 * VA * v + VA * c;
-			const unsigned od = a.D.at(a.di + min(gi, lastv), a.dj);
+			const int gi = 16 * VA * v + VA * c;
+			const O od = a.D.at(a.di + min(gi, lastv), a.dj);
 #pragma unroll
 			for (int r = 0; r < 4; r++)
 			{
-				const int gj = j0 + 16 * y + 4 * r + g;
-				const unsigned o = od + (unsigned)min(gj, n - 1) * CS;
+				const int gj = 16 * y + 4 * r + g;
+				const O o = od + (O)min(gj, n - 1) * CS;
 				T val[VA];
 				VV vv;
 #pragma unroll
@@ -218,12 +234,12 @@ __device__ __forceinline__ void gw_body(const GwArg<T, PS> &a, int i0, int j0)
 					*(BFA_GLOBAL VV *)(a.D.p + o) = vv;
 				else if (gj < n)
 				{
-					if (gi + VA <= m && !(SY && gi < gj))
+					if (gi + VA <= m && !(SY && a.low + gi < gj))
 						*(BFA_GLOBAL VV *)(a.D.p + o) = vv;
 					else
 #pragma unroll
 						for (int e = 0; e < VA; e++)
-							if (gi + e < m && !(SY && gi + e < gj))
+							if (gi + e < m && !(SY && a.low + gi + e < gj))
 								*(BFA_GLOBAL T *)(a.D.p + o + e * (unsigned)sizeof(T)) = val[e];
 				}
 			}
@@ -233,19 +249,19 @@ __device__ __forceinline__ void gw_body(const GwArg<T, PS> &a, int i0, int j0)
 
 // the loop for a tile's nb <= E column blocks
 template <typename T, int PS, int OP, int MX, int E, int DEPTH>
-__device__ __forceinline__ void gw_blocks(const GwArg<T, PS> &a, int i0, int j0, int nb)
+__device__ __forceinline__ void gw_blocks(const GwArg<T, PS, unsigned> &a, int nb)
 {
 	constexpr int VA = gw_rows<T, MX>();
 	if constexpr (E == 4)
 	{
 		if (nb == 4)
-			return gw_body<T, PS, OP, MX, 4, VA, DEPTH>(a, i0, j0);
+			return gw_body<T, PS, OP, MX, 4, VA, DEPTH>(a);
 		if (nb == 3)
-			return gw_body<T, PS, OP, MX, 3, VA, DEPTH>(a, i0, j0);
+			return gw_body<T, PS, OP, MX, 3, VA, DEPTH>(a);
 	}
 	if (nb >= 2)
-		return gw_body<T, PS, OP, MX, 2, VA, DEPTH>(a, i0, j0);
-	gw_body<T, PS, OP, MX, 1, VA, DEPTH>(a, i0, j0);
+		return gw_body<T, PS, OP, MX, 2, VA, DEPTH>(a);
+	gw_body<T, PS, OP, MX, 1, VA, DEPTH>(a);
 }
 
 // One wave per (instance, tile slot): `slots` slots per instance (the tile
@@ -264,41 +280,71 @@ __global__ __launch_bounds__(WAVE, (gw_waves<T, E>())) void k_gemm_wave(const ty
 	if (inst >= batch)
 		return;
 	const typename GemmArg<T>::type &r = args[inst];
-	GwArg<T, PS> a;
-	a.m = __builtin_amdgcn_readfirstlane(r.m);
-	a.n = OP == OP_SYRK ? a.m : __builtin_amdgcn_readfirstlane(r.n);
-	a.k = __builtin_amdgcn_readfirstlane(r.k);
-	if (a.m <= 0 || a.n <= 0)
+	const int m = __builtin_amdgcn_readfirstlane(r.m), n = OP == OP_SYRK ? m : __builtin_amdgcn_readfirstlane(r.n);
+	if (m <= 0 || n <= 0)
 		return;
 	if (threadIdx.x == 0 && slot == 0)
 		r.sD->use_dA = 0;
-	const int mt = (a.m + TE - 1) / TE, nt = (a.n + TE - 1) / TE;
+	const int mt = (m + TE - 1) / TE, nt = (n + TE - 1) / TE;
 	const int ntiles = gw_ntiles<OP>(mt, nt);
 	if (slot >= ntiles)
 		return;
-	a.A = strip_view<T, PS>(r.sA);
-	a.B = strip_view<T, PS>(r.sB);
-	a.C = strip_view<T, PS>(r.sC);
-	a.D = strip_view<T, PS>(r.sD);
-	a.ai = r.ai, a.aj = r.aj, a.bi = r.bi, a.bj = r.bj, a.ci = r.ci, a.cj = r.cj, a.di = r.di, a.dj = r.dj;
-	a.alpha = r.alpha;
-	a.beta = r.beta;
+	const StripView<T, PS> A = strip_view<T, PS>(r.sA), B = strip_view<T, PS>(r.sB), C = strip_view<T, PS>(r.sC), D = strip_view<T, PS>(r.sD);
+	const int k = __builtin_amdgcn_readfirstlane(r.k);
+	// the tile at (i0, j0)
+	auto tile = [&](auto &a, int i0, int j0) {
+		typedef typename std::remove_reference_t<decltype(a.A)>::ofs O;
+		a.m = m - i0, a.n = n - j0, a.k = k, a.low = i0 - j0;
+		a.ai = r.ai + i0, a.aj = r.aj;
+		a.bi = OP == OP_NN ? r.bi : r.bi + j0, a.bj = OP == OP_NN ? r.bj + j0 : r.bj;
+		a.ci = r.ci + i0, a.cj = r.cj + j0, a.di = r.di + i0, a.dj = r.dj + j0;
+		a.A = A.template block<O>(a.ai, a.aj);
+		a.B = B.template block<O>(a.bi, a.bj);
+		a.C = C.template block<O>(a.ci, a.cj);
+		a.D = D.template block<O>(a.di, a.dj);
+		a.alpha = r.alpha;
+		a.beta = r.beta;
+	};
+	if (__builtin_expect(!strip_fits<T, PS>(max(max(A.cn, B.cn), max(C.cn, D.cn))), 0))
+	{
+		// 32 x 32 at a time: 64-bit offsets of more would not leave the other form
+		// its registers
+		for (int t = slot; t < ntiles; t += slots)
+		{
+			int ti, tj;
+			gw_tile<OP>(t, mt, nt, ti, tj);
+#pragma unroll 1
+			for (int q = 0; q < E * E / 4; q++)
+			{
+				const int i0 = ti * TE + 32 * (q / (E / 2)), j0 = tj * TE + 32 * (q % (E / 2));
+				if (i0 < m && j0 < n)
+				{
+					GwArg<T, PS, size_t> a;
+					tile(a, i0, j0);
+					gw_body<T, PS, OP, 2, 2, 1, 2>(a);
+				}
+			}
+		}
+		return;
+	}
 	// rows in pieces: the matrices' rows start on a piece's boundary, in memory too
 	constexpr int VA = gw_rows<T, E>();
-	const unsigned long long low = (unsigned long long)(uintptr_t)a.A.p | (unsigned long long)(uintptr_t)a.C.p | (unsigned long long)(uintptr_t)a.D.p;
-	const bool pieces = ((a.ai | a.ci | a.di) & (VA - 1)) == 0 && (low & (VA * sizeof(T) - 1)) == 0;
+	const unsigned long long low = (unsigned long long)(uintptr_t)A.p | (unsigned long long)(uintptr_t)C.p | (unsigned long long)(uintptr_t)D.p;
+	const bool pieces = ((r.ai | r.ci | r.di) & (VA - 1)) == 0 && (low & (VA * sizeof(T) - 1)) == 0;
 	for (int t = slot; t < ntiles; t += slots)
 	{
 		int ti, tj;
 		gw_tile<OP>(t, mt, nt, ti, tj);
 		const int i0 = ti * TE, j0 = tj * TE;
-		const int nb = min(E, (a.n - j0 + 15) / 16);
+		GwArg<T, PS, unsigned> a;
+		tile(a, i0, j0);
+		const int nb = min(E, (a.n + 15) / 16);
 		if (!pieces)
-			gw_body<T, PS, OP, E, E, 1, 2>(a, i0, j0);
-		else if (E == 2 || a.m - i0 <= 32)
-			gw_blocks<T, PS, OP, 2, E, DEPTH>(a, i0, j0, nb);
+			gw_body<T, PS, OP, E, E, 1, 2>(a);
+		else if (E == 2 || a.m <= 32)
+			gw_blocks<T, PS, OP, 2, E, DEPTH>(a, nb);
 		else if constexpr (E == 4)
-			gw_blocks<T, PS, OP, 4, E, DEPTH>(a, i0, j0, nb);
+			gw_blocks<T, PS, OP, 4, E, DEPTH>(a, nb);
 	}
 }
 

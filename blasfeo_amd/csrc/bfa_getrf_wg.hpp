@@ -198,11 +198,11 @@ __device__ __forceinline__ void glu_panel(int R, int cf, int c0, T *P, int ldp, 
 // COLS: the tiles are 16 rows of L each (ot: the lane's row at column g) and share
 // 16 columns of U (os: the lane's column at row g, rows of U being rows of panels);
 // else the tiles are 16 columns of U each and share 16 rows of L.
-template <typename T, int PS, int NT, bool COLS>
-__device__ __forceinline__ void glu_products(const StripView<T, PS> &D, const unsigned (&ot)[4], unsigned os, int di, int kend,
+template <typename T, int PS, int NT, bool COLS, typename O>
+__device__ __forceinline__ void glu_products(const StripView<T, PS, O> &D, const O (&ot)[4], O os, int di, int kend,
 	typename Vec4<T>::type (&acc)[4])
 {
-	constexpr unsigned CS = StripView<T, PS>::CS;
+	constexpr unsigned CS = PS * sizeof(T);
 	const int g = lane_id() >> 4;
 	T ta[GLU_D][NT][2], sh[GLU_D][2];
 	auto load = [&](int k, T (&t)[NT][2], T (&s)[2]) {
@@ -211,7 +211,7 @@ __device__ __forceinline__ void glu_products(const StripView<T, PS> &D, const un
 		for (int u = 0; u < 2; u++)
 		{
 			// column of L and row of U of this step
-			const unsigned lc = (unsigned)(k + 4 * u) * CS, ur = D.at(di + k + 4 * u + g, 0);
+			const O lc = (unsigned)(k + 4 * u) * CS, ur = D.at(di + k + 4 * u + g, 0);
 			s[u] = COLS ? D.ld(0, os + ur) : D.ld(lc, os);
 #pragma unroll
 			for (int i = 0; i < NT; i++)
@@ -244,8 +244,8 @@ __device__ __forceinline__ void glu_products(const StripView<T, PS> &D, const un
 			step(ta[d], sh[d]);
 }
 
-template <typename T, int PS, bool COLS>
-__device__ __forceinline__ void glu_sum(int nt, const StripView<T, PS> &D, const unsigned (&ot)[4], unsigned os, int di, int kend,
+template <typename T, int PS, bool COLS, typename O>
+__device__ __forceinline__ void glu_sum(int nt, const StripView<T, PS, O> &D, const O (&ot)[4], O os, int di, int kend,
 	typename Vec4<T>::type (&acc)[4])
 {
 	if (kend <= 0)
@@ -260,34 +260,40 @@ __device__ __forceinline__ void glu_sum(int nt, const StripView<T, PS> &D, const
 		glu_products<T, PS, 1, COLS>(D, ot, os, di, kend, acc);
 }
 
-template <typename T, int PS, bool PIV, int NW>
-__global__ __launch_bounds__(NW * WAVE, 3) void k_getrf_wg(const typename FactArg<T>::type *__restrict__ args, int mmax,
-	int batch, const int *__restrict__ counts, const int *__restrict__ lists)
+// a wave-uniform offset in a scalar register
+template <typename O>
+__device__ __forceinline__ O glu_uniform(size_t v)
+{
+	if constexpr (sizeof(O) == 8)
+		return uniform_u64(v);
+	else
+		return (O)__builtin_amdgcn_readfirstlane((int)v);
+}
+
+// What the waves of a workgroup share besides the panel.
+template <typename T, int NW>
+struct GluShared
+{
+	T Ub[16 * GLU_UL], invs[16];
+	size_t mdst[32], msrc[32];   // the moved rows' places, byte offsets
+	int pivs[16], perm[NW * WAVE], src[NW * WAVE], mrow[32], mperm[32], mcount;
+};
+
+template <typename T, int PS, bool PIV, int NW, typename O>
+__device__ __forceinline__ void glu_instance(const typename FactArg<T>::type &a, int m, int n, const StripView<T, PS> &vC,
+	const StripView<T, PS> &vD, T *P, GluShared<T, NW> &sh)
 {
 	typedef typename Vec4<T>::type V4;
-	constexpr int NTH = NW * WAVE, LDP = NTH + 1;
-	constexpr unsigned CS = StripView<T, PS>::CS;
-	extern __shared__ unsigned char smem_raw[];
-	T *P = reinterpret_cast<T *>(smem_raw);      // [16][LDP], rows from c0 on
-	__shared__ T Ub[16 * GLU_UL];
-	__shared__ T invs[16];
-	__shared__ int pivs[16];
-	__shared__ int perm[NTH], src[NTH];
-	__shared__ unsigned mdst[32], msrc[32];   // the moved rows' places, byte offsets
-	__shared__ int mrow[32], mperm[32], mcount;
-	const int inst = __builtin_amdgcn_readfirstlane(getrf_order(blockIdx.x, batch, counts, lists));
-	if (inst < 0)
-		return;
-	const typename FactArg<T>::type &a = args[inst];
-	const int m = __builtin_amdgcn_readfirstlane(a.m), n = __builtin_amdgcn_readfirstlane(a.n);
-	if (threadIdx.x == 0)
-		a.sD->use_dA = (a.di == 0 && a.dj == 0) ? 1 : 0;
-	if (m <= 0 || n <= 0 || m > mmax || m > NTH)
-		return;
-	const StripView<T, PS> C = strip_view<T, PS>(a.sC), D = strip_view<T, PS>(a.sD);
-	const int ci = a.ci, cj = a.cj, di = a.di, dj = a.dj;
+	constexpr int NTH = NW * WAVE, LDP = NTH + 1;   // P: [16][LDP], rows from c0 on
+	constexpr unsigned CS = PS * sizeof(T);
+	T *const Ub = sh.Ub, *const invs = sh.invs;
+	int *const pivs = sh.pivs, *const perm = sh.perm, *const src = sh.src, *const mrow = sh.mrow, *const mperm = sh.mperm;
+	int &mcount = sh.mcount;
+	size_t *const mdst = sh.mdst, *const msrc = sh.msrc;
 	// in place: the rows of C still to come are exchanged too, and perm stays
-	const bool inplace = C.p == D.p && ci == di && cj == dj;
+	const bool inplace = vC.p == vD.p && a.ci == a.di && a.cj == a.dj;
+	int ci = a.ci, cj = a.cj, di = a.di, dj = a.dj;
+	const StripView<T, PS, O> C = vC.template block<O>(ci, cj), D = vD.template block<O>(di, dj);
 	BFA_GLOBAL T *dD = (BFA_GLOBAL T *)a.sD->dA;
 	BFA_GLOBAL int *ipiv = (BFA_GLOBAL int *)a.ipiv;
 	const int p = min(m, n);
@@ -310,9 +316,9 @@ __global__ __launch_bounds__(NW * WAVE, 3) void k_getrf_wg(const typename FactAr
 			const int g = lane >> 4, c = lane & 15, rid = strip_row<T>(c);
 			// column panel: row tiles w, w + 4, ... of 16
 			const int nt = min(4, max(0, ((R + 15) / 16 - w + NW - 1) / NW));
-			unsigned ot[4];
+			O ot[4];
 			V4 acc[4];   // products minus C
-			const unsigned pc = (unsigned)(cj + min(c0 + c, n - 1)) * CS;
+			const O pc = (O)(cj + min(c0 + c, n - 1)) * CS;
 #pragma unroll
 			for (int t = 0; t < 4; t++)
 			{
@@ -324,7 +330,7 @@ __global__ __launch_bounds__(NW * WAVE, 3) void k_getrf_wg(const typename FactAr
 					for (int r = 0; r < 4; r++)
 						acc[t][r] = -C.ld(0, C.at(ci + perm[min(i0 + 4 * r + g, m - 1)], 0) + pc);
 			}
-			glu_sum<T, PS, true>(nt, D, ot, (unsigned)(dj + min(c0 + c, n - 1)) * CS, di, c0, acc);
+			glu_sum<T, PS, true>(nt, D, ot, (O)(dj + min(c0 + c, n - 1)) * CS, di, c0, acc);
 #pragma unroll
 			for (int t = 0; t < 4; t++)
 				if (t < nt)
@@ -353,7 +359,7 @@ __global__ __launch_bounds__(NW * WAVE, 3) void k_getrf_wg(const typename FactAr
 		{
 			// the panel to D, in strips of 16 rows
 			const int g = lane >> 4, c = lane & 15;
-			const unsigned oc = (unsigned)(dj + c0 + g) * CS;
+			const O oc = (O)(dj + c0 + g) * CS;
 #pragma unroll
 			for (int t = 0; t < 4; t++)
 			{
@@ -361,7 +367,7 @@ __global__ __launch_bounds__(NW * WAVE, 3) void k_getrf_wg(const typename FactAr
 				if (16 * (w + NW * t) < R)
 				{
 					const int si = src[min(i, R - 1)];
-					const unsigned od = D.at(di + c0 + min(i, R - 1), 0) + oc;
+					const O od = D.at(di + c0 + min(i, R - 1), 0) + oc;
 					T v[4];
 #pragma unroll
 					for (int s = 0; s < 4; s++)
@@ -401,17 +407,17 @@ __global__ __launch_bounds__(NW * WAVE, 3) void k_getrf_wg(const typename FactAr
 				{
 					const int k0 = kb + tid;
 					const bool in = k0 < ncol;
-					const unsigned oc = (unsigned)(dj + (!in ? 0 : k0 < c0 ? k0 : k0 + 16)) * CS;
+					const O oc = (O)(dj + (!in ? 0 : k0 < c0 ? k0 : k0 + 16)) * CS;
 					T v[32];
 #pragma unroll
 					for (int u = 0; u < 32; u++)
-						v[u] = D.ld((unsigned)__builtin_amdgcn_readfirstlane((int)msrc[min(u, nm - 1)]), oc);
+						v[u] = D.ld(glu_uniform<O>(msrc[min(u, nm - 1)]), oc);
 					wave_sync();   // the rows' places looked up after the loads
 #pragma unroll
 					for (int u = 0; u < 32; u++)
 						if (u < nm)
 						{
-							const unsigned od = (unsigned)__builtin_amdgcn_readfirstlane((int)mdst[u]);
+							const O od = glu_uniform<O>(mdst[u]);
 							if (in)
 								D.st(od, oc, v[u]);
 						}
@@ -429,20 +435,20 @@ __global__ __launch_bounds__(NW * WAVE, 3) void k_getrf_wg(const typename FactAr
 #pragma unroll
 			for (int s = 0; s < 4; s++)
 				pr[s] = perm[min(c0 + 4 * s + g, m - 1)];
-			const unsigned os = D.at(di + min(c0 + rid, m - 1), dj + g);
+			const O os = D.at(di + min(c0 + rid, m - 1), dj + g);
 			const int ntc = (n - c0 - 1) / 16;   // column tiles right of the panel
 #pragma unroll 1
 			for (int t0 = w; t0 < ntc; t0 += 4 * NW)
 			{
 				const int nt = min(4, (ntc - t0 + NW - 1) / NW);
-				unsigned ot[4];
+				O ot[4];
 				V4 acc[4];
 #pragma unroll
 				for (int t = 0; t < 4; t++)
 				{
 					acc[t] = V4{0, 0, 0, 0};
 					const int j = min(c0 + 16 * (t0 + NW * t + 1) + c, n - 1);
-					ot[t] = (unsigned)(dj + j) * CS;
+					ot[t] = (O)(dj + j) * CS;
 					if (t < nt)
 #pragma unroll
 						for (int s = 0; s < 4; s++)
@@ -475,6 +481,29 @@ __global__ __launch_bounds__(NW * WAVE, 3) void k_getrf_wg(const typename FactAr
 		}
 		__syncthreads();
 	}
+}
+
+template <typename T, int PS, bool PIV, int NW>
+__global__ __launch_bounds__(NW * WAVE, sizeof(T) == 8 ? 3 : 4) void k_getrf_wg(const typename FactArg<T>::type *__restrict__ args, int mmax,
+	int batch, const int *__restrict__ counts, const int *__restrict__ lists)
+{
+	extern __shared__ unsigned char smem_raw[];
+	T *P = reinterpret_cast<T *>(smem_raw);
+	__shared__ GluShared<T, NW> sh;
+	const int inst = __builtin_amdgcn_readfirstlane(getrf_order(blockIdx.x, batch, counts, lists));
+	if (inst < 0)
+		return;
+	const typename FactArg<T>::type &a = args[inst];
+	const int m = __builtin_amdgcn_readfirstlane(a.m), n = __builtin_amdgcn_readfirstlane(a.n);
+	if (threadIdx.x == 0)
+		a.sD->use_dA = (a.di == 0 && a.dj == 0) ? 1 : 0;
+	if (m <= 0 || n <= 0 || m > mmax || m > NW * WAVE)
+		return;
+	const StripView<T, PS> C = strip_view<T, PS>(a.sC), D = strip_view<T, PS>(a.sD);
+	if (__builtin_expect(strip_fits<T, PS>(max(C.cn, D.cn)), 1))
+		glu_instance<T, PS, PIV, NW, unsigned>(a, m, n, C, D, P, sh);
+	else
+		glu_instance<T, PS, PIV, NW, size_t>(a, m, n, C, D, P, sh);
 }
 
 } // namespace bfa

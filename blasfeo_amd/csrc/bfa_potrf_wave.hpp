@@ -41,12 +41,13 @@ constexpr int potrf_wave_elems()
 // above by memory: the rows of L that are read back miss L2 for the most part
 // (n = 128: 1.9 GB read for 0.55 GB of input).
 // ---------------------------------------------------------------------------
-template <typename T, int PS, int NB>
-__device__ __forceinline__ void potrf_wave(int m, int n, const StripView<T, PS> C, int ci, int cj,
-	const StripView<T, PS> D, int di, int dj, BFA_GLOBAL T *dD, T *lds)
+template <typename T, int PS, int NB, typename O>
+__device__ __forceinline__ void potrf_wave(int m, int n, const StripView<T, PS> vC, int ci, int cj,
+	const StripView<T, PS> vD, int di, int dj, BFA_GLOBAL T *dD, T *lds)
 {
 	typedef typename Vec4<T>::type V4;
 	constexpr bool LDSL = potrf_wave_lds<NB>();
+	const StripView<T, PS, O> C = vC.template block<O>(ci, cj), D = vD.template block<O>(di, dj);
 	const int lane = lane_id(), g = lane >> 4, rid = strip_row<T>(lane & 15);
 	const int R = (m + 15) / 16, Cb = (n + 15) / 16;
 	T *tri = lds, *ldiag = lds + 64 * NB, *ltile = ldiag + 192 * (NB - 1);
@@ -62,7 +63,7 @@ __device__ __forceinline__ void potrf_wave(int m, int n, const StripView<T, PS> 
 		const int row = 16 * J + rj, rc = min(row, m - 1);
 		const int kend = min(J, Cb);            // blocks left of the diagonal
 		const int nblk = min(J + 1, Cb);
-		const unsigned oc = C.at(ci + rc, cj + gj), od = D.at(di + rc, dj + gj);
+		const O oc = C.at(ci + rc, cj + gj), od = D.at(di + rc, dj + gj);
 		V4 cn;
 		strip_load<4>(C, oc, gj, 0, n, cn);
 #pragma unroll 1
@@ -70,7 +71,7 @@ __device__ __forceinline__ void potrf_wave(int m, int n, const StripView<T, PS> 
 		{
 			// row block L_K: its steps left of the diagonal from lp / ol
 			const T *lp = ltile + 256 * (K * (K - 1) / 2) + lane;
-			const unsigned ol = LDSL ? 0 : D.at(di + min(16 * K + rj, m - 1), dj + gj);
+			const O ol = LDSL ? 0 : D.at(di + min(16 * K + rj, m - 1), dj + gj);
 			T lk[3], d[4], l[3][4];
 			auto load_l = [&](int p, T (&v)[4]) {
 				if constexpr (LDSL)
@@ -153,8 +154,13 @@ __global__ __launch_bounds__(WAVE, (strip_waves<T, NB>())) void k_potrf_wave(con
 	const int n = mn ? min(m, __builtin_amdgcn_readfirstlane(a.n)) : m;
 	if (m <= 0 || n <= 0 || m > mmax || n > 16 * NB)
 		return;
-	potrf_wave<T, PS, NB>(m, n, strip_view<T, PS>(a.sC), a.ci, a.cj, strip_view<T, PS>(a.sD), a.di, a.dj,
-		(BFA_GLOBAL T *)a.sD->dA, lds);
+	const StripView<T, PS> C = strip_view<T, PS>(a.sC), D = strip_view<T, PS>(a.sD);
+	BFA_GLOBAL T *dD = (BFA_GLOBAL T *)a.sD->dA;
+	// narrow offsets where the rows of L are read back (n = 256: 2048 of them 3 per cent)
+	if (!potrf_wave_lds<NB>() && __builtin_expect(strip_fits<T, PS>(max(C.cn, D.cn)), 1))
+		potrf_wave<T, PS, NB, unsigned>(m, n, C, a.ci, a.cj, D, a.di, a.dj, dD, lds);
+	else
+		potrf_wave<T, PS, NB, size_t>(m, n, C, a.ci, a.cj, D, a.di, a.dj, dD, lds);
 	if (threadIdx.x == 0)
 		a.sD->use_dA = (a.di == 0 && a.dj == 0) ? (mn ? 1 : m) : 0;
 }
@@ -184,7 +190,7 @@ __device__ __forceinline__ void potrf_coop(int m, int n, int k, const StripView<
 	const int rh = min(16 * max(ih, 0) + rid, m - 1), rl = min(16 * max(il, 0) + rid, m - 1);
 	V4 hi[2 * NW], lo[NW];
 	{
-		const unsigned oh = C.at(ci + rh, cj + g), ol = C.at(ci + rl, cj + g);
+		const size_t oh = C.at(ci + rh, cj + g), ol = C.at(ci + rl, cj + g);
 #pragma unroll
 		for (int J = 0; J < 2 * NW; J++)
 			if (J <= ih && J < Cb)
@@ -198,21 +204,21 @@ __device__ __forceinline__ void potrf_coop(int m, int n, int k, const StripView<
 	{
 		// rows of B of a strip past its n rows: row n - 1 again (their columns of
 		// the result are past n)
-		const unsigned ah = A.at(ai + rh, aj + g), al = A.at(ai + rl, aj + g);
-		const unsigned bh = B.at(bi + min(rh, n - 1), bj + g), bl = B.at(bi + min(rl, n - 1), bj + g);
+		const size_t ah = A.at(ai + rh, aj + g), al = A.at(ai + rl, aj + g);
+		const size_t bh = B.at(bi + min(rh, n - 1), bj + g), bl = B.at(bi + min(rl, n - 1), bj + g);
 		// the operands of columns kk .. kk+15, zero past k (nothing is read there)
-		auto load = [&](const StripView<T, PS> &v, unsigned o, int kk, T (&x)[4]) {
+		auto load = [&](const StripView<T, PS> &v, size_t o, int kk, T (&x)[4]) {
 			if (kk + 16 <= k)
 #pragma unroll
 				for (int s = 0; s < 4; s++)
-					x[s] = v.ld((unsigned)(kk + 4 * s) * CS, o);
+					x[s] = v.ld((size_t)(kk + 4 * s) * CS, o);
 			else
 #pragma unroll
 				for (int s = 0; s < 4; s++)
 				{
 					x[s] = T(0);
 					if (kk + 4 * s + g < k)
-						x[s] = v.ld((unsigned)(kk + 4 * s) * CS, o);
+						x[s] = v.ld((size_t)(kk + 4 * s) * CS, o);
 				}
 		};
 		T vh[4] = {}, vl[4] = {}, uh[4] = {}, ul[4] = {};   // rows of A, rows of B

@@ -173,7 +173,7 @@ __device__ __forceinline__ void ric_coop(const RicRec &a, int N, int nkmax, doub
 	};
 	// the strip's rows of BAbt, columns past n1 zero
 	auto load_b = [&](const StripView<double, PS> &v, int I, int m, int n1, V4 (&b)[NX]) {
-		const unsigned o = v.at(min(16 * I + c, m - 1), g);
+		const size_t o = v.at(min(16 * I + c, m - 1), g);
 #pragma unroll
 		for (int C = 0; C < NX; C++)
 			if (16 * C < n1)
@@ -186,7 +186,7 @@ __device__ __forceinline__ void ric_coop(const RicRec &a, int N, int nkmax, doub
 					{
 						b[C][s] = 0.0;
 						if (16 * C + 4 * s + g < n1)
-							b[C][s] = v.ld((unsigned)(16 * C + 4 * s) * CS, o);
+							b[C][s] = v.ld((size_t)(16 * C + 4 * s) * CS, o);
 					}
 			}
 	};
@@ -206,7 +206,7 @@ __device__ __forceinline__ void ric_coop(const RicRec &a, int N, int nkmax, doub
 		int gk = g, ck = c;   // (pinned: offsets of all blocks are not kept across the stages)
 		BFA_PIN(gk);
 		BFA_PIN(ck);
-		const unsigned oh = q.R.at(min(16 * max(ih, 0) + ck, m - 1), gk), ol = q.R.at(min(16 * max(il, 0) + ck, m - 1), gk);
+		const size_t oh = q.R.at(min(16 * max(ih, 0) + ck, m - 1), gk), ol = q.R.at(min(16 * max(il, 0) + ck, m - 1), gk);
 #pragma unroll
 		for (int J = 0; J < 2 * NW; J++)
 			if (J <= ih && 16 * J < nk)
@@ -226,7 +226,7 @@ __device__ __forceinline__ void ric_coop(const RicRec &a, int N, int nkmax, doub
 		BFA_PIN(ck);
 		auto strip = [&](int I) {
 			const int row = 16 * I + ck;
-			const unsigned o = q.L.at(min(row, m - 1), gk);
+			const size_t o = q.L.at(min(row, m - 1), gk);
 #pragma unroll 1
 			for (int J = 0; J <= I && 16 * J < nk; J++)
 			{

@@ -406,7 +406,7 @@ template <int PS, int MX>
 __device__ __forceinline__ void trs_fetch(const BFA_GLOBAL double *p, int cn, int m, int n, double (&v)[trs_regs<MX>()])
 {
 	const int h = threadIdx.x / MX, i = min((int)threadIdx.x % MX, m - 1);
-	p += (i & ~(PS - 1)) * cn + (i & (PS - 1));
+	p += (size_t)(i & ~(PS - 1)) * cn + (i & (PS - 1));
 #pragma unroll
 	for (int t = 0; t < trs_regs<MX>(); t++)
 		v[t] = p[min(WAVE / MX * t + h, n - 1) * PS];

@@ -32,33 +32,51 @@
 
 namespace bfa {
 
-// A panel-major matrix as the strip kernels address it: a wave-uniform base
-// and 32-bit byte offsets (a matrix takes less than 2^31 bytes, its memsize
-// being an int), so that an access is one instruction with a scalar base, a
-// 32-bit offset register and a constant for the column.
-template <typename T, int PS>
+// A panel-major matrix as the strip kernels address it: a wave-uniform base and byte
+// offsets of type O.  O = size_t reaches every matrix.  With O = unsigned an access is
+// one instruction with a scalar base, a 32-bit offset register and a constant
+// for the column; a matrix may take 4 GiB and more, so the base is first moved to
+// the block at hand (block()), and that the block's own offsets fit is asked of
+// the panel stride (strip_fits).  Where registers are short, the kernel has both forms
+// and takes the narrow one where it reaches (with size_t alone gemm in FP32 takes 1.12,
+// trsm_rltn 1.12, getrf 1.09 times as long); the Cholesky and Riccati kernels are no
+// slower with size_t.
+template <typename T, int PS, typename O = size_t>
 struct StripView
 {
+	typedef O ofs;
 	static constexpr unsigned CS = PS * sizeof(T);   // bytes from one column to the next
 	BFA_GLOBAL char *p;
 	unsigned cn;
 	// byte offset of element (i, j)
-	__device__ __forceinline__ unsigned at(int i, int j) const
+	__device__ __forceinline__ O at(int i, int j) const
 	{
-		return (((unsigned)i & ~(unsigned)(PS - 1)) * cn + (unsigned)j * PS + ((unsigned)i & (PS - 1))) * (unsigned)sizeof(T);
+		return ((O)((unsigned)i / PS) * cn + (unsigned)j) * CS + ((unsigned)i & (PS - 1)) * (unsigned)sizeof(T);
 	}
 	// the value at a wave-uniform offset u plus this lane's offset o
-	__device__ __forceinline__ T ld(unsigned u, unsigned o) const { return *(const BFA_GLOBAL T *)((p + u) + o); }
-	__device__ __forceinline__ void st(unsigned u, unsigned o, T v) const { *(BFA_GLOBAL T *)((p + u) + o) = v; }
+	__device__ __forceinline__ T ld(O u, O o) const { return *(const BFA_GLOBAL T *)((p + u) + o); }
+	__device__ __forceinline__ void st(O u, O o, T v) const { *(BFA_GLOBAL T *)((p + u) + o) = v; }
+	// The matrix from the panel of row i and column j on (wave-uniform): i becomes the row
+	// within that panel, j 0.
+	template <typename O2>
+	__device__ __forceinline__ StripView<T, PS, O2> block(int &i, int &j) const
+	{
+		StripView<T, PS, O2> r;
+		r.p = p + ((size_t)((unsigned)i / PS) * cn + (unsigned)j) * CS;
+		r.cn = cn;
+		i &= PS - 1;
+		j = 0;
+		return r;
+	}
 };
 
 // Steps 0 .. NS-1 of a strip's 16-column block that starts at column c (wave-
-// uniform) of n: og is this lane's row at column g.  Columns past n read
+// uniform) of n <= 256: og is this lane's row at column g.  Columns past n read
 // column n - 1.
-template <int NS, typename T, int PS, typename X>
-__device__ __forceinline__ void strip_load(const StripView<T, PS> &v, unsigned og, int g, int c, int n, X &x)
+template <int NS, typename T, int PS, typename O, typename X>
+__device__ __forceinline__ void strip_load(const StripView<T, PS, O> &v, O og, int g, int c, int n, X &x)
 {
-	constexpr unsigned CS = StripView<T, PS>::CS;
+	constexpr unsigned CS = PS * sizeof(T);
 	if (c + 16 <= n)
 	{
 #pragma unroll
@@ -69,24 +87,24 @@ __device__ __forceinline__ void strip_load(const StripView<T, PS> &v, unsigned o
 	{
 #pragma unroll
 		for (int s = 0; s < NS; s++)
-			x[s] = v.ld(0, og + (unsigned)(min(c + 4 * s + g, n - 1) - g) * CS);
+			x[s] = v.ld(0, og + (O)(ptrdiff_t)((min(c + 4 * s + g, n - 1) - g) * (int)CS));
 	}
 }
 // The same where the block is known to be inside.
-template <int NS, typename T, int PS, typename X>
-__device__ __forceinline__ void strip_load_full(const StripView<T, PS> &v, unsigned og, int c, X &x)
+template <int NS, typename T, int PS, typename O, typename X>
+__device__ __forceinline__ void strip_load_full(const StripView<T, PS, O> &v, O og, int c, X &x)
 {
-	constexpr unsigned CS = StripView<T, PS>::CS;
+	constexpr unsigned CS = PS * sizeof(T);
 #pragma unroll
 	for (int s = 0; s < NS; s++)
 		x[s] = v.ld((unsigned)c * CS + 4 * s * CS, og);
 }
 // Block x (columns c .. c+15 of n) to a strip's rows; ok: this lane's row is
 // one of the matrix's.
-template <typename T, int PS, typename X>
-__device__ __forceinline__ void strip_store(const StripView<T, PS> &v, unsigned og, int g, int c, int n, bool ok, const X &x)
+template <typename T, int PS, typename O, typename X>
+__device__ __forceinline__ void strip_store(const StripView<T, PS, O> &v, O og, int g, int c, int n, bool ok, const X &x)
 {
-	constexpr unsigned CS = StripView<T, PS>::CS;
+	constexpr unsigned CS = PS * sizeof(T);
 	if (c + 16 <= n)
 	{
 		if (ok)
@@ -104,11 +122,11 @@ __device__ __forceinline__ void strip_store(const StripView<T, PS> &v, unsigned 
 }
 // The lower triangle of a factored diagonal block (columns c .. c+15 of n) to D
 // and its reciprocal pivots to dD.
-template <typename T, int PS>
-__device__ __forceinline__ void strip_store_diag(const StripView<T, PS> &v, unsigned og, int g, int rid, int c, int n, bool ok,
+template <typename T, int PS, typename O>
+__device__ __forceinline__ void strip_store_diag(const StripView<T, PS, O> &v, O og, int g, int rid, int c, int n, bool ok,
 	const T (&l)[4], BFA_GLOBAL T *dD, const T (&iv)[4])
 {
-	constexpr unsigned CS = StripView<T, PS>::CS;
+	constexpr unsigned CS = PS * sizeof(T);
 #pragma unroll
 	for (int s = 0; s < 4; s++)
 	{
@@ -133,6 +151,14 @@ __device__ __forceinline__ StripView<T, PS> strip_view(const typename MatOf<T>::
 	r.p = (BFA_GLOBAL char *)(uintptr_t)uniform_u64((unsigned long long)(uintptr_t)v.p);
 	r.cn = (unsigned)__builtin_amdgcn_readfirstlane(v.cn);
 	return r;
+}
+
+// Do the byte offsets of a block of up to 256 rows (and a panel's remainder at either
+// end) fit 32 bits, the largest panel stride being cn?
+template <typename T, int PS>
+__device__ __forceinline__ bool strip_fits(unsigned cn)
+{
+	return cn <= 0xffffffffu / ((256 + 2 * PS) * (unsigned)sizeof(T));
 }
 
 // Row (0..15) of the 16-row strip that lane position c holds, and, the map

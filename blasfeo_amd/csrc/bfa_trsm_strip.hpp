@@ -38,7 +38,7 @@ constexpr size_t trsm_lds()
 template <typename T, int NB>
 constexpr int trsm_waves()
 {
-	return sizeof(T) * NB * trsm_strips<NB>() <= 64 ? 3 : 2;
+	return NB <= 4 ? (sizeof(T) == 8 ? 4 : 5) : sizeof(T) * NB * trsm_strips<NB>() <= 64 ? 3 : 2;
 }
 
 // Workgroup (instance, slot) solves the blocks of 64 S rows slot, slot + slots, ...
@@ -46,29 +46,18 @@ constexpr int trsm_waves()
 // DA_GIVEN: the reciprocal diagonal is read from sA->dA whatever use_dA says
 // (the trapezoid Cholesky, whose diagonal block was just factored into the same
 // descriptor with its reciprocals stored there).
-template <typename T, int PS, int NB, bool DA_GIVEN>
-__global__ __launch_bounds__(NT3, (trsm_waves<T, NB>())) void k_trsm_rltn(const typename TrsmArg<T>::type *__restrict__ args,
-	int batch, int slots, int nlo, int nmax)
+template <typename T, int PS, int NB, bool DA_GIVEN, typename O>
+__device__ __forceinline__ void trsm_rows(const typename TrsmArg<T>::type &a, int m, int n, const StripView<T, PS> &vA,
+	const StripView<T, PS> &vB, const StripView<T, PS> &vD, int slot, int slots, T *tiles, T *inv_s)
 {
 	typedef typename Vec4<T>::type V4;
 	constexpr int S = trsm_strips<NB>(), NW = NT3 / WAVE, NT = NB / NW;
-	extern __shared__ unsigned char smem_raw[];
-	T *tiles = reinterpret_cast<T *>(smem_raw);
-	__shared__ T inv_s[16 * NB];
-	int inst, slot;
-	xcd_inst_slot(slots, inst, slot);
-	if (inst >= batch)
-		return;
-	const typename TrsmArg<T>::type &a = args[inst];
-	const int m = __builtin_amdgcn_readfirstlane(a.m), n = __builtin_amdgcn_readfirstlane(a.n);
-	if (m <= 0 || n <= nlo || n > nmax || n > 16 * NB || slot * 64 * S >= m)
-		return;
-	const StripView<T, PS> A = strip_view<T, PS>(a.sA), B = strip_view<T, PS>(a.sB), D = strip_view<T, PS>(a.sD);
-	const int ai = a.ai, aj = a.aj;
+	int ai = a.ai, aj = a.aj;
+	const StripView<T, PS, O> A = vA.template block<O>(ai, aj);
 	const T alpha = a.alpha;
 	// reciprocal diagonal: cached copy when valid at launch, else 1/A_jj
 	// (an output aliasing A invalidates the cache first, as in the reference)
-	const bool cached = DA_GIVEN || (ai == 0 && aj == 0 && a.sD != a.sA && a.sA->use_dA >= n);
+	const bool cached = DA_GIVEN || (a.ai == 0 && a.aj == 0 && a.sD != a.sA && a.sA->use_dA >= n);
 	const BFA_GLOBAL T *dA = (const BFA_GLOBAL T *)a.sA->dA;
 	for (int j = threadIdx.x; j < 16 * NB; j += NT3)
 		inv_s[j] = j < n ? (cached ? dA[j] : T(1) / A.ld(0, A.at(ai + j, aj + j))) : T(0);
@@ -100,13 +89,16 @@ __global__ __launch_bounds__(NT3, (trsm_waves<T, NB>())) void k_trsm_rltn(const 
 		bool first = true;
 		for (int r0 = slot * 64 * S; r0 < m; r0 += slots * 64 * S)
 		{
-			int row[S];
+			// rows from r0 on
+			int row[S], bi = a.bi + r0, bj = a.bj, di = a.di + r0, dj = a.dj;
+			const int mr = m - r0;
+			const StripView<T, PS, O> B = vB.template block<O>(bi, bj), D = vD.template block<O>(di, dj);
 			V4 nx[S][NB];   // alpha B, then -X of the finished blocks
 #pragma unroll
 			for (int t = 0; t < S; t++)
 			{
-				row[t] = r0 + 16 * (S * w + t) + rid;
-				const unsigned ob = B.at(a.bi + min(row[t], m - 1), a.bj + g);
+				row[t] = 16 * (S * w + t) + rid;
+				const O ob = B.at(bi + min(row[t], mr - 1), bj + g);
 #pragma unroll
 				for (int K = 0; K < NB; K++)
 					if (K < nb)
@@ -124,7 +116,7 @@ __global__ __launch_bounds__(NT3, (trsm_waves<T, NB>())) void k_trsm_rltn(const 
 				first = false;
 			}
 			// the waves past the last row have shared in the loads above
-			if (r0 + 16 * S * w >= m)
+			if (16 * S * w >= mr)
 				continue;
 #pragma unroll
 			for (int K = 0; K < NB; K++)
@@ -166,8 +158,8 @@ __global__ __launch_bounds__(NT3, (trsm_waves<T, NB>())) void k_trsm_rltn(const 
 #pragma unroll
 					for (int t = 0; t < S; t++)
 					{
-						const unsigned od = D.at(a.di + min(row[t], m - 1), a.dj + g);
-						strip_store(D, od, g, 16 * K, n, row[t] < m, x[t]);
+						const O od = D.at(di + min(row[t], mr - 1), dj + g);
+						strip_store(D, od, g, 16 * K, n, row[t] < mr, x[t]);
 #pragma unroll
 						for (int s = 0; s < 4; s++)
 							nx[t][K][s] = -x[t][s];
@@ -180,7 +172,7 @@ __global__ __launch_bounds__(NT3, (trsm_waves<T, NB>())) void k_trsm_rltn(const 
 	// column later, to LDS
 	T st[NT][4];
 	auto fetch = [&](int K) {
-		const unsigned ol = A.at(ai + min(16 * K + rid, n - 1), aj + g);
+		const O ol = A.at(ai + min(16 * K + rid, n - 1), aj + g);
 #pragma unroll
 		for (int t = 0; t < NT; t++)
 			if (w + NW * t <= K)
@@ -197,14 +189,16 @@ __global__ __launch_bounds__(NT3, (trsm_waves<T, NB>())) void k_trsm_rltn(const 
 	};
 	for (int r0 = slot * 64 * S; r0 < m; r0 += slots * 64 * S)
 	{
-		int row[S];
-		unsigned ob[S];
+		int row[S], bi = a.bi + r0, bj = a.bj, di = a.di + r0, dj = a.dj;
+		const int mr = m - r0;
+		const StripView<T, PS, O> B = vB.template block<O>(bi, bj), D = vD.template block<O>(di, dj);
+		O ob[S];
 		V4 nx[S][NB], cn[S];
 #pragma unroll
 		for (int t = 0; t < S; t++)
 		{
-			row[t] = r0 + 16 * (S * w + t) + rid;
-			ob[t] = B.at(a.bi + min(row[t], m - 1), a.bj + g);
+			row[t] = 16 * (S * w + t) + rid;
+			ob[t] = B.at(bi + min(row[t], mr - 1), bj + g);
 			strip_load<4>(B, ob[t], g, 0, n, cn[t]);
 		}
 		fetch(0);
@@ -274,13 +268,35 @@ __global__ __launch_bounds__(NT3, (trsm_waves<T, NB>())) void k_trsm_rltn(const 
 #pragma unroll
 		for (int t = 0; t < S; t++)
 		{
-			const unsigned od = D.at(a.di + min(row[t], m - 1), a.dj + g);
+			const O od = D.at(di + min(row[t], mr - 1), dj + g);
 #pragma unroll
 			for (int K = 0; K < NB; K++)
 				if (K < nb)
-					strip_store(D, od, ge, 16 * K, n, row[t] < m, -nx[t][K]);
+					strip_store(D, od, ge, 16 * K, n, row[t] < mr, -nx[t][K]);
 		}
 	}
+}
+
+template <typename T, int PS, int NB, bool DA_GIVEN>
+__global__ __launch_bounds__(NT3, (trsm_waves<T, NB>())) void k_trsm_rltn(const typename TrsmArg<T>::type *__restrict__ args,
+	int batch, int slots, int nlo, int nmax)
+{
+	extern __shared__ unsigned char smem_raw[];
+	T *tiles = reinterpret_cast<T *>(smem_raw);
+	__shared__ T inv_s[16 * NB];
+	int inst, slot;
+	xcd_inst_slot(slots, inst, slot);
+	if (inst >= batch)
+		return;
+	const typename TrsmArg<T>::type &a = args[inst];
+	const int m = __builtin_amdgcn_readfirstlane(a.m), n = __builtin_amdgcn_readfirstlane(a.n);
+	if (m <= 0 || n <= nlo || n > nmax || n > 16 * NB || slot * 64 * trsm_strips<NB>() >= m)
+		return;
+	const StripView<T, PS> A = strip_view<T, PS>(a.sA), B = strip_view<T, PS>(a.sB), D = strip_view<T, PS>(a.sD);
+	if (__builtin_expect(strip_fits<T, PS>(max(A.cn, max(B.cn, D.cn))), 1))
+		trsm_rows<T, PS, NB, DA_GIVEN, unsigned>(a, m, n, A, B, D, slot, slots, tiles, inv_s);
+	else
+		trsm_rows<T, PS, NB, DA_GIVEN, size_t>(a, m, n, A, B, D, slot, slots, tiles, inv_s);
 }
 
 } // namespace bfa

@@ -152,3 +152,11 @@ def test_riccati_mixed(emu_build, ps):
     1e-9 of the oracle's FP64 factorisation + solve), and with tol 0 the FP64
     fallback for every instance (the oracle's results at the 1e-11 rule)."""
     run_case("case_ric.py", "mixed", ps)
+
+
+@pytest.mark.parametrize("geom", ["stride", "deep"])
+@pytest.mark.parametrize("ps", [4, 8])
+def test_more_than_4_gib(emu_build, ps, geom):
+    """Matrices of more than 4 GiB (sparse here): blocks whose byte offsets pass 2^32 within
+    the block, and blocks that lie behind it."""
+    run_case("case_wide.py", geom, ps)
