@@ -290,10 +290,11 @@ __device__ __forceinline__ void glu_instance(const typename FactArg<T>::type &a,
 	int *const pivs = sh.pivs, *const perm = sh.perm, *const src = sh.src, *const mrow = sh.mrow, *const mperm = sh.mperm;
 	int &mcount = sh.mcount;
 	size_t *const mdst = sh.mdst, *const msrc = sh.msrc;
-	// in place: the rows of C still to come are exchanged too, and perm stays
-	const bool inplace = vC.p == vD.p && a.ci == a.di && a.cj == a.dj;
 	int ci = a.ci, cj = a.cj, di = a.di, dj = a.dj;
 	const StripView<T, PS, O> C = vC.template block<O>(ci, cj), D = vD.template block<O>(di, dj);
+	// in place (the same elements, through whatever descriptors and offsets): the rows
+	// of C still to come are exchanged too, and perm stays
+	const bool inplace = C.p == D.p && ci == di && C.cn == D.cn;
 	BFA_GLOBAL T *dD = (BFA_GLOBAL T *)a.sD->dA;
 	BFA_GLOBAL int *ipiv = (BFA_GLOBAL int *)a.ipiv;
 	const int p = min(m, n);

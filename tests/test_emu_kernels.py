@@ -160,3 +160,10 @@ def test_more_than_4_gib(emu_build, ps, geom):
     """Matrices of more than 4 GiB (sparse here): blocks whose byte offsets pass 2^32 within
     the block, and blocks that lie behind it."""
     run_case("case_wide.py", geom, ps)
+
+
+@pytest.mark.parametrize("ps", [4, 8])
+@pytest.mark.parametrize("op", ["getrf_rp", "getrf_np"])
+def test_getrf_in_place_two_descriptors(emu_build, op, ps):
+    """LU in place where C and D are two descriptors of the same elements."""
+    run_case("case_alias.py", op, ps)
