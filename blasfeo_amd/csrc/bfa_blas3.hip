@@ -440,6 +440,11 @@ static int check_common(int ps, int batch, const void *args, bool is_float, cons
 	return BLASFEO_AMD_OK;
 }
 
+// threads of a launch (the CPU emulator of the kernels sets a smaller limit)
+#ifndef BFA_GRID_THREADS
+#define BFA_GRID_THREADS 0x7fffffffLL
+#endif
+
 // 1-D grid of batch * slots workgroups rounded up to a multiple of XCDS, for
 // kernels that map their workgroup id through xcd_local_index
 static int xcd_grid(int batch, int slots, int threads, dim3 *grid, const char *name)
@@ -531,14 +536,21 @@ static int launch_trsm_nb(int batch, const typename TrsmArg<T>::type *args, int 
 	constexpr int rows = 64 * trsm_strips<NB>();
 	const int slots = mmax > 0 ? min(64, (mmax + rows - 1) / rows) : 4;
 	constexpr size_t shm = trsm_lds<T, NB>();
-	dim3 grid;
-	int rc = xcd_grid(batch, slots, NT3, &grid, name);
-	if (!rc)
-		rc = lds_check(reinterpret_cast<const void *>(&k_trsm_rltn<T, PS, NB, GIVEN>), shm, name);
-	if (rc)
-		return rc;
-	hipLaunchKernelGGL((k_trsm_rltn<T, PS, NB, GIVEN>), grid, dim3(NT3), shm, st, args, batch, slots, nlo, nmax);
-	return check_launch(name);
+	int rc = lds_check(reinterpret_cast<const void *>(&k_trsm_rltn<T, PS, NB, GIVEN>), shm, name);
+	// a launch has fewer than BFA_GRID_THREADS threads: larger batches take several
+	const int most = max(1, ((int)((long long)BFA_GRID_THREADS / NT3) - XCDS) / slots);
+	for (int i = 0; i < batch && !rc; i += most)
+	{
+		const int part = min(most, batch - i);
+		dim3 grid;
+		if ((rc = xcd_grid(part, slots, NT3, &grid, name)))
+			break;
+		hipLaunchKernelGGL((k_trsm_rltn<T, PS, NB, GIVEN>), grid, dim3(NT3), shm, st, args + i, part, slots, nlo, nmax);
+		rc = check_launch(name);
+		if (batch - i <= most)
+			break;   // (i + most may pass the range of an int)
+	}
+	return rc;
 }
 template <typename T, int PS, bool GIVEN = false>
 static int launch_trsm_ps(int batch, const typename TrsmArg<T>::type *args, const blasfeo_amd_hint *hint, hipStream_t st, const char *name)

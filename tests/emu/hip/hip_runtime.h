@@ -198,3 +198,4 @@ inline hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return
 inline hipError_t hipGetLastError() { return hipSuccess; }
 inline hipError_t hipPeekAtLastError() { return hipSuccess; }
 inline const char *hipGetErrorString(hipError_t) { return "emulated"; }
+#define BFA_GRID_THREADS (1 << 14)   // trsm_rltn: batches over several launches from a few instances on

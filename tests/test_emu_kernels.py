@@ -167,3 +167,9 @@ def test_more_than_4_gib(emu_build, ps, geom):
 def test_getrf_in_place_two_descriptors(emu_build, op, ps):
     """LU in place where C and D are two descriptors of the same elements."""
     run_case("case_alias.py", op, ps)
+
+
+@pytest.mark.parametrize("ps", [4, 8])
+def test_trsm_rltn_several_launches(emu_build, ps):
+    """trsm_rltn of a batch whose workgroups pass a launch's limit."""
+    run_case("case_trsm.py", "launches", ps)
