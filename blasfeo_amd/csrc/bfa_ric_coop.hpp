@@ -47,7 +47,7 @@ struct CoopLower
 // LDS values for an instance of R strips and nxt state tiles at most.  The first
 // two hold a zero (the product's operand above the diagonal) and padding; then
 // the 4 x 4 triangles and the reciprocal diagonal.
-constexpr int RC_TRI = 2, RC_INV = RC_TRI + 128, RC_TILES = RC_INV + 128;
+constexpr int RC_TRI = 2, RC_INV = RC_TRI + 128, RC_TILES = RC_INV + 128;   // (ric_beyond takes 512 of at least 530)
 __host__ __device__ constexpr int ric_coop_elems(int R, int nxt)
 {
 	return RC_TILES + R * (R + 1) / 2 * RT_SZ + (R > 0 ? R - 1 : 0) * nxt * 256;
@@ -434,24 +434,115 @@ __device__ __forceinline__ void ric_coop(const RicRec &a, int N, int nkmax, doub
 		store_l(done);
 }
 
+// An instance of up to 128 rows that does not fit a direct launch, its hint being too
+// small: one wave, the stage matrix in L[k] itself, four columns of W at a time in LDS.
+// What it takes does not matter, only that such an instance is factorised as the class
+// launches factorise it.
+template <int PS, bool AUG>
+__device__ __forceinline__ void ric_beyond(const RicRec &a, int N, double *W)
+{
+	constexpr int XR = AUG ? 1 : 0, RW = 128;
+	const int lane = lane_id();
+	int n1 = 0, u1 = 0;   // sizes of stage k + 1
+#pragma unroll 1
+	for (int k = N; k >= 0; k--)
+	{
+		const int x = a.nx[k], u = k < N ? a.nu[k] : 0, nk = x + u, m = nk > 0 || AUG ? nk + XR : 0;
+		const PM<double, PS> C = view<double, PS>(a.BAbt + (k < N ? k : 0)), R = view<double, PS>(a.RSQrq + k);
+		const PM<double, PS> L = view<double, PS>(a.L + k), L1 = view<double, PS>(a.L + min(k + 1, N));
+#pragma unroll 1
+		for (int i = lane; i < m; i += WAVE)
+#pragma unroll 1
+			for (int j = 0; j <= min(i, nk - 1); j++)
+				L.at(i, j) = R.at(i, j);
+#pragma unroll 1
+		for (int c = 0; k < N && c < n1; c += 4)
+		{
+			const int cw = min(4, n1 - c);
+#pragma unroll 1
+			for (int i = lane; i < m; i += WAVE)
+#pragma unroll 1
+				for (int q = 0; q < cw; q++)
+				{
+					double w = 0.0;
+#pragma unroll 1
+					for (int l = c + q; l < n1; l++)
+						w += C.at(i, l) * L1.at(u1 + l, u1 + c + q);
+					if (AUG && i == nk)
+						w += L1.at(u1 + n1, u1 + c + q);
+					W[q * RW + i] = w;
+				}
+			wave_sync();
+#pragma unroll 1
+			for (int i = lane; i < m; i += WAVE)
+#pragma unroll 1
+				for (int j = 0; j <= min(i, nk - 1); j++)
+				{
+					double w = 0.0;
+#pragma unroll 1
+					for (int q = 0; q < cw; q++)
+						w += W[q * RW + i] * W[q * RW + j];
+					L.at(i, j) += w;
+				}
+			wave_sync();
+		}
+#pragma unroll 1
+		for (int j = 0; j < nk; j++)
+		{
+			double v[2] = {0.0, 0.0};   // rows lane and lane + 64 of column j
+#pragma unroll
+			for (int q = 0; q < 2; q++)
+				if (lane + WAVE * q >= j && lane + WAVE * q < m)
+				{
+					double w = 0.0;
+#pragma unroll 1
+					for (int p = 0; p < j; p++)
+						w += L.at(lane + WAVE * q, p) * L.at(j, p);
+					v[q] = L.at(lane + WAVE * q, j) - w;
+				}
+			const double d = j < WAVE ? readlane(v[0], j) : readlane(v[1], j - WAVE);
+			const double inv = d > 0.0 ? rsqrt_fast(d) : 0.0;
+#pragma unroll
+			for (int q = 0; q < 2; q++)
+				if (lane + WAVE * q >= j && lane + WAVE * q < m)
+					L.at(lane + WAVE * q, j) = v[q] * inv;
+			if (lane == 0)
+				a.L[k].dA[j] = inv;
+			wave_sync();
+		}
+		if (lane == 0)
+		{
+			a.L[k].use_dA = (k == N && !AUG) ? nk : 1;
+			if (k < N)
+				a.work->use_dA = 0;
+		}
+		n1 = x;
+		u1 = u;
+	}
+}
+
 // Waves per SIMD that the kernels are compiled for.
 constexpr int ric_coop_waves(int NW) { return NW == 1 ? 3 : 2; }
 
-// One instance per workgroup (list == nullptr: workgroup b takes instance b), or a
-// persistent launch over a class list, the workgroups taking instances from the
-// atomic queue head.  Rcap: the strips that the launch's LDS holds; instances that
-// do not fit the launch (rcap, nx > 16 NX or negative sizes) are left alone.
-template <int PS, int NW, int NX, bool AUG>
+// DIRECT: one instance per workgroup (workgroup b takes instance b); else a persistent
+// launch over a class list, the workgroups taking instances from the atomic queue
+// head.  Rcap: the strips that the launch's LDS holds.  A direct launch has the plan's rule
+// (ric_class) for instances larger than the hint (mmax rows): up to 64 states and 128
+// rows, with AUG the augmented one among them, or up to mmax rows whatever their states
+// (not with AUG) they are factorised all the same, others are left alone, as are
+// negative sizes.
+template <int PS, int NW, int NX, bool AUG, bool DIRECT>
 __global__ __launch_bounds__(NW * WAVE, (ric_coop_waves(NW))) void k_ric_coop(const typename RicArg<AUG>::type *__restrict__ args,
-	int Rcap, const int *__restrict__ count, const int *__restrict__ list, int *head)
+	int Rcap, int mmax, const int *__restrict__ count, const int *__restrict__ list, int *head)
 {
 	extern __shared__ double smem_d[];
 	__shared__ int qslot;
-	const int cnt = list ? *count : 0;
+	constexpr int XR = AUG ? 1 : 0;
+	const int cnt = DIRECT ? 0 : *count;
 	for (;;)
 	{
 		int i = blockIdx.x;
-		if (list)
+		if (!DIRECT)
 		{
 			__syncthreads();   // every wave has left the previous instance
 			if (threadIdx.x == 0)
@@ -468,14 +559,19 @@ __global__ __launch_bounds__(NW * WAVE, (ric_coop_waves(NW))) void k_ric_coop(co
 		{
 			int nk, nx, least;
 			ric_sizes(a, N, nk, nx, least);
-			if (least >= 0 && nx <= 16 * NX && (nk + (AUG ? 1 : 0) + 15) / 16 <= Rcap)
+			if (least >= 0 && nx <= 16 * NX && (nk + XR + 15) / 16 <= Rcap)
 			{
 				if (threadIdx.x < 2)
 					smem_d[threadIdx.x] = 0.0;   // read after the first barrier at the earliest
 				ric_coop<PS, NW, NX, AUG>(a, N, nk, smem_d);
 			}
+			else if (DIRECT && least >= 0 && nk + XR <= 128 && (nx <= 64 || (!AUG && nk <= mmax)))
+			{
+				if (wave_id() == 0)
+					ric_beyond<PS, AUG>(a, N, smem_d);
+			}
 		}
-		if (!list)
+		if (DIRECT)
 			return;
 	}
 }

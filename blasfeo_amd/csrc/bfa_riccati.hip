@@ -620,20 +620,19 @@ struct RicStreams
 	}
 };
 
-// One launch of k_ric_coop: the class of R strips (its list), or every instance
-// (lists == nullptr).
-template <int PS, int NW, bool AUG>
-static int launch_coop(int R, int grid, const typename RicArg<AUG>::type *args, int *counts, const int *lists, int batch,
+// One launch of k_ric_coop: the class of R strips (its list), or every instance (DIRECT).
+template <int PS, int NW, bool AUG, bool DIRECT = false>
+static int launch_coop(int R, int grid, const typename RicArg<AUG>::type *args, int mmax, int *counts, const int *lists, int batch,
 	hipStream_t st, const char *name)
 {
 	constexpr int NX = NW == 1 ? 2 : 4;
 	const size_t shm = sizeof(double) * ric_coop_elems(R, NX);
-	if (const int rc = lds_check(reinterpret_cast<const void *>(&k_ric_coop<PS, NW, NX, AUG>), shm, name))
+	if (const int rc = lds_check(reinterpret_cast<const void *>(&k_ric_coop<PS, NW, NX, AUG, DIRECT>), shm, name))
 		return rc;
 	const int cls = R - 1;
-	hipLaunchKernelGGL((k_ric_coop<PS, NW, NX, AUG>), dim3(grid), dim3(NW * WAVE), shm, st, args, R,
-		lists ? counts + cls : (const int *)nullptr, lists ? lists + (size_t)cls * batch : (const int *)nullptr,
-		lists ? counts + RIC_HEAD + cls : (int *)nullptr);
+	hipLaunchKernelGGL((k_ric_coop<PS, NW, NX, AUG, DIRECT>), dim3(grid), dim3(NW * WAVE), shm, st, args, R, mmax,
+		DIRECT ? (const int *)nullptr : counts + cls, DIRECT ? (const int *)nullptr : lists + (size_t)cls * batch,
+		DIRECT ? (int *)nullptr : counts + RIC_HEAD + cls);
 	return check_launch(name);
 }
 
@@ -655,9 +654,9 @@ static int launch_ric_coop(int batch, const typename RicArg<AUG>::type *args, in
 		tuned = tuned || tune_value(TUNE_RIC_THREADS, c) || tune_value(TUNE_RIC_PER_CU, c);
 	const bool direct = resident && !tuned;
 	if (direct && rmax <= 2)
-		return launch_coop<PS, 1, AUG>(rmax, batch, args, nullptr, nullptr, batch, st, name);
+		return launch_coop<PS, 1, AUG, true>(rmax, batch, args, mmax, nullptr, nullptr, batch, st, name);
 	if (direct && batch <= cus)
-		return launch_coop<PS, 4, AUG>(RIC_NCLASS, batch, args, nullptr, nullptr, batch, st, name);
+		return launch_coop<PS, 4, AUG, true>(RIC_NCLASS, batch, args, mmax, nullptr, nullptr, batch, st, name);
 	int *counts = ws;
 	int *lists = ws + 64;
 	hipLaunchKernelGGL(k_ric_zero, dim3(1), dim3(64), 0, st, counts);
@@ -702,11 +701,11 @@ static int launch_ric_coop(int batch, const typename RicArg<AUG>::type *args, in
 			per_cu = v;
 		const int grid = min(batch, R > rmax ? 16 : cus * per_cu);
 		if (nw == 1)
-			rc = launch_coop<PS, 1, AUG>(R, grid, args, counts, lists, batch, sc, name);
+			rc = launch_coop<PS, 1, AUG>(R, grid, args, mmax, counts, lists, batch, sc, name);
 		else if (nw == 2)
-			rc = launch_coop<PS, 2, AUG>(R, grid, args, counts, lists, batch, sc, name);
+			rc = launch_coop<PS, 2, AUG>(R, grid, args, mmax, counts, lists, batch, sc, name);
 		else
-			rc = launch_coop<PS, 4, AUG>(R, grid, args, counts, lists, batch, sc, name);
+			rc = launch_coop<PS, 4, AUG>(R, grid, args, mmax, counts, lists, batch, sc, name);
 	}
 	const int rj = str.join(name);
 	return rc ? rc : rj;

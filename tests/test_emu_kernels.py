@@ -173,3 +173,12 @@ def test_getrf_in_place_two_descriptors(emu_build, op, ps):
 def test_trsm_rltn_several_launches(emu_build, ps):
     """trsm_rltn of a batch whose workgroups pass a launch's limit."""
     run_case("case_trsm.py", "launches", ps)
+
+
+@pytest.mark.parametrize("path", ["direct", "plan", "beyond"])
+@pytest.mark.parametrize("ps", [4, 8])
+@pytest.mark.parametrize("entry", ["trf", "sv"])
+def test_riccati_paths(emu_build, entry, ps, path):
+    """The FP64 Riccati sweep by launch path: direct (one and four waves), planned (one,
+    two and four), and instances larger than the hint on both."""
+    run_case("case_ric_paths.py", entry, path, ps)
