@@ -194,13 +194,16 @@ __device__ __forceinline__ void glu_panel(int R, int cf, int c0, T *P, int ldp, 
 			src[pos[q]] = lane + WAVE * q;
 }
 
-// acc[t] += sum over k < kend (a multiple of 16) of the products of tiles t = 0 .. NT-1.
+// acc[t] = C minus the sum over k < kend (a multiple of 16) of the products of tiles
+// t = 0 .. NT-1; ldc(lane, t, r): element r of C's tile t.  The sum begins at zero and C joins
+// last: begun at C the sum is rounded at C's size in
+// every step, which made the factors' errors 2.4 times as large.
 // COLS: the tiles are 16 rows of L each (ot: the lane's row at column g) and share
 // 16 columns of U (os: the lane's column at row g, rows of U being rows of panels);
 // else the tiles are 16 columns of U each and share 16 rows of L.
-template <typename T, int PS, int NT, bool COLS, typename O>
+template <typename T, int PS, int NT, bool COLS, typename O, typename LDC>
 __device__ __forceinline__ void glu_products(const StripView<T, PS, O> &D, const O (&ot)[4], O os, int di, int kend,
-	typename Vec4<T>::type (&acc)[4])
+	const LDC &ldc, typename Vec4<T>::type (&acc)[4])
 {
 	constexpr unsigned CS = PS * sizeof(T);
 	const int g = lane_id() >> 4;
@@ -225,39 +228,53 @@ __device__ __forceinline__ void glu_products(const StripView<T, PS, O> &D, const
 			for (int i = 0; i < NT; i++)
 				acc[i] = COLS ? mfma16(t[i][u], s[u], acc[i]) : mfma16(s[u], t[i][u], acc[i]);
 	};
-#pragma unroll
-	for (int d = 0; d < GLU_D; d++)
-		load(8 * d, ta[d], sh[d]);
-	int k = 0;
-	for (; k + 8 * GLU_D < kend; k += 8 * GLU_D)
+	static_assert(8 * GLU_D == 16, "kend ends on a whole number of rounds");
+	if (kend > 0)
 	{
 #pragma unroll
 		for (int d = 0; d < GLU_D; d++)
+			load(8 * d, ta[d], sh[d]);
+		for (int k = 0; k + 8 * GLU_D < kend; k += 8 * GLU_D)
 		{
-			step(ta[d], sh[d]);
-			load(k + 8 * (GLU_D + d), ta[d], sh[d]);
-		}
-	}
 #pragma unroll
-	for (int d = 0; d < GLU_D; d++)
-		if (k + 8 * d < kend)
+			for (int d = 0; d < GLU_D; d++)
+			{
+				step(ta[d], sh[d]);
+				load(k + 8 * (GLU_D + d), ta[d], sh[d]);
+			}
+		}
+#pragma unroll
+		for (int d = 0; d < GLU_D; d++)
 			step(ta[d], sh[d]);
+	}
+	// (pinned: C's places are looked up when the operands' registers are free)
+	int lane = lane_id();
+	BFA_PIN(lane);
+	T cv[NT][4];
+#pragma unroll
+	for (int i = 0; i < NT; i++)
+#pragma unroll
+		for (int r = 0; r < 4; r++)
+			cv[i][r] = ldc(lane, i, r);
+#pragma unroll
+	for (int i = 0; i < NT; i++)
+#pragma unroll
+		for (int r = 0; r < 4; r++)
+			acc[i][r] = cv[i][r] - acc[i][r];
 }
 
-template <typename T, int PS, bool COLS, typename O>
+template <typename T, int PS, bool COLS, typename O, typename LDC>
 __device__ __forceinline__ void glu_sum(int nt, const StripView<T, PS, O> &D, const O (&ot)[4], O os, int di, int kend,
-	typename Vec4<T>::type (&acc)[4])
+	const LDC &ldc, typename Vec4<T>::type (&acc)[4])
 {
-	if (kend <= 0)
-		return;
 	if (nt == 4)
-		glu_products<T, PS, 4, COLS>(D, ot, os, di, kend, acc);
+		glu_products<T, PS, 4, COLS>(D, ot, os, di, kend, ldc, acc);
 	else if (nt == 3)
-		glu_products<T, PS, 3, COLS>(D, ot, os, di, kend, acc);
+		glu_products<T, PS, 3, COLS>(D, ot, os, di, kend, ldc, acc);
 	else if (nt == 2)
-		glu_products<T, PS, 2, COLS>(D, ot, os, di, kend, acc);
+		glu_products<T, PS, 2, COLS>(D, ot, os, di, kend, ldc, acc);
 	else if (nt == 1)
-		glu_products<T, PS, 1, COLS>(D, ot, os, di, kend, acc);
+		glu_products<T, PS, 1, COLS>(D, ot, os, di, kend, ldc, acc);
 }
 
 // a wave-uniform offset in a scalar register
@@ -318,26 +335,20 @@ __device__ __forceinline__ void glu_instance(const typename FactArg<T>::type &a,
 			// column panel: row tiles w, w + 4, ... of 16
 			const int nt = min(4, max(0, ((R + 15) / 16 - w + NW - 1) / NW));
 			O ot[4];
-			V4 acc[4];   // products minus C
-			const O pc = (O)(cj + min(c0 + c, n - 1)) * CS;
+			V4 acc[4];
 #pragma unroll
 			for (int t = 0; t < 4; t++)
-			{
-				acc[t] = V4{0, 0, 0, 0};
-				const int i0 = c0 + 16 * (w + NW * t);
-				ot[t] = D.at(di + min(i0 + rid, m - 1), dj + g);
-				if (t < nt)
-#pragma unroll
-					for (int r = 0; r < 4; r++)
-						acc[t][r] = -C.ld(0, C.at(ci + perm[min(i0 + 4 * r + g, m - 1)], 0) + pc);
-			}
-			glu_sum<T, PS, true>(nt, D, ot, (O)(dj + min(c0 + c, n - 1)) * CS, di, c0, acc);
+				acc[t] = V4{0, 0, 0, 0}, ot[t] = D.at(di + min(c0 + 16 * (w + NW * t) + rid, m - 1), dj + g);
+			auto ldc = [&](int l, int t, int r) {
+				return C.ld(0, C.at(ci + perm[min(c0 + 16 * (w + NW * t) + 4 * r + (l >> 4), m - 1)], cj + min(c0 + (l & 15), n - 1)));
+			};
+			glu_sum<T, PS, true>(nt, D, ot, (O)(dj + min(c0 + c, n - 1)) * CS, di, c0, ldc, acc);
 #pragma unroll
 			for (int t = 0; t < 4; t++)
 				if (t < nt)
 #pragma unroll
 					for (int r = 0; r < 4; r++)
-						P[c * LDP + 16 * (w + NW * t) + 4 * r + g] = -acc[t][r];
+						P[c * LDP + 16 * (w + NW * t) + 4 * r + g] = acc[t][r];
 			if (w == 0 && lane == 0)
 				mcount = 0;
 		}
@@ -432,10 +443,6 @@ __device__ __forceinline__ void glu_instance(const typename FactArg<T>::type &a,
 			__syncthreads();
 			BFA_PIN(lane);
 			const int g = lane >> 4, c = lane & 15, rid = strip_row<T>(c);
-			int pr[4];
-#pragma unroll
-			for (int s = 0; s < 4; s++)
-				pr[s] = perm[min(c0 + 4 * s + g, m - 1)];
 			const O os = D.at(di + min(c0 + rid, m - 1), dj + g);
 			const int ntc = (n - c0 - 1) / 16;   // column tiles right of the panel
 #pragma unroll 1
@@ -446,16 +453,11 @@ __device__ __forceinline__ void glu_instance(const typename FactArg<T>::type &a,
 				V4 acc[4];
 #pragma unroll
 				for (int t = 0; t < 4; t++)
-				{
-					acc[t] = V4{0, 0, 0, 0};
-					const int j = min(c0 + 16 * (t0 + NW * t + 1) + c, n - 1);
-					ot[t] = (O)(dj + j) * CS;
-					if (t < nt)
-#pragma unroll
-						for (int s = 0; s < 4; s++)
-							acc[t][s] = -C.ld(0, C.at(ci + pr[s], cj + j));
-				}
-				glu_sum<T, PS, false>(nt, D, ot, os, di, c0, acc);
+					acc[t] = V4{0, 0, 0, 0}, ot[t] = (O)(dj + min(c0 + 16 * (t0 + NW * t + 1) + c, n - 1)) * CS;
+				auto ldc = [&](int l, int t, int s) {
+					return C.ld(0, C.at(ci + perm[min(c0 + 4 * s + (l >> 4), m - 1)], cj + min(c0 + 16 * (t0 + NW * t + 1) + (l & 15), n - 1)));
+				};
+				glu_sum<T, PS, false>(nt, D, ot, os, di, c0, ldc, acc);
 				// the factored diagonal block for strip_solve; its 4 x 4 triangles
 				// with unit reciprocals
 				T l[3], d[4];
@@ -471,7 +473,7 @@ __device__ __forceinline__ void glu_instance(const typename FactArg<T>::type &a,
 					if (t < nt)
 					{
 						T x[4];
-						strip_solve<T>(-acc[t], l, d, x);
+						strip_solve<T>(acc[t], l, d, x);
 						const int j = c0 + 16 * (t0 + NW * t + 1) + c;
 #pragma unroll
 						for (int s = 0; s < 4; s++)

@@ -182,3 +182,9 @@ def test_riccati_paths(emu_build, entry, ps, path):
     """The FP64 Riccati sweep by launch path: direct (one and four waves), planned (one,
     two and four), and instances larger than the hint on both."""
     run_case("case_ric_paths.py", entry, path, ps)
+
+
+@pytest.mark.parametrize("op", ["getrf"])
+def test_rounding_error(emu_build, op):
+    """Errors against extended precision no larger than with every sum begun at zero."""
+    run_case("case_err.py", op)
