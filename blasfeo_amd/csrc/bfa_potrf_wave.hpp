@@ -3,6 +3,7 @@
 // few that share its strips.
 #pragma once
 #include "bfa_strip.hpp"
+#include <type_traits>
 
 namespace bfa {
 
@@ -189,6 +190,16 @@ __device__ __forceinline__ void potrf_coop(int m, int n, int k, const StripView<
 	const int ih = R - 1 - w, il = R - 2 * NW + w;
 	const int rh = min(16 * max(ih, 0) + rid, m - 1), rl = min(16 * max(il, 0) + rid, m - 1);
 	V4 hi[2 * NW], lo[NW];
+	if (SYRK)
+	{
+#pragma unroll
+		for (int J = 0; J < 2 * NW; J++)
+			hi[J] = V4{0, 0, 0, 0};
+#pragma unroll
+		for (int J = 0; J < NW; J++)
+			lo[J] = V4{0, 0, 0, 0};
+	}
+	else
 	{
 		const size_t oh = C.at(ci + rh, cj + g), ol = C.at(ci + rl, cj + g);
 #pragma unroll
@@ -271,6 +282,39 @@ __device__ __forceinline__ void potrf_coop(int m, int n, int k, const StripView<
 							lo[J < NW ? J : 0] = mfma16(b[s], cl[s], lo[J < NW ? J : 0]);
 				}
 		}
+	}
+	if (SYRK)
+	{
+		// C joins last, four tiles at a time with no branch between their loads (columns
+		// past n read column n - 1): sums begun at C are rounded at C's size in every
+		// step, which made the factors' errors up to 1.7 times as large
+		int ge = g, re = rid;
+		BFA_PIN(ge);
+		BFA_PIN(re);
+		auto add = [&](int I, int J0, auto &acc, auto cnt) {
+			constexpr int CNT = decltype(cnt)::value;
+			if (J0 > I || J0 >= Cb)
+				return;
+			const size_t o = C.at(ci + min(16 * I + re, m - 1), cj);
+			T cv[CNT][4];
+#pragma unroll
+			for (int t = 0; t < CNT; t++)
+#pragma unroll
+				for (int s = 0; s < 4; s++)
+					cv[t][s] = C.ld(0, o + (size_t)((unsigned)min(16 * (J0 + t) + 4 * s + ge, n - 1) * CS));
+#pragma unroll
+			for (int t = 0; t < CNT; t++)
+#pragma unroll
+				for (int s = 0; s < 4; s++)
+					acc[J0 + t][s] += cv[t][s];
+		};
+		typedef std::integral_constant<int, NW < 4 ? NW : 4> Cnt;
+#pragma unroll
+		for (int J = 0; J < 2 * NW; J += Cnt::value)
+			add(ih, J, hi, Cnt());
+#pragma unroll
+		for (int J = 0; J < NW; J += Cnt::value)
+			add(il, J, lo, Cnt());
 		// the first column's tiles go to the buffer that the last chunk may still
 		// be read from
 		__syncthreads();

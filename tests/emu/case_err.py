@@ -3,7 +3,7 @@ extended precision, beside those of the same factorisation in numpy's float64 wi
 finished blocks' products summed from zero and the matrix element joined last.  A sum begun at the
 element is rounded at the element's size in every step, and on these inputs the errors
 are then more than twice as large; 1.25 leaves room for the order of the sums.
-Usage: python case_err.py <getrf>"""
+Usage: python case_err.py <getrf | syrk_dpotrf>"""
 import ctypes
 import sys
 
@@ -74,6 +74,34 @@ def run_getrf(E):
         exact = lu(B.astype(np.longdouble))
         kernel.append(rms(get(D, n, n), exact))
         plain.append(rms(lu(B), exact))
+    return kernel, plain
+
+
+def chol(A):
+    A, n = A.copy(), len(A)
+    for j in range(n):
+        A[j:, j] *= A.dtype.type(1) / np.sqrt(A[j, j])
+        A[j + 1:, j + 1:] -= np.outer(A[j + 1:, j], A[j + 1:, j])
+    return np.tril(A)
+
+
+def spd(rng, n):
+    B = rng.standard_normal((n, n))
+    return B @ B.T / n + np.eye(n)
+
+
+def run_syrk_dpotrf(E):
+    rng = np.random.default_rng(6)
+    kernel, plain = [], []
+    for n in (32, 64, 90, 128):
+        C, A = 10 * spd(rng, n), 0.1 * rng.standard_normal((n, n))
+        a, D = mat(A), mat(np.zeros((n, n)))
+        print("emu error of dsyrk_dpotrf_ln n=%d" % n, flush=True)
+        call(E, "dsyrk_dpotrf_ln", bfa.DSYRK_DPOTRF_ARG, [dict(m=n, n=n, k=n, sA=a, sB=a, sC=mat(C), sD=D)], (n, n, n))
+        X = A.astype(np.longdouble)
+        exact = chol(C.astype(np.longdouble) + products(X, X.T))
+        kernel.append(rms(np.tril(get(D, n, n)), exact))
+        plain.append(rms(chol(C + products(A, A.T)), exact))
     return kernel, plain
 
 
