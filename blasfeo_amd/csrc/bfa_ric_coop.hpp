@@ -339,14 +339,16 @@ __device__ __forceinline__ void ric_coop(const RicRec &a, int N, int nkmax, doub
 					}
 			}
 			__syncthreads();
-			// M_IJ += W_I W_J^T
+			// M_IJ += W_I W_J^T, a tile's products summed from zero (begun at RSQ they
+			// are rounded at its size in every step)
 #pragma unroll
-			for (int C = 0; C < NX; C++)
-				if (C < n1t)
+			for (int J = 0; J < 2 * NW; J++)
+				if (J <= ih && J < Cb)
 				{
+					V4 ah = V4{0, 0, 0, 0}, al = V4{0, 0, 0, 0};
 #pragma unroll
-					for (int J = 0; J < 2 * NW; J++)
-						if (J <= ih && J < Cb)
+					for (int C = 0; C < NX; C++)
+						if (C < n1t)
 						{
 							double x[4];
 							if (J == R - 1)
@@ -359,12 +361,15 @@ __device__ __forceinline__ void ric_coop(const RicRec &a, int N, int nkmax, doub
 									x[s] = W[256 * (J * NX + C) + 64 * s + lane];
 #pragma unroll
 							for (int s = 0; s < 4; s++)
-								hi[J] = mfma16(x[s], bh[C][s], hi[J]);
+								ah = mfma16(x[s], bh[C][s], ah);
 							if (J < NW && J <= il)
 #pragma unroll
 								for (int s = 0; s < 4; s++)
-									lo[J < NW ? J : 0] = mfma16(x[s], bl[C][s], lo[J < NW ? J : 0]);
+									al = mfma16(x[s], bl[C][s], al);
 						}
+					hi[J] += ah;
+					if (J < NW && J <= il)
+						lo[J < NW ? J : 0] += al;
 				}
 		}
 		// the next stage's descriptors and strips of BAbt, loaded beside the Cholesky

@@ -3,7 +3,7 @@ extended precision, beside those of the same factorisation in numpy's float64 wi
 finished blocks' products summed from zero and the matrix element joined last.  A sum begun at the
 element is rounded at the element's size in every step, and on these inputs the errors
 are then more than twice as large; 1.25 leaves room for the order of the sums.
-Usage: python case_err.py <getrf | syrk_dpotrf>"""
+Usage: python case_err.py <getrf | syrk_dpotrf | riccati>"""
 import ctypes
 import sys
 
@@ -102,6 +102,38 @@ def run_syrk_dpotrf(E):
         exact = chol(C.astype(np.longdouble) + products(X, X.T))
         kernel.append(rms(np.tril(get(D, n, n)), exact))
         plain.append(rms(chol(C + products(A, A.T)), exact))
+    return kernel, plain
+
+
+class Table:
+    """An array in its own block, as a field of a record."""
+
+    def __init__(self, a):
+        self.desc = Block(a.nbytes)
+        self.desc.write(a)
+
+
+def run_riccati(E):
+    """One stage, RSQ large beside W W^T: the factor of stage 0."""
+    rng = np.random.default_rng(7)
+    kernel, plain = [], []
+    for nx, nu in ((20, 6), (40, 12), (64, 20), (64, 60)):
+        n = nx + nu
+        BA, R, Q = 0.1 * rng.standard_normal((n, nx)), 10 * spd(rng, n), spd(rng, nx)
+        b, r, q, l0, l1, w = (mat(M) for M in (BA, R, Q, np.zeros((n, n)), np.zeros((nx, nx)), np.zeros((n, nx))))
+        desc = lambda *ms: Table(np.concatenate([m.desc.read(bfa.DMAT) for m in ms]))  # noqa: E731
+        print("emu error of d_back_ric_trf nx=%d nu=%d" % (nx, nu), flush=True)
+        call(E, "d_back_ric_trf", bfa.RICCATI_ARG,
+             [dict(N=1, nx=Table(np.array([nx, nx], np.int32)).desc.addr, nu=Table(np.array([nu, 0], np.int32)).desc.addr,
+                   BAbt=desc(b).desc.addr, RSQrq=desc(r, q).desc.addr, L=desc(l0, l1).desc.addr, work=w)], (n, nx, 0))
+        for f, out in ((np.longdouble, None), (np.float64, plain)):
+            W = products(BA.astype(f), chol(Q.astype(f)))
+            L = chol(R.astype(f) + products(W, W.T))
+            if out is None:
+                exact = L
+            else:
+                out.append(rms(L, exact))
+        kernel.append(rms(np.tril(get(l0, n, n)), exact))
     return kernel, plain
 
 

@@ -184,7 +184,7 @@ def test_riccati_paths(emu_build, entry, ps, path):
     run_case("case_ric_paths.py", entry, path, ps)
 
 
-@pytest.mark.parametrize("op", ["getrf", "syrk_dpotrf"])
+@pytest.mark.parametrize("op", ["getrf", "syrk_dpotrf", "riccati"])
 def test_rounding_error(emu_build, op):
     """Errors against extended precision no larger than with every sum begun at zero."""
     run_case("case_err.py", op)
