@@ -477,7 +477,7 @@ static int launch_gemm_ps(int batch, const typename GemmArg<T>::type *args, cons
 	// The large tile reads a quarter of the operands that the small one reads per
 	// product but leaves a batch of few or uneven instances with too few waves.
 	// It is taken above 256 rows or columns (64 dgemm_nn of 512: 270 us against 348,
-	// 16 of them 74 against 120), without bounds, and above 128 (FP32 96) where the
+	// 16 of them 74 against 120), and above 128 (FP32 96) where the
 	// batch has 16384 of its tiles (4096 dgemm_nt + dsyrk_ln of U{16..256}: 1052
 	// against 1132 us, 512 of them 219 against 180; 4096 of 128: 738 against 788, of
 	// U{4..128} 260 against 229; 4096 FP32 of U{4..128} 157 against 166, of U{4..96}
@@ -485,6 +485,19 @@ static int launch_gemm_ps(int batch, const typename GemmArg<T>::type *args, cons
 	const int knob = tune_value(TUNE_GEMM_WAVE, 0);
 	const int slots = gemm_slots<OP>(hint, 64);
 	const int maxm = hint ? hint->max_m : 0, maxn = OP == OP_SYRK ? maxm : hint ? hint->max_n : 0;
+	// A bound missing: small tiles, and as many slots per instance as make 65536 waves of
+	// the batch, 4 to 64 (dgemm_nt, us, against one slot of large tiles and the four
+	// waves of the 64 x 64 LDS tile before them: one of 1024 737, 30957, 20992; one of 64
+	// 5.9, 12.6, 10.2; 64 of 512 343, 4049, 2785; 512 of U{16..256} 94, 519, 409; 4096
+	// 791, 1215, 1337; 2048 of 64 49, 44, 57; 65536 of U{4..32} 176, 231, 623).  Large
+	// tiles with as many slots are up to 1.5 times faster on the largest and up to 5
+	// times slower on the smallest.
+	if (knob == 0 && (maxm <= 0 || maxn <= 0))
+	{
+		const int cap = tune_value(TUNE_GEMM_GRID_Y, 0);
+		const int s = min(cap > 0 ? cap : 64, max(4, min(64, 65536 / batch)));
+		return launch_gemm_tile<T, PS, OP, 2>(batch, args, s, st, name);
+	}
 	const int most = maxm > 0 && maxn > 0 ? max(maxm, maxn) : 512;
 	const bool large = most > 256 || (most > (sizeof(T) == 8 ? 128 : 96) && (long long)batch * slots >= 16384);
 	if (knob == 2 || (knob == 0 && large))
