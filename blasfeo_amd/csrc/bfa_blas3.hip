@@ -224,13 +224,14 @@ __global__ __launch_bounds__(NT3) void k_trsm_left(const typename TrsmArg<T>::ty
 constexpr int THIN_RHS = 4;
 constexpr int THIN_Q = 4;
 
-template <typename T, int PS, int MODE, typename O>
+template <typename T, int PS, int MODE, int Q>
 __device__ __forceinline__ void trsm_thin(const typename TrsmArg<T>::type &a, int m, int nrhs, const StripView<T, PS> &vA,
 	const StripView<T, PS> &vB, const StripView<T, PS> &vD)
 {
 	constexpr bool BACK = tl_back(MODE);
 	constexpr bool UNIT = MODE == TL_LLNU;
 	constexpr unsigned CS = PS * sizeof(T);
+	typedef unsigned O;
 	int ai = a.ai, aj = a.aj, bi = a.bi, bj = a.bj, di = a.di, dj = a.dj;
 	const StripView<T, PS, O> A = vA.template block<O>(ai, aj), B = vB.template block<O>(bi, bj), D = vD.template block<O>(di, dj);
 	const int lane = threadIdx.x;
@@ -238,10 +239,10 @@ __device__ __forceinline__ void trsm_thin(const typename TrsmArg<T>::type &a, in
 	const BFA_GLOBAL T *dA = (const BFA_GLOBAL T *)a.sA->dA;
 	// this lane's rows of A (lltn: columns; rows past the end read the last one)
 	// and their reciprocal diagonals
-	O oa[THIN_Q];
-	T rd[THIN_Q];
+	O oa[Q];
+	T rd[Q];
 #pragma unroll
-	for (int q = 0; q < THIN_Q; q++)
+	for (int q = 0; q < Q; q++)
 		if (q * WAVE < m)
 		{
 			const int i = min(lane + q * WAVE, m - 1);
@@ -249,9 +250,9 @@ __device__ __forceinline__ void trsm_thin(const typename TrsmArg<T>::type &a, in
 			rd[q] = UNIT ? T(1) : cached ? dA[i] : T(1) / A.ld(0, A.at(ai + i, aj + i));
 		}
 	// columns j0 .. j0+3 of the solve, slots q0 .. q1-1
-	auto coef = [&](int j0, int q0, int q1, T (&e)[THIN_Q][4]) {
+	auto coef = [&](int j0, int q0, int q1, T (&e)[Q][4]) {
 #pragma unroll
-		for (int q = 0; q < THIN_Q; q++)
+		for (int q = 0; q < Q; q++)
 			if (q >= q0 && q < q1 && q * WAVE < m)
 #pragma unroll
 				for (int t = 0; t < 4; t++)
@@ -264,23 +265,27 @@ __device__ __forceinline__ void trsm_thin(const typename TrsmArg<T>::type &a, in
 	for (int c0 = 0; c0 < nrhs; c0 += THIN_RHS)
 	{
 		const int n = min(THIN_RHS, nrhs - c0);
-		T x[THIN_Q][THIN_RHS];
+		// (pinned, here and at the end: the rows' offsets in B and D, the same for every
+		// group, would be kept in registers across the sweep)
+		int lb0 = lane;
+		BFA_PIN(lb0);
+		T x[Q][THIN_RHS];
 #pragma unroll
-		for (int q = 0; q < THIN_Q; q++)
+		for (int q = 0; q < Q; q++)
 #pragma unroll
 			for (int c = 0; c < THIN_RHS; c++)
 			{
-				const int i = lane + q * WAVE;
+				const int i = lb0 + q * WAVE;
 				x[q][c] = (i < m && c < n) ? a.alpha * B.ld(0, B.at(bi + i, bj + c0 + c)) : T(0);
 			}
-		T e[THIN_Q][4];
-		coef(BACK ? (m - 1) & ~3 : 0, 0, THIN_Q, e);
+		T e[Q][4];
+		coef(BACK ? (m - 1) & ~3 : 0, 0, Q, e);
 		// grouped by the register slot qb = j / 64 that holds row j (unrolled, so
 		// that every register index is a constant)
 #pragma unroll
-		for (int qq = 0; qq < THIN_Q; qq++)
+		for (int qq = 0; qq < Q; qq++)
 		{
-			const int qb = BACK ? THIN_Q - 1 - qq : qq;
+			const int qb = BACK ? Q - 1 - qq : qq;
 #pragma unroll 1
 			for (int l4 = 0; l4 < WAVE; l4 += 4)
 			{
@@ -292,9 +297,9 @@ __device__ __forceinline__ void trsm_thin(const typename TrsmArg<T>::type &a, in
 						continue;
 					break;
 				}
-				T en[THIN_Q][4];
+				T en[Q][4];
 				if (BACK ? j0 > 0 : j0 + 4 < m)
-					coef(BACK ? j0 - 4 : j0 + 4, BACK ? 0 : qb, BACK ? qb + 1 : THIN_Q, en);
+					coef(BACK ? j0 - 4 : j0 + 4, BACK ? 0 : qb, BACK ? qb + 1 : Q, en);
 #pragma unroll
 				for (int tt = 0; tt < 4; tt++)
 				{
@@ -313,7 +318,7 @@ __device__ __forceinline__ void trsm_thin(const typename TrsmArg<T>::type &a, in
 						// value, scaled by its reciprocal after the sweep
 						const bool open = BACK ? lane < lb + t : lane > lb + t;
 #pragma unroll
-						for (int q = 0; q < THIN_Q; q++)
+						for (int q = 0; q < Q; q++)
 						{
 							if (BACK ? q > qb : q < qb)
 								continue;
@@ -329,7 +334,7 @@ __device__ __forceinline__ void trsm_thin(const typename TrsmArg<T>::type &a, in
 					}
 				}
 #pragma unroll
-				for (int q = 0; q < THIN_Q; q++)
+				for (int q = 0; q < Q; q++)
 #pragma unroll
 					for (int t = 0; t < 4; t++)
 						e[q][t] = en[q][t];
@@ -337,10 +342,12 @@ __device__ __forceinline__ void trsm_thin(const typename TrsmArg<T>::type &a, in
 		}
 		// row i's solved value is its unscaled value times the reciprocal the
 		// sweep used for column i (the same product the broadcast formed)
+		int ld0 = lane;
+		BFA_PIN(ld0);
 #pragma unroll
-		for (int q = 0; q < THIN_Q; q++)
+		for (int q = 0; q < Q; q++)
 		{
-			const int i = lane + q * WAVE;
+			const int i = ld0 + q * WAVE;
 			if (i < m)
 #pragma unroll
 				for (int c = 0; c < THIN_RHS; c++)
@@ -350,18 +357,61 @@ __device__ __forceinline__ void trsm_thin(const typename TrsmArg<T>::type &a, in
 	}
 }
 
+// The same with X in D, for panel strides too large for 32-bit offsets and for instances
+// larger than the launch's slots.  (With 64-bit offsets the code above spills, and
+// scratch costs the launches of small instances that never use it: 16384 of 24 rows
+// 45 -> 66 us.)
 template <typename T, int PS, int MODE>
-__global__ __launch_bounds__(WAVE, 4) void k_trsm_left_thin(const typename TrsmArg<T>::type *__restrict__ args)
+__device__ __forceinline__ void trsm_thin_wide(const typename TrsmArg<T>::type &a, int m, int nrhs, const StripView<T, PS> &A,
+	const StripView<T, PS> &B, const StripView<T, PS> &D)
+{
+	constexpr bool BACK = tl_back(MODE), UNIT = MODE == TL_LLNU;
+	const int lane = threadIdx.x;
+	const bool cached = !UNIT && a.ai == 0 && a.aj == 0 && a.sD != a.sA && a.sA->use_dA >= m;
+	const BFA_GLOBAL T *dA = (const BFA_GLOBAL T *)a.sA->dA;
+#pragma unroll 1
+	for (int c = 0; c < nrhs; c++)
+	{
+#pragma unroll 1
+		for (int i = lane; i < m; i += WAVE)
+			D.st(0, D.at(a.di + i, a.dj + c), a.alpha * B.ld(0, B.at(a.bi + i, a.bj + c)));
+		wave_sync();
+#pragma unroll 1
+		for (int t = 0; t < m; t++)
+		{
+			const int j = BACK ? m - 1 - t : t;
+			const size_t oj = D.at(a.di + j, a.dj + c);
+			const T d = UNIT ? T(1) : cached ? dA[j] : T(1) / A.ld(0, A.at(a.ai + j, a.aj + j));
+			const T x = D.ld(0, oj) * d;
+			wave_sync();   // every lane has read row j
+			if (lane == 0)
+				D.st(0, oj, x);
+#pragma unroll 1
+			for (int i = (BACK ? 0 : j + 1) + lane; i < (BACK ? j : m); i += WAVE)
+			{
+				const size_t o = D.at(a.di + i, a.dj + c);
+				D.st(0, o, D.ld(0, o) - A.ld(0, MODE == TL_LLTN ? A.at(a.ai + j, a.aj + i) : A.at(a.ai + i, a.aj + j)) * x);
+			}
+			wave_sync();
+		}
+	}
+}
+
+// Q: the row slots that the hint's bound asks for.  Each form is compiled for as many waves
+// as leave it without scratch (with four slots for every bound 16384 dtrsm_lunn of
+// U{4..64} took 120 us, the column at a time before it 113, one and two slots 73).
+template <typename T, int PS, int MODE, int Q>
+__global__ __launch_bounds__(WAVE, Q == 4 ? 3 : 4) void k_trsm_left_thin(const typename TrsmArg<T>::type *__restrict__ args)
 {
 	const typename TrsmArg<T>::type &a = args[blockIdx.x];
 	const int m = __builtin_amdgcn_readfirstlane(a.m), nrhs = __builtin_amdgcn_readfirstlane(a.n);
 	if (m <= 0 || nrhs <= 0 || m > THIN_Q * WAVE)
 		return;
 	const StripView<T, PS> A = strip_view<T, PS>(a.sA), B = strip_view<T, PS>(a.sB), D = strip_view<T, PS>(a.sD);
-	if (__builtin_expect(strip_fits<T, PS>(max(A.cn, max(B.cn, D.cn))), 1))
-		trsm_thin<T, PS, MODE, unsigned>(a, m, nrhs, A, B, D);
+	if (__builtin_expect(m <= Q * WAVE && strip_fits<T, PS>(max(A.cn, max(B.cn, D.cn))), 1))
+		trsm_thin<T, PS, MODE, Q>(a, m, nrhs, A, B, D);
 	else
-		trsm_thin<T, PS, MODE, size_t>(a, m, nrhs, A, B, D);
+		trsm_thin_wide<T, PS, MODE>(a, m, nrhs, A, B, D);
 }
 
 // Cache update after trsm_rltn / trsm_llnn / trsm_lltn, in the reference's
@@ -610,8 +660,12 @@ static int launch_trsm(int ps, int batch, const typename TrsmArg<T>::type *args,
 template <typename T, int PS, int MODE>
 static int launch_trsml_ps(int batch, const typename TrsmArg<T>::type *args, dim3 grid, size_t shm, int mmax, bool thin, hipStream_t st, const char *name)
 {
-	if (thin)
-		hipLaunchKernelGGL((k_trsm_left_thin<T, PS, MODE>), dim3(batch), dim3(WAVE), 0, st, args);
+	if (thin && mmax <= WAVE)
+		hipLaunchKernelGGL((k_trsm_left_thin<T, PS, MODE, 1>), dim3(batch), dim3(WAVE), 0, st, args);
+	else if (thin && mmax <= 2 * WAVE)
+		hipLaunchKernelGGL((k_trsm_left_thin<T, PS, MODE, 2>), dim3(batch), dim3(WAVE), 0, st, args);
+	else if (thin)
+		hipLaunchKernelGGL((k_trsm_left_thin<T, PS, MODE, 4>), dim3(batch), dim3(WAVE), 0, st, args);
 	else
 		hipLaunchKernelGGL((k_trsm_left<T, PS, MODE>), grid, dim3(NT3), shm, st, args, mmax);
 	int rc = check_launch(name);

@@ -46,11 +46,12 @@ constexpr int trsm_waves()
 // DA_GIVEN: the reciprocal diagonal is read from sA->dA whatever use_dA says
 // (the trapezoid Cholesky, whose diagonal block was just factored into the same
 // descriptor with its reciprocals stored there).
-template <typename T, int PS, int NB, bool DA_GIVEN, typename O>
+template <typename T, int PS, int NB, bool DA_GIVEN>
 __device__ __forceinline__ void trsm_rows(const typename TrsmArg<T>::type &a, int m, int n, const StripView<T, PS> &vA,
 	const StripView<T, PS> &vB, const StripView<T, PS> &vD, int slot, int slots, T *tiles, T *inv_s)
 {
 	typedef typename Vec4<T>::type V4;
+	typedef unsigned O;
 	constexpr int S = trsm_strips<NB>(), NW = NT3 / WAVE, NT = NB / NW;
 	int ai = a.ai, aj = a.aj;
 	const StripView<T, PS, O> A = vA.template block<O>(ai, aj);
@@ -277,6 +278,30 @@ __device__ __forceinline__ void trsm_rows(const typename TrsmArg<T>::type &a, in
 	}
 }
 
+// The rows r0 .. r0+rows-1 and every step-th such block of an instance whose panel strides
+// are too large for 32-bit offsets: a thread per row, finished columns read back
+// from D.  (The code above with 64-bit offsets spills, and scratch costs the launches
+// of small instances that never use it.)
+template <typename T, int PS, bool DA_GIVEN>
+__device__ __forceinline__ void trsm_rows_wide(const typename TrsmArg<T>::type &a, int m, int n, const StripView<T, PS> &A,
+	const StripView<T, PS> &B, const StripView<T, PS> &D, int r0, int rows, int step)
+{
+	const bool cached = DA_GIVEN || (a.ai == 0 && a.aj == 0 && a.sD != a.sA && a.sA->use_dA >= n);
+	const BFA_GLOBAL T *dA = (const BFA_GLOBAL T *)a.sA->dA;
+	for (; r0 < m; r0 += step)
+		for (int i = r0 + threadIdx.x; i < min(m, r0 + rows); i += NT3)
+#pragma unroll 1
+			for (int j = 0; j < n; j++)
+			{
+				T w = T(0);
+#pragma unroll 1
+				for (int l = 0; l < j; l++)
+					w += D.ld(0, D.at(a.di + i, a.dj + l)) * A.ld(0, A.at(a.ai + j, a.aj + l));
+				const T d = cached ? dA[j] : T(1) / A.ld(0, A.at(a.ai + j, a.aj + j));
+				D.st(0, D.at(a.di + i, a.dj + j), (a.alpha * B.ld(0, B.at(a.bi + i, a.bj + j)) - w) * d);
+			}
+}
+
 template <typename T, int PS, int NB, bool DA_GIVEN>
 __global__ __launch_bounds__(NT3, (trsm_waves<T, NB>())) void k_trsm_rltn(const typename TrsmArg<T>::type *__restrict__ args,
 	int batch, int slots, int nlo, int nmax)
@@ -294,9 +319,9 @@ __global__ __launch_bounds__(NT3, (trsm_waves<T, NB>())) void k_trsm_rltn(const 
 		return;
 	const StripView<T, PS> A = strip_view<T, PS>(a.sA), B = strip_view<T, PS>(a.sB), D = strip_view<T, PS>(a.sD);
 	if (__builtin_expect(strip_fits<T, PS>(max(A.cn, max(B.cn, D.cn))), 1))
-		trsm_rows<T, PS, NB, DA_GIVEN, unsigned>(a, m, n, A, B, D, slot, slots, tiles, inv_s);
+		trsm_rows<T, PS, NB, DA_GIVEN>(a, m, n, A, B, D, slot, slots, tiles, inv_s);
 	else
-		trsm_rows<T, PS, NB, DA_GIVEN, size_t>(a, m, n, A, B, D, slot, slots, tiles, inv_s);
+		trsm_rows_wide<T, PS, DA_GIVEN>(a, m, n, A, B, D, slot * 64 * trsm_strips<NB>(), 64 * trsm_strips<NB>(), slots * 64 * trsm_strips<NB>());
 }
 
 } // namespace bfa

@@ -3,6 +3,8 @@ record sets of the GPU tests (tests/trsm_cases.py), checked against the
 oracle element for element (NaN and Inf included).
 Usage: python case_trsm.py nonfinite <op> <thin: 0|1>
        python case_trsm.py rltn <ps> <finite: 0|1>   (trsm_rltn, trsm_cases.rltn)
+       python case_trsm.py slots <op> <bound>   (one wave per instance with the row slots of
+           the bound; the instances beyond it take the form of any size)
        python case_trsm.py launches <ps>   (the same with a bound of 4096 rows: an instance
            a launch under the emulator's limit of a launch's threads)"""
 import ctypes
@@ -45,7 +47,11 @@ def check(E, op, ps, cases, hint):
 
 
 if __name__ == "__main__":
-    if sys.argv[1] == "launches":
+    if sys.argv[1] == "slots":
+        lib = emu_lib("emu_lapack")
+        assert lib.blasfeo_amd_tune_set(b"trsm_thin", 0, 1) == 0
+        check(lib, sys.argv[2], 4, trsm_cases.nonfinite(4, sys.argv[2], 985), (int(sys.argv[3]), 4, 0))
+    elif sys.argv[1] == "launches":
         check(emu_lib("emu_lapack"), "trsm_rltn", int(sys.argv[2]), trsm_cases.rltn(int(sys.argv[2]), 995, True), (4096, 256, 0))
     elif sys.argv[1] == "rltn":
         psz, fin = int(sys.argv[2]), int(sys.argv[3])

@@ -188,3 +188,11 @@ def test_riccati_paths(emu_build, entry, ps, path):
 def test_rounding_error(emu_build, op):
     """Errors against extended precision no larger than with every sum begun at zero."""
     run_case("case_err.py", op)
+
+
+@pytest.mark.parametrize("bound", [64, 128])
+@pytest.mark.parametrize("op", ["trsm_llnn", "trsm_lltn", "trsm_llnu", "trsm_lunn"])
+def test_trsm_left_slots(emu_build, op, bound):
+    """The one-wavefront left solves with one and two row slots, Inf and NaN included; the
+    instances larger than the bound are solved too."""
+    run_case("case_trsm.py", "slots", op, bound)
