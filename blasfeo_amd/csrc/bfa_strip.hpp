@@ -30,6 +30,13 @@
 #define BFA_PIN(x) asm volatile("" : "+v"(x))
 #endif
 
+// Wants these wave-uniform values, each as "s"(x), in scalar registers here: their loads
+// from the argument record are then issued together before this point, not waited for
+// one by one after the next branches.
+#ifndef BFA_NEED
+#define BFA_NEED(...) asm volatile("" : : __VA_ARGS__)
+#endif
+
 namespace bfa {
 
 // A panel-major matrix as the strip kernels address it: a wave-uniform base and byte

@@ -58,8 +58,10 @@ __device__ __forceinline__ void trsm_rows(const typename TrsmArg<T>::type &a, in
 	const T alpha = a.alpha;
 	// reciprocal diagonal: cached copy when valid at launch, else 1/A_jj
 	// (an output aliasing A invalidates the cache first, as in the reference)
-	const bool cached = DA_GIVEN || (a.ai == 0 && a.aj == 0 && a.sD != a.sA && a.sA->use_dA >= n);
-	const BFA_GLOBAL T *dA = (const BFA_GLOBAL T *)a.sA->dA;
+	// (through global-memory pointers: a wait for flat loads waits for LDS as well)
+	const BFA_GLOBAL typename MatOf<T>::type *sA = (const BFA_GLOBAL typename MatOf<T>::type *)a.sA;
+	const bool cached = DA_GIVEN || (a.ai == 0 && a.aj == 0 && a.sD != a.sA && sA->use_dA >= n);
+	const BFA_GLOBAL T *dA = (const BFA_GLOBAL T *)sA->dA;
 	for (int j = threadIdx.x; j < 16 * NB; j += NT3)
 		inv_s[j] = j < n ? (cached ? dA[j] : T(1) / A.ld(0, A.at(ai + j, aj + j))) : T(0);
 	const int w = __builtin_amdgcn_readfirstlane(wave_id());
@@ -318,6 +320,7 @@ __global__ __launch_bounds__(NT3, (trsm_waves<T, NB>())) void k_trsm_rltn(const 
 	if (m <= 0 || n <= nlo || n > nmax || n > 16 * NB || slot * 64 * trsm_strips<NB>() >= m)
 		return;
 	const StripView<T, PS> A = strip_view<T, PS>(a.sA), B = strip_view<T, PS>(a.sB), D = strip_view<T, PS>(a.sD);
+	BFA_NEED("s"(a.ai), "s"(a.aj), "s"(a.bi), "s"(a.bj), "s"(a.di), "s"(a.dj), "s"(a.alpha));
 	if (__builtin_expect(strip_fits<T, PS>(max(A.cn, max(B.cn, D.cn))), 1))
 		trsm_rows<T, PS, NB, DA_GIVEN>(a, m, n, A, B, D, slot, slots, tiles, inv_s);
 	else
