@@ -34,10 +34,12 @@ def ric_footprint(nkmax, nxmax):
     return ((nkt * (nkt + 1) // 2 + nkt * nxt) * _RT_SZ + nkt * 16) * 8 + 16
 
 
-def ric_strip_class(nkmax, nxmax):
+def ric_strip_class(nkmax, nxmax, aug=False):
     """Class of an instance of the FP64 sweep: the 16-row strips of its largest
-    stage, less one (0..7), or 8 for the global-memory sweep."""
-    return 8 if nxmax > 64 or nkmax > 128 else max(0, (nkmax + 15) // 16 - 1)
+    stage (aug: with the extra row of the fused factorisation and solve), less one
+    (0..7), or 8 for the global-memory sweep."""
+    rows = nkmax + (1 if aug else 0)
+    return 8 if nxmax > 64 or rows > 128 else max(0, (rows + 15) // 16 - 1)
 
 
 def ric_strip_lds(cls, nt):

@@ -648,9 +648,9 @@ static int launch_ric_coop(int batch, const typename RicArg<AUG>::type *args, in
 	// No plan where one launch serves every instance: a batch that gives no CU
 	// more than one (four waves each, the LDS of the largest size), and sizes of
 	// up to 32 rows (one wave each, their LDS differs little).  The tuning knobs
-	// shape the class launches.
+	// shape the class launches: a knob of a class that the hint admits asks for them.
 	bool tuned = false;
-	for (int c = 0; c < RIC_NCLASS; c++)
+	for (int c = 0; c < rmax; c++)
 		tuned = tuned || tune_value(TUNE_RIC_THREADS, c) || tune_value(TUNE_RIC_PER_CU, c);
 	const bool direct = resident && !tuned;
 	if (direct && rmax <= 2)
@@ -691,13 +691,13 @@ static int launch_ric_coop(int batch, const typename RicArg<AUG>::type *args, in
 		if (R > rmax && R < RIC_NCLASS)
 			continue;
 		int nw = R <= 2 ? 1 : R <= 4 ? 2 : 4;
-		if (const int v = tune_value(TUNE_RIC_THREADS, R - 1))
+		if (const int v = R <= rmax ? tune_value(TUNE_RIC_THREADS, R - 1) : 0)
 			if (v / WAVE * 2 >= R)
 				nw = v / WAVE;
 		// as many workgroups as the registers and the LDS of a CU hold
 		const int lds = (int)sizeof(double) * ric_coop_elems(R, nw == 1 ? 2 : 4);
 		int per_cu = max(1, min(4 * ric_coop_waves(nw) / nw, RIC_LDS_MAX / lds));
-		if (const int v = tune_value(TUNE_RIC_PER_CU, R - 1))
+		if (const int v = R <= rmax ? tune_value(TUNE_RIC_PER_CU, R - 1) : 0)
 			per_cu = v;
 		const int grid = min(batch, R > rmax ? 16 : cus * per_cu);
 		if (nw == 1)
@@ -737,14 +737,10 @@ static int launch_ric_f32(int batch, const blasfeo_amd_riccati_arg *args, int mm
 		const int cls = sched[e][0];
 		hipStream_t sc = str.ss[sched[e][1]];
 		// two waves per instance up to 24 KB, four above; as many resident
-		// instances as LDS and three waves per SIMD allow.  The tuning knobs
-		// override both.
-		int nt = h_ric_cap[cls] <= 24576 ? 128 : 256;
-		int per_cu = min(nt == 128 ? 6 : 3, RIC_LDS_MAX / h_ric_cap[cls]);
-		if (const int v = tune_value(TUNE_RIC_PER_CU, cls))
-			per_cu = v;
-		if (const int v = tune_value(TUNE_RIC_THREADS, cls))
-			nt = v;
+		// instances as LDS and three waves per SIMD allow.  (The tuning knobs are not
+		// for these: they count the FP64 sweep's classes.)
+		const int nt = h_ric_cap[cls] <= 24576 ? 128 : 256;
+		const int per_cu = min(nt == 128 ? 6 : 3, RIC_LDS_MAX / h_ric_cap[cls]);
 		const int grid = min(batch, cus * per_cu);
 		rc = nt <= 128 ? launch_class<PS, 128, float>(cls, grid, args, counts, lists, batch, sc, name)
 		               : launch_class<PS, 256, float>(cls, grid, args, counts, lists, batch, sc, name);

@@ -129,12 +129,16 @@ const char *blasfeo_amd_last_error(void);
  * in the reference, whose block sizes are fixed at build time).  Set by the
  * autotuner (blasfeo_amd/autotune.py) from measurements on the caller's
  * workload; 0 restores the built-in choice.
- *   "ric_per_cu",  index = Riccati class 0..7 (FP64: the 16-row strips of the
- *                  largest stage, less one; FP32: LDS footprint): resident
- *                  instances per CU of the class's persistent launch (1..64);
+ *   "ric_per_cu",  index = class 0..7 of the FP64 Riccati sweep (the 16-row strips
+ *                  of the largest stage, with d_back_ric_sv's extra row, less
+ *                  one): resident instances per CU of the class's persistent
+ *                  launch (1..64);
  *   "ric_threads", index = class 0..7: threads per instance (64, 128 or 256;
  *                  64 only for classes 0..4; a wave holds two strips at most,
- *                  a smaller value than that needs is not used);
+ *                  a smaller value than that needs is not used).  A value of
+ *                  either for a class within the call's hint sends also the
+ *                  batches to the class launches that would go out directly
+ *                  (stages of at most 32 rows, or one instance per CU);
  *   "gemm_grid_y", index 0: most workgroups per gemm/syrk/trmm instance (1..64);
  *   "potrf_bw",    index 0: potrf_l(_mn) up to 256 columns with one wave per
  *                  instance (1) or with several (2, 4); built-in: one when the

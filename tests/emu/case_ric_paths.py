@@ -4,8 +4,10 @@ path, factors, reciprocal diagonals and their flags (sv: ux and pi too) against 
           instance per CU (four waves each);
   plan    the class launches, one, two and four waves per instance (a knob of a class
           that the hint admits sends the batch there);
-  beyond  instances larger than the hint, on both paths: factorised all the same.
-Usage: python case_ric_paths.py <trf | sv> <direct | plan | beyond> <ps>"""
+  beyond  instances larger than the hint, on both paths: factorised all the same;
+  knobs   which launches a knob changes: of the FP64 sweep those of batches whose hint
+          admits its class, none of the FP32 sweep (of the mixed-precision solve).
+Usage: python case_ric_paths.py <trf | sv> <direct | plan | beyond | knobs> <ps>"""
 import ctypes
 import sys
 
@@ -81,9 +83,35 @@ def check(entry, ps, nxs, nus, hint, knob):
                         "%s[%d] instance %d" % (kind, k, i))
 
 
+def knobs(entry, ps):
+    E = emu_lib("emu_lapack")
+
+    def launches(f, knob, cls, value):
+        E.blasfeo_amd_tune_set(knob, cls, value)
+        n = E.emu_launches(0), E.emu_launches(1)
+        f()
+        E.blasfeo_amd_tune_set(knob, cls, 0)
+        return E.emu_launches(0) - n[0], E.emu_launches(1) - n[1]
+
+    small = lambda: check(entry, ps, *SMALL, (31, 29, 0), 0)  # noqa: E731
+    plain = launches(small, b"ric_per_cu", 1, 0)
+    assert plain[0] <= 2, plain   # the sweep, and sv's forward substitution
+    for cls in range(2, 8):
+        assert launches(small, b"ric_per_cu", cls, 1) == plain, cls
+        assert launches(small, b"ric_threads", cls, 256) == plain, cls
+    assert launches(small, b"ric_per_cu", 1, 1)[0] > 2
+    if entry == "trf":
+        import case_ric
+        case_ric.NXS, case_ric.NUS = SMALL   # classes 0 and 1 of the FP64 sweep
+        mixed = lambda: case_ric.run_mixed(ps)  # noqa: E731
+        assert launches(mixed, b"ric_threads", 4, 128) == launches(mixed, b"ric_threads", 4, 0)
+
+
 def run(entry, path, ps):
     top = 127 if entry == "sv" else 128
-    if path == "direct":
+    if path == "knobs":
+        knobs(entry, ps)
+    elif path == "direct":
         check(entry, ps, *SMALL, (31, 29, 0), 0)
         check(entry, ps, *MIXED, (127, 64, 0), 0)
     elif path == "plan":

@@ -297,8 +297,12 @@ static void run_block(std::vector<Fiber> &fib, dim3 grid, dim3 block, unsigned b
 	}
 }
 
+static int g_launches, g_launch_threads;   // of all launches; their workgroups' threads
+
 void run_grid(dim3 grid, dim3 block, size_t shm, block_fn fn, void *ctx)
 {
+	g_launches++;
+	g_launch_threads += (int)block.x;
 	const int nt = (int)(block.x * block.y * block.z);
 	if (shm > EMU_LDS_MAX || nt <= 0 || nt > 1024 || block.y != 1 || block.z != 1)
 	{
@@ -357,4 +361,5 @@ void *plan_workspace(size_t bytes, hipStream_t)
 	return ws.data();
 }
 }
+extern "C" int emu_launches(int threads) { return threads ? emu::g_launch_threads : emu::g_launches; }
 extern "C" const char *emu_last_error() { return bfa::g_err; }
