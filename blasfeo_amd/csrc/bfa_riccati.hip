@@ -585,38 +585,56 @@ static RicFork *ric_fork_state()
 	return f;
 }
 
-// The fork of the caller's stream to the helpers and the join back, RAII: the
-// helpers are joined also after a launch error, so that the caller's stream never
-// runs ahead of them.
+// The fork of the caller's stream to the helpers and the join back.  Every helper that
+// waits on the caller's stream is joined, also after an error in the fork, in a launch
+// or in another helper's join (the destructor joins what is left), so that the caller's
+// stream never runs ahead of them and a capture finds no helper left open.
 struct RicStreams
 {
 	RicFork *fk = nullptr;
+	int forked = 0;   // helpers that wait on the caller's stream and are not joined
 	std::unique_lock<std::mutex> lock;
 	hipStream_t ss[1 + RIC_AUX];
 	explicit RicStreams(hipStream_t st) { for (hipStream_t &s : ss) s = st; }
+	RicStreams(const RicStreams &) = delete;
+	RicStreams &operator=(const RicStreams &) = delete;
+	~RicStreams() { join(nullptr); }
 	int fork(const char *name)
 	{
 		fk = ric_fork_state();
 		if (!fk)
 			return set_error(BLASFEO_AMD_ELAUNCH, "%s: cannot create the helper streams", name);
 		lock = std::unique_lock<std::mutex>(fk->mu);
-		if (hipEventRecord(fk->fork, ss[0]) != hipSuccess)
-			return check_launch(name);
+		if (const hipError_t e = hipEventRecord(fk->fork, ss[0]))
+			return failed(e, name);
 		for (int i = 0; i < RIC_AUX; i++)
 		{
 			ss[1 + i] = fk->aux[i];
-			if (hipStreamWaitEvent(fk->aux[i], fk->fork, 0) != hipSuccess)
-				return check_launch(name);
+			if (const hipError_t e = hipStreamWaitEvent(fk->aux[i], fk->fork, 0))
+				return failed(e, name);
+			forked = i + 1;
 		}
 		return BLASFEO_AMD_OK;
 	}
 	int join(const char *name)
 	{
-		for (int i = 0; fk && i < RIC_AUX; i++)
-			if (hipEventRecord(fk->join[i], fk->aux[i]) != hipSuccess ||
-				hipStreamWaitEvent(ss[0], fk->join[i], 0) != hipSuccess)
-				return check_launch(name);
-		return BLASFEO_AMD_OK;
+		hipError_t first = hipSuccess;
+		for (int i = 0; i < forked; i++)
+		{
+			hipError_t e = hipEventRecord(fk->join[i], fk->aux[i]);
+			if (e == hipSuccess)
+				e = hipStreamWaitEvent(ss[0], fk->join[i], 0);
+			if (first == hipSuccess)
+				first = e;
+		}
+		forked = 0;
+		return first == hipSuccess ? BLASFEO_AMD_OK : failed(first, name);
+	}
+	// (the runtime's last error is taken, so that the next call does not report it)
+	static int failed(hipError_t e, const char *name)
+	{
+		(void)hipGetLastError();
+		return name ? set_error(BLASFEO_AMD_ELAUNCH, "%s: helper streams: %s", name, hipGetErrorString(e)) : BLASFEO_AMD_ELAUNCH;
 	}
 };
 

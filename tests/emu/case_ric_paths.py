@@ -6,8 +6,10 @@ path, factors, reciprocal diagonals and their flags (sv: ux and pi too) against 
           that the hint admits sends the batch there);
   beyond  instances larger than the hint, on both paths: factorised all the same;
   knobs   which launches a knob changes: of the FP64 sweep those of batches whose hint
-          admits its class, none of the FP32 sweep (of the mixed-precision solve).
-Usage: python case_ric_paths.py <trf | sv> <direct | plan | beyond | knobs> <ps>"""
+          admits its class, none of the FP32 sweep (of the mixed-precision solve);
+  join    an event record or wait that fails: the call reports it, and every helper stream
+          that waits on the caller's is waited for by it.
+Usage: python case_ric_paths.py <trf | sv> <direct | plan | beyond | knobs | join> <ps>"""
 import ctypes
 import sys
 
@@ -107,10 +109,32 @@ def knobs(entry, ps):
         assert launches(mixed, b"ric_threads", 4, 128) == launches(mixed, b"ric_threads", 4, 0)
 
 
+def join(entry, ps):
+    E = emu_lib("emu_lapack")
+    E.emu_fail_stream(0)
+    check(entry, ps, [5], [2], (7, 5, 0), 2)
+    helpers = E.emu_waits(1)
+    assert helpers == E.emu_waits(0) > 0
+    # the fork's record, its waits, then a record and a wait for each helper's join
+    for n in range(1, 1 + 1 + 3 * helpers):
+        E.emu_fail_stream(n)
+        try:
+            check(entry, ps, [5], [2], (7, 5, 0), 2)
+            failed = False
+        except AssertionError as e:
+            failed = b"helper streams" in e.args[0]
+        assert failed, n
+        broken = n > 1 + helpers   # a helper whose own join failed cannot be waited for
+        assert E.emu_waits(0) == E.emu_waits(1) - broken, (n, E.emu_waits(0), E.emu_waits(1))
+    E.emu_fail_stream(0)
+
+
 def run(entry, path, ps):
     top = 127 if entry == "sv" else 128
     if path == "knobs":
         knobs(entry, ps)
+    elif path == "join":
+        join(entry, ps)
     elif path == "direct":
         check(entry, ps, *SMALL, (31, 29, 0), 0)
         check(entry, ps, *MIXED, (127, 64, 0), 0)

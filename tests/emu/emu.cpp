@@ -297,6 +297,7 @@ static void run_block(std::vector<Fiber> &fib, dim3 grid, dim3 block, unsigned b
 	}
 }
 
+int stream_calls, stream_fail, waits[2];
 static int g_launches, g_launch_threads;   // of all launches; their workgroups' threads
 
 void run_grid(dim3 grid, dim3 block, size_t shm, block_fn fn, void *ctx)
@@ -362,4 +363,11 @@ void *plan_workspace(size_t bytes, hipStream_t)
 }
 }
 extern "C" int emu_launches(int threads) { return threads ? emu::g_launch_threads : emu::g_launches; }
+// the n-th event record or wait from now on fails (0: none); waits of the null stream (0), of others (1)
+extern "C" void emu_fail_stream(int n)
+{
+	emu::stream_calls = emu::waits[0] = emu::waits[1] = 0;
+	emu::stream_fail = n;
+}
+extern "C" int emu_waits(int other) { return emu::waits[other]; }
 extern "C" const char *emu_last_error() { return bfa::g_err; }

@@ -192,10 +192,20 @@ inline void emu_launch(void (*k)(KA...), dim3 grid, dim3 block, size_t shm, A...
 #define HIP_SYMBOL(x) (&(x))
 inline hipError_t hipGetSymbolAddress(void **p, const void *sym) { *p = const_cast<void *>(sym); return hipSuccess; }
 inline hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
+namespace emu {
+extern int stream_calls, stream_fail;   // event records and waits so far; the one that fails (0: none)
+extern int waits[2];                    // waits that were made: of the null stream, of others
+}
 inline hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { *e = nullptr; return hipSuccess; }
-inline hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { *s = nullptr; return hipSuccess; }
-inline hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
-inline hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+inline hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { *s = s; return hipSuccess; }
+inline hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return ++emu::stream_calls == emu::stream_fail ? hipErrorInvalidValue : hipSuccess; }
+inline hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t, unsigned)
+{
+	if (++emu::stream_calls == emu::stream_fail)
+		return hipErrorInvalidValue;
+	emu::waits[s != nullptr]++;
+	return hipSuccess;
+}
 inline hipError_t hipGetLastError() { return hipSuccess; }
 inline hipError_t hipPeekAtLastError() { return hipSuccess; }
 inline const char *hipGetErrorString(hipError_t) { return "emulated"; }

@@ -175,7 +175,7 @@ def test_trsm_rltn_several_launches(emu_build, ps):
     run_case("case_trsm.py", "launches", ps)
 
 
-@pytest.mark.parametrize("path", ["direct", "plan", "beyond", "knobs"])
+@pytest.mark.parametrize("path", ["direct", "plan", "beyond", "knobs", "join"])
 @pytest.mark.parametrize("ps", [4, 8])
 @pytest.mark.parametrize("entry", ["trf", "sv"])
 def test_riccati_paths(emu_build, entry, ps, path):
