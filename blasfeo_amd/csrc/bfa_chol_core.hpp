@@ -415,21 +415,10 @@ __device__ __forceinline__ void chol_acc(const ACC M, int m, int n, T *invd, con
 		__syncthreads();
 }
 
-
-// Column-major LDS matrix: element (r, c) at p[c*ld + r].
-template <typename T>
-struct ColMajor
-{
-	T *p;
-	int ld;
-	__device__ __forceinline__ T &operator()(int r, int c) const { return p[c * ld + r]; }
-};
-
 // Packed lower tiles in LDS: 16x16 tiles with a leading dimension of 17 inside
 // the tile (a row of a tile then spans distinct banks), tile (I,J), I >= J,
-// at I(I+1)/2 + J.  The Riccati sweep keeps its stage matrix so, and the
-// size-bucketed LDS Cholesky its trapezoid: mt(mt+1)/2 tiles for mt tile
-// rows, 78 KB at 128 rows against 133 KB for the square column-major form.
+// at I(I+1)/2 + J.  The Riccati sweeps keep their stage matrix so: mt(mt+1)/2 tiles
+// for mt tile rows, 78 KB at 128 rows in FP64 against 133 KB for a square.
 constexpr int RT_LD = 17;
 constexpr int RT_SZ = 16 * RT_LD;
 
@@ -445,11 +434,5 @@ struct TileLowerT
 		return p[ric_tix(r >> 4, c >> 4) * RT_SZ + (c & 15) * RT_LD + (r & 15)];
 	}
 };
-
-template <typename T, int NT = NTL, int NMAX = 128>
-__device__ __forceinline__ void chol_lds(T *M, int ld, int n, T *invd)
-{
-	chol_acc<T, NT, NMAX>(ColMajor<T>{M, ld}, n, n, invd);
-}
 
 } // namespace bfa

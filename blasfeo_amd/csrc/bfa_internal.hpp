@@ -23,10 +23,6 @@ int lds_check(const void *fn, size_t dyn, const char *what);
 // captured an earlier block still finds it.  Launches on one stream are
 // ordered, so reusing a block across calls on that stream is safe.
 void *workspace(size_t bytes, hipStream_t stream);
-// A second such block for the size plans of the leaf launches (the LDS-resident
-// factorisations), which composite entries call while their own records sit in
-// workspace().
-void *plan_workspace(size_t bytes, hipStream_t stream);
 
 // D = B * A^{-T} (trsm_rltn, alpha from the records) with the reciprocal
 // diagonal of A read from sA->dA whatever its use_dA, and no cache update:

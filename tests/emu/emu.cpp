@@ -354,13 +354,6 @@ void *workspace(size_t bytes, hipStream_t)
 		ws.resize(bytes);
 	return ws.data();
 }
-void *plan_workspace(size_t bytes, hipStream_t)
-{
-	static std::vector<unsigned char> ws;
-	if (ws.size() < bytes)
-		ws.resize(bytes);
-	return ws.data();
-}
 }
 extern "C" int emu_launches(int threads) { return threads ? emu::g_launch_threads : emu::g_launches; }
 // the n-th event record or wait from now on fails (0: none); waits of the null stream (0), of others (1)
