@@ -16,10 +16,10 @@
 // per shape), so that the edges cost no products beyond their last block.
 // Measured (MI355X; before: 32 x 32 tiles with 8-byte loads up to 256, a 64 x 64
 // tile staged through LDS by four waves above): 1024 dgemm_nn of U{64..512}, ps = 8,
-// 1929 -> 1055 us (49 TFLOP/s), 256 of 512^3 1697 -> 1030 us (67 TFLOP/s, the rate of
-// a large library product here), 8192 sgemm_nt + ssyrk_ln of U{16..256} 1855 -> 1115 us
-// (3.4 TB/s, 60 TFLOP/s): bound by the matrix cores and the last blocks' padding.
-// 32768 dgemm_nt + dsyrk_ln of U{4..128} 1939 -> 1690 us (4.3 TB/s), 16384 of 64^3
+// 1925 -> 1117 us (46 TFLOP/s), 256 of 512^3 1697 -> 1030 us (67 TFLOP/s, the rate of
+// a large library product here), 8192 sgemm_nt + ssyrk_ln of U{16..256} 1851 -> 1141 us
+// (3.3 TB/s, 60 TFLOP/s): bound by the matrix cores and the last blocks' padding.
+// 32768 dgemm_nt + dsyrk_ln of U{4..128} 1943 -> 1683 us (4.3 TB/s), 16384 of 64^3
 // 698 -> 648 us (4.95 TB/s, a large copy's rate): bound by memory.
 #pragma once
 #include "bfa_gemm_core.hpp"

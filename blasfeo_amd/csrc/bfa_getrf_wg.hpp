@@ -18,18 +18,23 @@
 // most 32 rows, all loads before the stores.
 // Measured (MI355X, dgetrf_rp; before: 16-column panels brought up to date block by
 // block with two barriers each, exchanges one after the other): 8192 of
-// U{16..256} 3850 -> 3110 us, with the solves of 4 right-hand sides 4600 -> 3916;
-// 4096 of 64 with the solves 603 -> 304 us, 2048 of 128 911 -> 683, 512 of 256 1162 ->
-// 859.  Bound by latency: of 5550 cycles a column takes (three workgroups per
-// CU) 1760 are the panel's chain of search, reciprocal and broadcast, 1110 the
-// column and 1440 the row panel's products and gathers, 700 the exchanges.
+// U{16..256} 3840 -> 2990 us, with the solves of 4 right-hand sides 4600 -> 3600;
+// 4096 of 64 479 -> 154 us, 2048 of 128 711 -> 444, 512 of 256 982 -> 632.  The
+// products are summed from zero and C joins last: sums begun at C are rounded at C's
+// size in every step, and cost registers besides (3180 us of the first batch, errors
+// up to 2.5 times as large).  Bound by latency: of 5550 cycles a column of panels
+// took with sums begun at C (three workgroups per CU) 1760 were the panel's chain of
+// search, reciprocal and broadcast, 1110 the column and 1440 the row panel's products
+// and gathers, 700 the exchanges, the rest the panel's way to D and the barriers.
 #pragma once
 #include "bfa_strip.hpp"
 
 namespace bfa {
 
 constexpr int GLU_M = 256;            // most rows
-constexpr int GLU_D = 2;              // pairs of K steps in flight: with 3 or 4 registers spill (4059 -> 4322, 4437 us)
+// Pairs of K steps in flight: with 3 or 4 registers spilled (with the solves and sums begun
+// at C 4059 -> 4322, 4437 us).
+constexpr int GLU_D = 2;
 constexpr int GLU_UL = 18;            // stride of the rows of U put aside
 
 // The upper (float: all) and the lower 32 bits of |v|: the order of the values is that

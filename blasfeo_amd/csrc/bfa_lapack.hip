@@ -741,8 +741,8 @@ extern "C" {
 
 int blasfeo_amd_dpotrf_l_batched(int ps, int batch, const blasfeo_amd_dfact_arg *args, const blasfeo_amd_hint *hint, blasfeo_amd_stream_t s)
 { return launch_potrf<double, 0>(ps, batch, args, hint, (hipStream_t)s, "blasfeo_amd_dpotrf_l_batched"); }
-// m <= 128: the LDS-resident forms; larger m: the trapezoid as potrf_l of
-// the top block plus the solve of the rows below (see launch_potrf_mn_split).
+// Large m: the trapezoid as potrf_l of the top block plus the solve of the rows
+// below (launch_potrf_mn_split).
 int blasfeo_amd_dpotrf_l_mn_batched(int ps, int batch, const blasfeo_amd_dfact_arg *args, const blasfeo_amd_hint *hint, blasfeo_amd_stream_t s)
 { return launch_potrf<double, 1>(ps, batch, args, hint, (hipStream_t)s, "blasfeo_amd_dpotrf_l_mn_batched"); }
 int blasfeo_amd_dsyrk_dpotrf_ln_batched(int ps, int batch, const blasfeo_amd_dsyrk_dpotrf_arg *args, const blasfeo_amd_hint *hint, blasfeo_amd_stream_t s)

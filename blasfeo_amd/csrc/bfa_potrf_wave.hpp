@@ -35,8 +35,8 @@ constexpr int potrf_wave_elems()
 // all there is, and the other waves of the SIMD, each with an instance of its own,
 // fill its latencies.  NB bounds the block columns (n <= 16 NB).
 // Measured (MI355X, 8192 FP64 instances, ps = 4; before: four waves per instance,
-// the trapezoid in LDS, one wave factoring the panels): n = 32 41.7 -> 27 us,
-// n = 64 490 -> 87 us, n = 128 1935 -> 480 us, n = 256 3257 -> 2715 us.
+// the trapezoid in LDS, one wave factoring the panels): n = 32 40 -> 25 us,
+// n = 64 487 -> 86 us, n = 128 1932 -> 480 us, n = 256 3237 -> 2650 us.
 // Bound up to 64 columns by the vector instructions of the solves and diagonal
 // factorisations (3050 of them and 70 matrix-core steps per wave at n = 64),
 // above by memory: the rows of L that are read back miss L2 for the most part
@@ -173,8 +173,9 @@ __global__ __launch_bounds__(WAVE, (strip_waves<T, NB>())) void k_potrf_wave(con
 // strips' rows of A, which it loads itself (the same registers where A is B); the
 // next chunk's loads are in flight meanwhile.  A and B are read once.
 // Measured (MI355X, FP64, ps = 4, before: as above): syrk_dpotrf_ln, 8192 of
-// m = k = 64 629 -> 237 us, of m = k = 128 2983 -> 890 us; potrf_l, 256 of
-// n = 128 117 -> 41 us, of n = 256 268 -> 117 us.  Bound by the chain of
+// m = k = 64 629 -> 249 us, of m = k = 128 2978 -> 892 us (863 with the sums begun at
+// C, whose errors were up to 1.7 times as large); potrf_l, 256 of n = 128 113 -> 35 us,
+// of n = 256 268 -> 108 us.  Bound by the chain of
 // one diagonal block and one solve per block column (three instances per CU).
 // ---------------------------------------------------------------------------
 template <typename T, int PS, int NW, bool SYRK>

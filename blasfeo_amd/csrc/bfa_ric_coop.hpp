@@ -7,7 +7,8 @@
 //                           previous stage's Cholesky) times the previous factor
 //                           (LDS tiles); the result replaces them, and goes to LDS
 //                           as operand tiles for the other strips
-//   M_IJ = RSQ_IJ + W_I W_J^T   accumulators loaded from RSQ while W is formed
+//   M_IJ = RSQ_IJ + W_I W_J^T   summed from zero, RSQ added last: sums begun at RSQ are
+//                           rounded at its size in every step
 //   L = chol(M)             chol_coop; its column tiles are the LDS tiles that the
 //                           next stage's product reads
 // Barriers: one after W, one per block column of the Cholesky and two before
@@ -20,8 +21,8 @@
 // no other strip reads.
 // Measured (MI355X; before: the stage matrix in LDS, its panels factored by one of
 // the waves, nine launches a call): 8192 x N = 20, nx ~ U{8..64}, nu ~ U{2..16}
-// 5.45 -> 4.35 ms, 2048 sv of N = 15, nx ~ U{6..40} 1.33 -> 0.93 ms, one instance
-// of N = 20, nx = 8, nu = 3 184 -> 68 us.  Bound by instruction issue (about two
+// 5.47 -> 4.49 ms, 2048 sv of N = 15, nx ~ U{6..40} 1.33 -> 0.93 ms, one instance
+// of N = 20, nx = 8, nu = 3 203 -> 79 us (whole calls).  Bound by instruction issue (about two
 // thirds of the SIMDs' cycles on the first batch: 78 cycles per matrix-core step,
 // 1830 per 16 x 16 diagonal block, 560 per strip and column solve) and by the
 // chain solve - diagonal block of each block column (about 5000 cycles).
@@ -196,7 +197,7 @@ __device__ __forceinline__ void ric_coop(const RicRec &a, int N, int nkmax, doub
 	if (N > 0)
 		raw = ric_fetch(a, N, N - 1);
 	int n1 = 0, u1 = 0;   // sizes of stage k + 1
-	// M starts from RSQ[k]
+	// RSQ[k], added to the products at the end
 	auto load_m = [&](const RicStage<PS> &q, V4 (&th)[2 * NW], V4 (&tl)[NW]) {
 		const int nk = q.nu + q.nx, m = nk + XR;
 		int R, ih, il;

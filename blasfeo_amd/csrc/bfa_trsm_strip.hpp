@@ -11,9 +11,9 @@
 // every wave for itself they came from L2 at a rate that bound the kernel).
 // Per block column one barrier.
 // Measured (MI355X, 8192 FP64 solves, ps = 4; before: the row block in LDS, one of
-// four waves solving the diagonal blocks): m = n = 32 125 -> 54 us, 64 235 -> 159,
-// 128 1608 -> 795, 256 15.3 -> 4.4 ms (31 TFLOP/s; 6.2 ms with every wave reading
-// A for itself); m, n ~ U{16..256} 4.61 -> 1.80 ms (1.69 with the sum begun at B_K,
+// four waves solving the diagonal blocks): m = n = 32 124 -> 56 us, 64 234 -> 169,
+// 128 1608 -> 702, 256 15.3 -> 5.0 ms (27 TFLOP/s; every wave reading A for itself
+// took 1.4 times as long); m, n ~ U{16..256} 4.60 -> 1.79 ms (1.69 with the sum begun at B_K,
 // whose error was 2.4 times as large).  Bound by memory up to 64
 // columns, then by the matrix cores and the substitution's vector instructions,
 // with two waves per SIMD.

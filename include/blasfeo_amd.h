@@ -424,7 +424,7 @@ struct blasfeo_amd_riccati_arg
 	};
 
 /* Fused backward factorisation sweep, one workgroup per instance, all stages in
- * one launch (the per-stage trmm_rlnn + syrk_dpotrf_ln chain of
+ * one call (the per-stage trmm_rlnn + syrk_dpotrf_ln chain of
  * examples/example_d_riccati_recursion.c:120-138).  hint->max_m bounds
  * nu[k]+nx[k] (at most 1024) and hint->max_n bounds nx[k] (0: max_m). */
 int blasfeo_amd_d_back_ric_trf_batched(int ps, int batch, const struct blasfeo_amd_riccati_arg *args, const struct blasfeo_amd_hint *hint, blasfeo_amd_stream_t stream);
@@ -499,7 +499,7 @@ struct blasfeo_amd_riccati_sv_arg
 	};
 
 /* Batched d_back_ric_sv_libstr: the backward sweep on the augmented matrices
- * (the LDS-resident sweep of blasfeo_amd_d_back_ric_trf_batched, the factor's
+ * (the on-chip sweep of blasfeo_amd_d_back_ric_trf_batched, the factor's
  * last row carrying the linear terms), then one wavefront per instance for the
  * forward substitution.  hint->max_m bounds nu[k]+nx[k] (at most 127) and
  * hint->max_n bounds nx[k] (at most 64); larger bounds return
